@@ -60,88 +60,124 @@ void rcb(const std::vector<double>& C, std::vector<int>& idx, int lo, int hi, in
 
 }  // namespace
 
-// The forward (L) or backward (Dinv, Dinv U) stream of the partitioned
-// ILU(0) apply, in the layout PiluStream describes.  Left empty (kmax = 0)
-// when a row has more than kPiluKD blocks in the sweep.
-static void build_pilu_stream(const Mesh& m, bool bwd, PiluStream& ps) {
-    ps.kmax = 0;
-    ps.nBlk = 0;
-    std::vector<int32_t> subStart(m.nParts + 1, 0), sub, ord, lc, src, row, jn;
-    int kmaxAll = 0;
-    struct RowBlocks {
-        int t, cnt;
-        int32_t src[kPiluKD], lc[kPiluKD];
+// The record stream of the partitioned ILU(0) apply, in the layout StreamSet
+// describes.  Left empty (kmax = 0) when a row has more than kStreamKD
+// off-diagonal blocks in one sweep or the stream passes 64 GiB.
+static void build_stream(const Mesh& m, bool fp32, StreamSet& ps) {
+    int kmax = 1;
+    for (int i = 0; i < m.nC; ++i) {
+        int lo = 0, up = 0;
+        for (int s = m.rowPtr[i]; s < m.rowPtr[i + 1]; ++s)
+            if (m.localCol[s] >= 0 && s != m.slotDiag[i]) (s < m.slotDiag[i] ? lo : up)++;
+        kmax = std::max(kmax, std::max(lo, up));
+    }
+    if (kmax > kStreamKD) return;
+    ps.ent = stream_entry(kmax);
+    const int ring = stream_ring(fp32), cap = stream_record(fp32), blk = 25 * (fp32 ? 4 : 8);
+    struct Row {
+        int t, i, cnt;
     };
-    std::vector<RowBlocks> rows;
+    std::vector<Row> rows;
+    ps.recBeg.assign(1, 0);
+    ps.recRows.assign(1, 0);
+    ps.recBlk.assign(1, 0);
+    size_t pos = 0;
+    auto size_of = [&](int nr, int nb) { return nr * ps.ent + ((nb * blk + 15) & ~15); };
     for (int p = 0; p < m.nParts; ++p) {
         const int rs = m.partRowStart[p];
         const int l0 = m.partLevStart[p], nl = m.partLevStart[p + 1] - l0 - 1;
-        for (int li = 0; li < nl; ++li) {
-            const int L = bwd ? nl - 1 - li : li;
-            rows.clear();
-            for (int t = m.partLevPtr[l0 + L]; t < m.partLevPtr[l0 + L + 1]; ++t) {
-                const int i = m.partRows[t];
-                RowBlocks rb;
-                rb.t = t - rs;
-                rb.cnt = 0;
-                auto add = [&](int32_t sv, int32_t lv) {
-                    if (rb.cnt == kPiluKD) { rb.cnt = kPiluKD + 1; return; }
-                    if (rb.cnt > kPiluKD) return;
-                    rb.src[rb.cnt] = sv;
-                    rb.lc[rb.cnt] = lv;
-                    ++rb.cnt;
-                };
-                if (!bwd) {
-                    for (int s = m.rowPtr[i]; s < m.slotDiag[i]; ++s)
-                        if (m.localCol[s] >= 0) add(s, m.localCol[s]);
-                    if (rb.cnt == 0) continue;  // y = r on this row
-                } else {
-                    add(-(i + 1), t - rs);
-                    for (int s = m.slotDiag[i] + 1; s < m.rowPtr[i + 1]; ++s)
-                        if (m.localCol[s] >= 0) add(s, m.localCol[s]);
+        const size_t base = pos;
+        for (int sweep = 0; sweep < 2; ++sweep) {
+            if (sweep == 1) ps.recMid.push_back((int32_t)ps.hdr.size());
+            for (int li = 0; li < nl; ++li) {
+                const int L = sweep ? nl - 1 - li : li;
+                rows.clear();
+                for (int t = m.partLevPtr[l0 + L]; t < m.partLevPtr[l0 + L + 1]; ++t) {
+                    const int i = m.partRows[t];
+                    const int s0 = sweep ? m.slotDiag[i] + 1 : m.rowPtr[i], s1 = sweep ? m.rowPtr[i + 1] : m.slotDiag[i];
+                    int cnt = 0;
+                    for (int s = s0; s < s1; ++s) cnt += m.localCol[s] >= 0;
+                    if (sweep || cnt) rows.push_back({t - rs, i, cnt});  // forward: y = r on a row without L
                 }
-                if (rb.cnt > kPiluKD) return;  // stays unbuilt
-                rows.push_back(rb);
-            }
-            for (size_t r0 = 0; r0 < rows.size(); r0 += kPiluSubRows) {
-                const size_t r1 = std::min(rows.size(), r0 + kPiluSubRows);
-                std::stable_sort(rows.begin() + r0, rows.begin() + r1,
-                                 [](const RowBlocks& a, const RowBlocks& b) { return a.cnt > b.cnt; });
-                const int nr = (int)(r1 - r0), km = rows[r0].cnt;
-                kmaxAll = std::max(kmaxAll, km);
-                int32_t d[kPiluSubW] = {0};
-                d[0] = (int32_t)ord.size();
-                d[1] = nr;
-                d[2] = km;
-                for (size_t q = r0; q < r1; ++q) ord.push_back(rows[q].t);
-                for (int k = 0; k < km; ++k) {
-                    int nk = 0;
-                    while (nk < nr && rows[r0 + nk].cnt > k) ++nk;
-                    d[4 + k] = (int32_t)src.size();
-                    d[4 + kPiluKD + k] = nk;
-                    for (int j = 0; j < nk; ++j) {
-                        const RowBlocks& rb = rows[r0 + j];
-                        src.push_back(rb.src[k]);
-                        lc.push_back(rb.lc[k]);
-                        row.push_back(m.partRows[rs + rb.t]);
-                        jn.push_back(j | (nk << 8));
+                // rows of one block count together: a wavefront's rows run the same products
+                std::stable_sort(rows.begin(), rows.end(), [](const Row& a, const Row& b) { return a.cnt > b.cnt; });
+                for (size_t r0 = 0; r0 < rows.size();) {
+                    // as many rows as a record, and the ring up to its end, hold
+                    int room = ring - (int)((pos - base) % ring);
+                    if (size_of(1, rows[r0].cnt + sweep) > room) {
+                        pos += room;
+                        ps.hdr.back() += (uint32_t)(room / 16) << 16;
+                        room = ring;
                     }
+                    room = std::min(room, cap);
+                    size_t r1 = r0;
+                    int nb = 0;
+                    while (r1 < rows.size() && r1 - r0 < (size_t)kStreamRows &&
+                           size_of((int)(r1 - r0) + 1, nb + rows[r1].cnt + sweep) <= room)
+                        nb += rows[r1++].cnt + sweep;
+                    const int nr = (int)(r1 - r0), bytes = size_of(nr, nb);
+                    int first = 0;
+                    for (size_t q = r0; q < r1; ++q) {
+                        const Row& w = rows[q];
+                        const size_t e0 = ps.entries.size();
+                        ps.entries.resize(e0 + ps.ent / 2, 0);
+                        uint16_t* e = ps.entries.data() + e0;
+                        e[0] = (uint16_t)(5 * w.t);
+                        e[1] = (uint16_t)(first | w.cnt << 8);
+                        if (sweep) {
+                            ps.src.push_back(-(w.i + 1));
+                            ps.rowCell.push_back(w.i);
+                        }
+                        int k = 2;
+                        const int s0 = sweep ? m.slotDiag[w.i] + 1 : m.rowPtr[w.i],
+                                  s1 = sweep ? m.rowPtr[w.i + 1] : m.slotDiag[w.i];
+                        for (int s = s0; s < s1; ++s)
+                            if (m.localCol[s] >= 0) {
+                                ps.src.push_back(s);
+                                ps.rowCell.push_back(sweep ? w.i : -1);
+                                e[k++] = (uint16_t)(5 * m.localCol[s]);
+                            }
+                        first += w.cnt + sweep;
+                    }
+                    ps.start.push_back((uint32_t)(pos / 16));
+                    ps.hdr.push_back((uint32_t)nr | (uint32_t)(bytes / 16) << 16);
+                    ps.recRows.push_back(ps.recRows.back() + nr);
+                    ps.recBlk.push_back((int32_t)ps.src.size());
+                    pos += bytes;
+                    r0 = r1;
                 }
-                sub.insert(sub.end(), d, d + kPiluSubW);
             }
         }
-        subStart[p + 1] = (int32_t)(sub.size() / kPiluSubW);
+        ps.recBeg.push_back((int32_t)ps.hdr.size());
+        pos = (pos + 1023) & ~(size_t)1023;  // the loader copies 1 KB pieces
+        if (pos / 16 > 0xffffffffull) return;
     }
-    sub.insert(sub.end(), kPiluSubW, 0);
-    ps.kmax = std::max(kmaxAll, 1);
-    ps.nBlk = (long)src.size();
-    ps.subStart.swap(subStart);
-    ps.sub.swap(sub);
-    ps.ord.swap(ord);
-    ps.lc.swap(lc);
-    ps.src.swap(src);
-    ps.row.swap(row);
-    ps.jn.swap(jn);
+    ps.start.push_back((uint32_t)(pos / 16));
+    ps.nRec = (int)ps.hdr.size();
+    ps.kmax = kmax;
+}
+
+void StreamSet::upload() {
+    if (kmax == 0) return;
+    d_recBeg.upload(recBeg);
+    d_recMid.upload(recMid);
+    d_recRows.upload(recRows);
+    d_recBlk.upload(recBlk);
+    d_entries.upload(entries);
+    d_hdr.upload(hdr);
+    d_start.upload(start);
+    d_src.upload(src);
+    d_rowCell.upload(rowCell);
+}
+
+StreamSet& mesh_stream(Mesh& m, bool fp32) {
+    StreamSet& ps = m.ps[fp32];
+    if (!ps.tried) {
+        build_stream(m, fp32, ps);
+        ps.upload();
+        ps.tried = true;
+    }
+    return ps;
 }
 
 // Partition-local level of every cell (longest chain of in-partition lower
@@ -253,8 +289,6 @@ void build_partitions(Mesh& m, int maxCells) {
     m.localCol.swap(ps.localCol);
     m.maxPartRows = ps.maxRows;
     m.maxPartLevels = ps.maxLevels;
-    build_pilu_stream(m, false, m.pf);
-    build_pilu_stream(m, true, m.pb);
 }
 
 void mesh_build(Mesh& m, const rdst_mesh_desc* d, const rdst_mesh_geometry* g) {
@@ -671,16 +705,6 @@ void mesh_upload(Mesh& m) {
     m.sa.d_levStart.upload(m.sa.levStart);
     m.sa.d_levPtr.upload(m.sa.levPtr);
     m.sa.d_localCol.upload(m.sa.localCol);
-    for (PiluStream* ps : {&m.pf, &m.pb}) {
-        if (ps->kmax == 0) continue;
-        ps->d_subStart.upload(ps->subStart);
-        ps->d_sub.upload(ps->sub);
-        ps->d_ord.upload(ps->ord);
-        ps->d_lc.upload(ps->lc);
-        ps->d_src.upload(ps->src);
-        ps->d_row.upload(ps->row);
-        ps->d_jn.upload(ps->jn);
-    }
     m.d_sellPtr.upload(m.sellPtr);
     m.d_sellOfSlot.upload(m.sellOfSlot);
     m.d_sellWidth.upload(m.sellWidth);

@@ -73,35 +73,42 @@ static constexpr uint32_t ELL_IDX_MASK = 0x3fffffffu;
 
 // ---------------------------------------------------------------------------
 // Mesh: polyMesh primitives, fvMesh geometry (host), device copies.
-// One sweep of the partitioned ILU(0) apply laid out for coalesced loads.
-// The rows of a partition-local level are independent; a level is cut into
-// sub-levels of at most kPiluSubRows rows, and inside a sub-level the rows are
-// ordered by their block count, largest first, so that block k of every row
-// that has one forms a contiguous "jagged diagonal": diagonal k of sub-level
-// s holds n_k blocks at stream positions blk_k .. blk_k + n_k - 1, row j's at
-// blk_k + j.  Block values are stored per diagonal as five planes (column c of
-// the block) of 5 n_k values, entry (j, r, c) at
-// 25 blk_k + 5 n_k c + 5 j + r, so the five lanes of a row and the rows of a
-// wavefront read contiguous memory.  Sub-level s is described by
-// sub[kPiluSubW s ..]: rowOff (into ord), nRows, kmax, 0, blk_0..blk_7,
-// n_0..n_7.  The forward stream holds each row's in-partition L blocks (rows
-// without one are left out); the backward stream holds, per row, Dinv first
-// (its column is the row itself) and then Dinv U for each in-partition U
+// The sweeps of a partitioned ILU(0) apply as one stream of records per
+// partition, read linearly through a ring in LDS.  The rows of a
+// partition-local level are independent; a level is cut into records.  A record
+// holds a 16-byte entry per row (5 x its partition-local index, its first block
+// and block count, 5 x the partition-local columns of its off-diagonal blocks;
+// 32 bytes when a row has more than four) and then the rows' blocks, 25 values
+// each, padded to 16 bytes.  hdr[q]: rows | distance to the next record / 16 <<
+// 16.  The forward records hold each row's in-partition L blocks (rows without
+// one are left out); the backward ones, which follow them, hold per row Dinv
+// first (its column is the row itself) and then Dinv U for each in-partition U
 // block, so x = Dinv y - sum (Dinv U) x needs no separate diagonal solve.
-constexpr int kPiluKD = 8;                  // most blocks of a row in one sweep
-constexpr int kPiluSubW = 4 + 2 * kPiluKD;  // ints per sub-level descriptor
-constexpr int kPiluSubRows = 48;            // 4 wavefronts x 12 rows of 5 lanes
-struct PiluStream {
-    int kmax = 0;                  // largest row block count (0: not built)
-    long nBlk = 0;
-    std::vector<int32_t> subStart;  // [nParts + 1]
-    std::vector<int32_t> sub;       // [nSub + 1][kPiluSubW] (one zero descriptor of padding)
-    std::vector<int32_t> ord;       // partition-local row of each sub-level position
-    std::vector<int32_t> lc;        // [nBlk] partition-local column
-    std::vector<int32_t> src;       // [nBlk] block-CSR slot, or -(cell + 1) for the row's Dinv
-    std::vector<int32_t> row;       // [nBlk] cell of the block's row
-    std::vector<int32_t> jn;        // [nBlk] j | n_k << 8
-    DBuf<int32_t> d_subStart, d_sub, d_ord, d_lc, d_src, d_row, d_jn;
+constexpr int kStreamKD = 8;     // most off-diagonal blocks of a row in one sweep
+constexpr int kStreamRows = 48;  // rows of a record: 4 wavefronts x 12 rows of 5 lanes
+// Ring bytes.  With the partition's vector (at most 1024 rows) that leaves
+// three workgroups per CU in FP32 and one in FP64, 64-96 KB in flight per CU
+// either way.  A partition starts at the ring's start and no record crosses its
+// end, so a record's addresses need no wrapping.
+constexpr int stream_ring(bool fp32) { return fp32 ? 32768 : 65536; }
+// most bytes of a record: the ring holds three and their padding
+constexpr int stream_record(bool fp32) { return stream_ring(fp32) / 64 * 19; }
+constexpr int stream_entry(int kmax) { return kmax <= 4 ? 16 : 32; }
+struct StreamSet {
+    bool tried = false;               // built, or found not to fit
+    int kmax = 0;                     // most off-diagonal blocks of a row (0: not built)
+    int ent = 16;                     // bytes of a row entry
+    int nRec = 0;
+    std::vector<int32_t> recBeg, recMid;    // [nParts + 1], [nParts]: forward records [recBeg, recMid), backward to the next recBeg
+    std::vector<int32_t> recRows, recBlk;   // [nRec + 1] first row entry, first block
+    std::vector<uint16_t> entries;          // [rows][ent / 2]
+    std::vector<uint32_t> hdr, start;       // [nRec]; [nRec + 1] first 16-byte unit
+    std::vector<int32_t> src, rowCell;      // [blocks] block-CSR slot, or -(cell + 1) for Dinv; the row's cell in a backward record, else -1
+    DBuf<int32_t> d_recBeg, d_recMid, d_recRows, d_recBlk, d_src, d_rowCell;
+    DBuf<uint16_t> d_entries;
+    DBuf<uint32_t> d_hdr, d_start;
+    size_t bytes() const { return 16 * (size_t)start.back(); }
+    void upload();
 };
 
 // A set of compact cell partitions in sweep order: rows of partition p at
@@ -161,9 +168,9 @@ struct Mesh {
     // Spalart-Allmaras Gauss-Seidel sweep
     std::vector<int32_t> saPart;
     PartSet sa;
-    // coalesced streams of the partitioned ILU(0) apply (forward: the
-    // in-partition L blocks; backward: Dinv and Dinv U): see PiluStream
-    PiluStream pf, pb;
+    // the record streams of the partitioned ILU(0) apply, FP64 and FP32 (made
+    // by the first case that uses one)
+    StreamSet ps[2];
     // sliced-ELL copy of the block-CSR pattern for the SpMV: slices of 64
     // rows, slice s holds sellWidth[s] block columns; block p of row r sits at
     // block position sellPtr[s] + 64 p + (r - 64 s), its entry e at value
@@ -212,6 +219,7 @@ constexpr int kMaxPartLevels = 32;
 void mesh_build(Mesh& m, const rdst_mesh_desc* d, const rdst_mesh_geometry* g = nullptr);
 void build_partitions(Mesh& m, int maxCells);
 void mesh_upload(Mesh& m);
+StreamSet& mesh_stream(Mesh& m, bool fp32);  // the record stream, built and uploaded on first use
 
 // ---------------------------------------------------------------------------
 // Device-side views passed to kernels by value.

@@ -1,0 +1,89 @@
+"""The block ILU(0) factor and its sweeps against a dense-block numpy ILU(0) of
+the same system: one GMRES direction on A x = b from zero gives x parallel to
+M^-1 b, so the normalised x is the normalised M^-1 b whatever the scale."""
+import numpy as np
+import pytest
+
+from rhodst_amd import _capi, cases, meshgen
+
+pytestmark = pytest.mark.gpu
+
+# 1 cell, a record of 48 rows and its neighbours, several partitions, rows
+# with one to six lower blocks, chains longer than a partition's levels
+MESHES = {
+    "one": lambda: meshgen.box_2d(1, 1),
+    "line47": lambda: meshgen.channel_1d(47),
+    "line200": lambda: meshgen.channel_1d(200),
+    "box7x49": lambda: meshgen.box_2d(7, 49, jitter=0.2),
+    "box40": lambda: meshgen.box_2d(40, 40, jitter=0.2),
+    "step60": lambda: meshgen.forward_step(60, 20),
+    "tets": lambda: meshgen.tet_prism_box(7, 6, 8, prism_layers=3, jitter=0.1),
+    "wing": lambda: meshgen.swept_wing(n_wake=6, n_surf=12, n_normal=12, n_span_wing=6, n_span_out=3, n_layers=6),
+}
+
+
+def numpy_ilu(n, rows, diag, off, b):
+    """M^-1 b of the block ILU(0) on the given pattern: rows[i] = sorted
+    neighbours, off[(i, j)] = block."""
+    lu = {k: v.copy() for k, v in off.items()}
+    d = diag.copy()
+    dinv = np.zeros_like(diag)
+    for i in range(n):
+        for k in [k for k in rows[i] if k < i]:
+            lu[i, k] = lu[i, k] @ dinv[k]
+            for j in rows[k]:
+                if j <= k:
+                    continue
+                if j == i:
+                    d[i] -= lu[i, k] @ lu[k, j]
+                elif j in rows[i]:
+                    lu[i, j] -= lu[i, k] @ lu[k, j]
+        dinv[i] = np.linalg.inv(d[i])
+    y = b.copy()
+    for i in range(n):
+        for k in rows[i]:
+            if k < i:
+                y[i] -= lu[i, k] @ y[k]
+    for i in reversed(range(n)):
+        for j in rows[i]:
+            if j > i:
+                y[i] -= lu[i, j] @ y[j]
+        y[i] = dinv[i] @ y[i]
+    return y
+
+
+@pytest.mark.parametrize("order,precision,tol", [
+    # FP64: sweeps of at most a few hundred dependent rows of well conditioned blocks, ~1e3 eps; FP32: the same in its eps
+    ("natural", "fp64", 1e-12), ("partitioned", "fp64", 1e-12), ("partitioned", "mixed", 1e-4)])
+@pytest.mark.parametrize("name", sorted(MESHES))
+def test_one_direction_is_the_ilu_apply(name, order, precision, tol):
+    mesh = MESHES[name]()
+    dm = _capi.DeviceMesh(mesh)
+    n, nI = mesh.n_cells, len(mesh.neighbour)
+    rng = np.random.default_rng(len(name))
+    upper, lower = rng.uniform(-0.5, 0.5, (2, nI, 5, 5))
+    own, nei = np.asarray(mesh.owner[:nI]), np.asarray(mesh.neighbour)
+    diag = rng.uniform(-0.5, 0.5, (n, 5, 5)) + 8.0 * np.eye(5)
+    b = rng.standard_normal((n, 5))
+    kw = dict(n_directions=1, max_iter=1, min_iter=1, tolerance=0.0, rel_tol=0.0, ilu_order=order, precision=precision)
+    patches = {p[0]: {"p": "zeroGradient", "T": "zeroGradient", "U": "zeroGradient"} for p in mesh.patches if p[1] != 3}
+    from rhodst_amd._abi import make_bcs, make_settings, make_thermo
+    spec = cases.CaseSpec("ilu", mesh, make_thermo(), make_bcs(mesh, patches), make_settings(**kw),
+                          np.ones(n), np.ones(n), np.zeros((n, 3)))
+    dc = _capi.DeviceCase(spec, dm)
+    x, _ = dc.ldu_solve(diag, upper, lower, b, np.zeros((n, 5)))
+    part = dm.get_int(_capi.M_PARTITION) if order == "partitioned" else np.zeros(n, dtype=int)
+    rows, off = [set() for _ in range(n)], {}
+    for f in range(nI):
+        if part[own[f]] == part[nei[f]]:
+            rows[own[f]].add(nei[f])
+            rows[nei[f]].add(own[f])
+            off[own[f], nei[f]] = upper[f]
+            off[nei[f], own[f]] = lower[f]
+    ref = numpy_ilu(n, [sorted(r) for r in rows], diag, off, b)
+    x, ref = x.ravel() / np.linalg.norm(x), ref.ravel() / np.linalg.norm(ref)
+    err = np.abs(x * np.sign(x @ ref) - ref).max() / np.abs(ref).max()
+    assert err <= tol, (name, order, precision, err)
+    # the same system again: the sweeps leave no state behind
+    x2, _ = dc.ldu_solve(diag, upper, lower, b, np.zeros((n, 5)))
+    assert np.array_equal(x2.ravel() / np.linalg.norm(x2), x)
