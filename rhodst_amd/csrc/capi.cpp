@@ -297,6 +297,8 @@ int rdst_case_create(rdst_mesh* mesh, const rdst_thermo* thermo, const rdst_bc* 
         }
         if (s.precond == RDST_PRECOND_ILU0 && s.ilu_order == RDST_ILU_PARTITIONED)
             mesh_stream(*m, s.precision == RDST_PREC_MIXED);
+        if (s.precond == RDST_PRECOND_ILU0 && s.ilu_order == RDST_ILU_NATURAL)
+            mesh_tiles(*m, s.precision == RDST_PREC_MIXED);
         Case* c = new Case();
         try {
             c->mesh = m;

@@ -304,6 +304,126 @@ __global__ __launch_bounds__(STREAM_THREADS) void k_stream_apply(const int32_t* 
     scatter_rows(rows + rs, nl5, y, x);
 }
 
+// ---------------------------------------------------------------- natural order
+// The sweeps of the natural-order ILU(0) by tiles (TileSet).  Workgroups take
+// tiles in an order that respects their dependencies (a ticket counter), so a
+// tile only waits for tiles that running workgroups already hold, and the
+// launch ends whatever number of workgroups is resident.  A value another tile
+// needs is its own flag: the vector is filled with kUnset before the sweep, a
+// reader polls until the value has arrived (device-scope loads and stores), a
+// result with that bit pattern is stored as another NaN.
+// Against one launch per level (8-10 us each, or 3.3 us per level in a
+// single-workgroup run of small levels) a level costs 0.35 us inside a tile and
+// a tile about 4 us of waiting.  Measured per apply (both sweeps): see stream_launch.
+template <class T>
+struct Unset;
+template <>
+struct Unset<double> {
+    using U = unsigned long long;
+    static constexpr U bits = 0x7ffc5ad3e1b0972full;
+};
+template <>
+struct Unset<float> {
+    using U = unsigned int;
+    static constexpr U bits = 0x7fe5ad3eu;
+};
+template <class T>
+__device__ __forceinline__ typename Unset<T>::U load_dev(const T* p) {
+    return __hip_atomic_load(reinterpret_cast<const typename Unset<T>::U*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void store_dev(T* p, T v) {
+    using U = typename Unset<T>::U;
+    U u = __builtin_bit_cast(U, v);
+    if (u == Unset<T>::bits) u ^= 1;  // a NaN either way
+    __hip_atomic_store(reinterpret_cast<U*>(p), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__global__ __launch_bounds__(256) void k_fill_unset(long n, T* y, int* tickets) {
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
+        reinterpret_cast<typename Unset<T>::U*>(y)[i] = Unset<T>::bits;
+    if (blockIdx.x == 0 && threadIdx.x < 2) tickets[threadIdx.x] = 0;
+}
+
+// Values of the halo cells into LDS, each awaited.
+template <class TV>
+__device__ __forceinline__ void await_rows(const int32_t* cells, int n5, const TV* x, TV* y) {
+    constexpr int U = 4, ST = 64 * STREAM_WAVES;
+    for (int b = 0; b < n5; b += U * ST) {
+        int i[U];
+        typename Unset<TV>::U v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int t = min(b + u * ST + (int)threadIdx.x, n5 - 1);
+            i[u] = 5 * cells[t / 5] + t % 5;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = load_dev(x + i[u]);
+        for (;;) {
+            bool wait = false;
+#pragma unroll
+            for (int u = 0; u < U; ++u) wait |= v[u] == Unset<TV>::bits;
+            if (!__any(wait)) break;
+            __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (v[u] == Unset<TV>::bits) v[u] = load_dev(x + i[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int t = b + u * ST + (int)threadIdx.x;
+            if (t < n5) y[t] = __builtin_bit_cast(TV, v[u]);
+        }
+    }
+}
+
+// One sweep.  Forward: out = y from in = r, reset = x for the backward sweep.
+// Backward: out = x from in = y, reset = y for the next forward sweep.  Each
+// resets the other's ticket counter (the launches are ordered).
+template <class TM, class TV, int KDU, bool BWD>
+__global__ __launch_bounds__(STREAM_THREADS) void k_tile_sweep(int nT, int* tickets, const int32_t* __restrict__ rowStart,
+                                                               const int32_t* __restrict__ rows,
+                                                               const int32_t* __restrict__ haloStart,
+                                                               const int32_t* __restrict__ halo,
+                                                               const int32_t* __restrict__ recBeg,
+                                                               const int32_t* __restrict__ recMid,
+                                                               const uint32_t* __restrict__ hdr,
+                                                               const uint32_t* __restrict__ start,
+                                                               const uint8_t* __restrict__ stream, const TV* in, TV* out,
+                                                               TV* reset) {
+    constexpr int RING = stream_ring(sizeof(TM) == 4), ST = 64 * STREAM_WAVES;
+    extern __shared__ __align__(1024) unsigned char smem_raw[];
+    __shared__ int next[2];
+    uint8_t* ring = smem_raw;
+    TV* y = reinterpret_cast<TV*>(smem_raw + RING);
+    const bool loader = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == STREAM_WAVES;
+    if (threadIdx.x == 0) next[0] = atomicAdd(tickets + BWD, 1);
+    __syncthreads();
+    for (int round = 0;; ++round) {
+        const int ticket = __builtin_amdgcn_readfirstlane(next[round & 1]);
+        if (ticket >= nT) break;
+        const int tl = BWD ? nT - 1 - ticket : ticket;
+        const int r0 = BWD ? recMid[tl] : recBeg[tl], r1 = BWD ? recBeg[tl + 1] : recMid[tl];
+        if (loader) {
+            if (r1 > r0) stream_load<RING>(stream, start, r0, r1, ring);
+            if ((threadIdx.x & 63) == 0) next[(round + 1) & 1] = atomicAdd(tickets + BWD, 1);
+        } else {
+            if (ticket == 0 && threadIdx.x == 0) tickets[!BWD] = 0;
+            const int rs = rowStart[tl], nl5 = (rowStart[tl + 1] - rs) * 5;
+            const int h0 = haloStart[tl], nh5 = (haloStart[tl + 1] - h0) * 5;
+            gather_rows(rows + rs, nl5, in, y);
+            await_rows(halo + h0, nh5, (const TV*)out, y + nl5);
+            if (r1 > r0) stream_compute<TM, TV, KDU, RING>(hdr, r0, BWD ? 0 : r1 - r0, r1 - r0, ring, y);
+            // (no record: every thread stores the entries that it gathered itself)
+            for (int t = threadIdx.x; t < nl5; t += ST) {
+                const size_t i = 5 * (size_t)rows[rs + t / 5] + t % 5;
+                store_dev(out + i, y[t]);
+                reinterpret_cast<typename Unset<TV>::U*>(reset)[i] = Unset<TV>::bits;
+            }
+        }
+        __syncthreads();
+    }
+}
 // the row entries of every record into the stream (once per buffer)
 __global__ __launch_bounds__(64) void k_stream_entries(int ent, const int32_t* recRows, const uint4* entries,
                                                        const uint32_t* start, uint8_t* stream) {

@@ -60,15 +60,23 @@ void rcb(const std::vector<double>& C, std::vector<int>& idx, int lo, int hi, in
 
 }  // namespace
 
-// The record stream of the partitioned ILU(0) apply, in the layout StreamSet
-// describes.  Left empty (kmax = 0) when a row has more than kStreamKD
-// off-diagonal blocks in one sweep or the stream passes 64 GiB.
-static void build_stream(const Mesh& m, bool fp32, StreamSet& ps) {
+// The partitions of an ILU(0) apply as build_stream reads them (PartSet).
+struct PartView {
+    int nParts;
+    const std::vector<int32_t>&rowStart, &rows, &levStart, &levPtr, &localCol;
+};
+
+// The record stream of an ILU(0) apply, in the layout StreamSet describes.
+// split: the two sweeps of a partition are read by separate launches, so the
+// backward records start a ring of their own.  Left empty (kmax = 0) when a row
+// has more than kStreamKD off-diagonal blocks in one sweep or the stream passes
+// 64 GiB.
+static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp32, StreamSet& ps) {
     int kmax = 1;
     for (int i = 0; i < m.nC; ++i) {
         int lo = 0, up = 0;
         for (int s = m.rowPtr[i]; s < m.rowPtr[i + 1]; ++s)
-            if (m.localCol[s] >= 0 && s != m.slotDiag[i]) (s < m.slotDiag[i] ? lo : up)++;
+            if (pv.localCol[s] >= 0 && s != m.slotDiag[i]) (s < m.slotDiag[i] ? lo : up)++;
         kmax = std::max(kmax, std::max(lo, up));
     }
     if (kmax > kStreamKD) return;
@@ -83,20 +91,23 @@ static void build_stream(const Mesh& m, bool fp32, StreamSet& ps) {
     ps.recBlk.assign(1, 0);
     size_t pos = 0;
     auto size_of = [&](int nr, int nb) { return nr * ps.ent + ((nb * blk + 15) & ~15); };
-    for (int p = 0; p < m.nParts; ++p) {
-        const int rs = m.partRowStart[p];
-        const int l0 = m.partLevStart[p], nl = m.partLevStart[p + 1] - l0 - 1;
-        const size_t base = pos;
+    for (int p = 0; p < pv.nParts; ++p) {
+        const int rs = pv.rowStart[p];
+        const int l0 = pv.levStart[p], nl = pv.levStart[p + 1] - l0 - 1;
+        size_t base = pos;
         for (int sweep = 0; sweep < 2; ++sweep) {
-            if (sweep == 1) ps.recMid.push_back((int32_t)ps.hdr.size());
+            if (sweep == 1) {
+                ps.recMid.push_back((int32_t)ps.hdr.size());
+                if (split) base = pos = (pos + 1023) & ~(size_t)1023;
+            }
             for (int li = 0; li < nl; ++li) {
                 const int L = sweep ? nl - 1 - li : li;
                 rows.clear();
-                for (int t = m.partLevPtr[l0 + L]; t < m.partLevPtr[l0 + L + 1]; ++t) {
-                    const int i = m.partRows[t];
+                for (int t = pv.levPtr[l0 + L]; t < pv.levPtr[l0 + L + 1]; ++t) {
+                    const int i = pv.rows[t];
                     const int s0 = sweep ? m.slotDiag[i] + 1 : m.rowPtr[i], s1 = sweep ? m.rowPtr[i + 1] : m.slotDiag[i];
                     int cnt = 0;
-                    for (int s = s0; s < s1; ++s) cnt += m.localCol[s] >= 0;
+                    for (int s = s0; s < s1; ++s) cnt += pv.localCol[s] >= 0;
                     if (sweep || cnt) rows.push_back({t - rs, i, cnt});  // forward: y = r on a row without L
                 }
                 // rows of one block count together: a wavefront's rows run the same products
@@ -132,10 +143,10 @@ static void build_stream(const Mesh& m, bool fp32, StreamSet& ps) {
                         const int s0 = sweep ? m.slotDiag[w.i] + 1 : m.rowPtr[w.i],
                                   s1 = sweep ? m.rowPtr[w.i + 1] : m.slotDiag[w.i];
                         for (int s = s0; s < s1; ++s)
-                            if (m.localCol[s] >= 0) {
+                            if (pv.localCol[s] >= 0) {
                                 ps.src.push_back(s);
                                 ps.rowCell.push_back(sweep ? w.i : -1);
-                                e[k++] = (uint16_t)(5 * m.localCol[s]);
+                                e[k++] = (uint16_t)(5 * pv.localCol[s]);
                             }
                         first += w.cnt + sweep;
                     }
@@ -173,7 +184,7 @@ void StreamSet::upload() {
 StreamSet& mesh_stream(Mesh& m, bool fp32) {
     StreamSet& ps = m.ps[fp32];
     if (!ps.tried) {
-        build_stream(m, fp32, ps);
+        build_stream(m, {m.nParts, m.partRowStart, m.partRows, m.partLevStart, m.partLevPtr, m.localCol}, false, fp32, ps);
         ps.upload();
         ps.tried = true;
     }
@@ -262,6 +273,136 @@ static void order_partitions(const Mesh& m, const std::vector<int32_t>& part, in
     for (int c = 0; c < n; ++c)
         for (int s = m.rowPtr[c]; s < m.rowPtr[c + 1]; ++s)
             if (part[m.cols[s]] == part[c]) ps.localCol[s] = local[m.cols[s]];
+}
+
+// Tiles of the natural-order ILU(0).  Every lower neighbour of a row gets a
+// class by how far back in the numbering it lies (next to it, or one of two
+// groups of larger distances; i, j and k neighbours of a structured numbering);
+// coordinate c of a row is the largest number of class-c steps on a chain of
+// dependencies ending there.  All three never decrease along a dependency, so
+// boxes in them form an acyclic tile graph whatever the mesh, and on a
+// structured numbering they are boxes of its indices, the shape with the
+// shortest chain of tiles.  A box of more than kTileCells rows is cut by level.
+static void build_tiles(const Mesh& m, TileSet& ts) {
+    const int n = m.nC;
+    double lmin = 1e300, lmax = 0.0;
+    std::vector<double> hist(32 * 8, 0.0);
+    auto bin_of = [&](int d) { return std::min((int)hist.size() - 1, (int)(8.0 * std::log2((double)d))); };
+    for (int i = 0; i < n; ++i)
+        for (int s = m.rowPtr[i]; s < m.slotDiag[i]; ++s) {
+            const int d = i - m.cols[s];
+            if (d <= 1) continue;
+            hist[bin_of(d)] += 1.0;
+            lmin = std::min(lmin, std::log2((double)d));
+            lmax = std::max(lmax, std::log2((double)d));
+        }
+    // two groups of log(distance) by 2-means; one group when they are within a factor of four
+    double c0 = lmin, c1 = lmax;
+    for (int it = 0; it < 20; ++it) {
+        double s0 = 0, w0 = 0, s1 = 0, w1 = 0;
+        for (size_t q = 0; q < hist.size(); ++q) {
+            const double x = (q + 0.5) / 8.0;
+            if (std::fabs(x - c0) <= std::fabs(x - c1)) { s0 += hist[q] * x; w0 += hist[q]; }
+            else { s1 += hist[q] * x; w1 += hist[q]; }
+        }
+        if (w0 > 0) c0 = s0 / w0;
+        if (w1 > 0) c1 = s1 / w1;
+    }
+    const bool three = c1 - c0 > 2.0;
+    const double cut = 0.5 * (c0 + c1);
+    std::vector<int32_t> x(3 * (size_t)n, 0), lev(n, 0);
+    for (int i = 0; i < n; ++i)
+        for (int s = m.rowPtr[i]; s < m.slotDiag[i]; ++s) {
+            const int j = m.cols[s], d = i - j;
+            const int cl = d <= 1 ? 0 : (three && std::log2((double)d) > cut ? 2 : 1);
+            for (int c = 0; c < 3; ++c) x[3 * (size_t)i + c] = std::max(x[3 * (size_t)i + c], x[3 * (size_t)j + c] + (c == cl ? 1 : 0));
+            lev[i] = std::max(lev[i], lev[j] + 1);
+        }
+    const int T[3] = {three ? 8 : 16, three ? 8 : 16, 8};
+    std::vector<int32_t> tile(n, 0);
+    int nT = 0;
+    if (n <= kPartCells) {
+        nT = n ? 1 : 0;
+    } else {
+        // cells by (wavefront of boxes, box, level, index)
+        struct Key {
+            int32_t sum, k0, k1, k2, lev, c;
+        };
+        std::vector<Key> key(n);
+        for (int i = 0; i < n; ++i) {
+            const int32_t k0 = x[3 * (size_t)i] / T[0], k1 = x[3 * (size_t)i + 1] / T[1], k2 = x[3 * (size_t)i + 2] / T[2];
+            key[i] = {k0 + k1 + k2, k0, k1, k2, lev[i], i};
+        }
+        std::sort(key.begin(), key.end(), [](const Key& a, const Key& b) {
+            if (a.sum != b.sum) return a.sum < b.sum;
+            if (a.k0 != b.k0) return a.k0 < b.k0;
+            if (a.k1 != b.k1) return a.k1 < b.k1;
+            if (a.k2 != b.k2) return a.k2 < b.k2;
+            return a.lev != b.lev ? a.lev < b.lev : a.c < b.c;
+        });
+        int cnt = 0;
+        for (int q = 0; q < n; ++q) {
+            const Key &k = key[q], &p = key[q ? q - 1 : 0];
+            const bool box = q == 0 || k.sum != p.sum || k.k0 != p.k0 || k.k1 != p.k1 || k.k2 != p.k2;
+            if (box || cnt == kTileCells) {
+                ++nT;
+                cnt = 0;
+            }
+            tile[k.c] = nT - 1;
+            ++cnt;
+        }
+    }
+    order_partitions(m, tile, nT, ts);
+    // columns outside the tile: halo cells, each once per tile and sweep
+    ts.haloFStart.assign(1, 0);
+    ts.haloBStart.assign(1, 0);
+    std::vector<int32_t> seen(n, -1), slot(n, 0);
+    for (int sweep = 0; sweep < 2; ++sweep) {
+        std::vector<int32_t>&hs = sweep ? ts.haloBStart : ts.haloFStart, &h = sweep ? ts.haloB : ts.haloF;
+        std::fill(seen.begin(), seen.end(), -1);
+        for (int t = 0; t < nT; ++t) {
+            const int rs = ts.rowStart[t], nr = ts.rowStart[t + 1] - rs;
+            for (int q = rs; q < rs + nr; ++q) {
+                const int i = ts.rows[q];
+                const int s0 = sweep ? m.slotDiag[i] + 1 : m.rowPtr[i], s1 = sweep ? m.rowPtr[i + 1] : m.slotDiag[i];
+                for (int s = s0; s < s1; ++s) {
+                    const int j = m.cols[s];
+                    if (tile[j] == t) continue;
+                    if (seen[j] != t) {
+                        seen[j] = t;
+                        slot[j] = nr + (int)h.size() - hs.back();
+                        h.push_back(j);
+                    }
+                    ts.localCol[s] = slot[j];
+                }
+            }
+            hs.push_back((int32_t)h.size());
+            ts.maxSlots = std::max(ts.maxSlots, nr + hs[t + 1] - hs[t]);
+        }
+    }
+}
+
+TileSet& mesh_tiles(Mesh& m, bool fp32) {
+    TileSet& ts = m.tiles;
+    if (!ts.tried) {
+        build_tiles(m, ts);
+        ts.d_rowStart.upload(ts.rowStart);
+        ts.d_rows.upload(ts.rows);
+        ts.d_haloFStart.upload(ts.haloFStart);
+        ts.d_haloF.upload(ts.haloF);
+        ts.d_haloBStart.upload(ts.haloBStart);
+        ts.d_haloB.upload(ts.haloB);
+        // the tile's vector and its halo next to the ring in 160 KB of LDS, 16-bit columns
+        ts.ok = 40 * (size_t)ts.maxSlots + stream_ring(false) + 4096 <= 160 * 1024;
+        ts.tried = true;
+    }
+    StreamSet& ps = ts.ps[fp32];
+    if (!ps.tried && ts.ok) {
+        build_stream(m, {ts.nParts, ts.rowStart, ts.rows, ts.levStart, ts.levPtr, ts.localCol}, ts.nParts > 1, fp32, ps);
+        ps.upload();
+    }
+    ps.tried = true;
+    return ts;
 }
 
 // Partitions for the block-Jacobi ILU(0): couplings between partitions are

@@ -128,6 +128,21 @@ struct PartSet {
     DBuf<int32_t> d_rowStart, d_rows, d_levStart, d_levPtr, d_localCol;
 };
 
+// The natural-order ILU(0) in tiles: sets of cells whose dependency graph has
+// no cycle, in an order that respects it, so that tiles taken in that order
+// only ever wait for tiles taken before (backward: in reverse).  As a PartSet,
+// with localCol numbering the cells outside the tile that a row reads behind
+// the tile's own: halo cell q of tile t's forward sweep is haloF[haloFStart[t]
+// + q], column nRows(t) + q.
+struct TileSet : PartSet {
+    bool tried = false, ok = false;
+    int maxSlots = 0;  // most rows + halo cells of a tile
+    std::vector<int32_t> haloFStart, haloF, haloBStart, haloB;
+    DBuf<int32_t> d_haloFStart, d_haloF, d_haloBStart, d_haloB;
+    StreamSet ps[2];   // FP64, FP32
+};
+constexpr int kTileCells = 512;  // most rows of a tile
+
 struct Mesh {
     int nC = 0, nI = 0, nB = 0, nF = 0;  // nF = nI + nB surface-field length
     int nPatches = 0;
@@ -171,6 +186,7 @@ struct Mesh {
     // the record streams of the partitioned ILU(0) apply, FP64 and FP32 (made
     // by the first case that uses one)
     StreamSet ps[2];
+    TileSet tiles;  // of the natural-order ILU(0), made by the first case that uses it
     // sliced-ELL copy of the block-CSR pattern for the SpMV: slices of 64
     // rows, slice s holds sellWidth[s] block columns; block p of row r sits at
     // block position sellPtr[s] + 64 p + (r - 64 s), its entry e at value
@@ -220,6 +236,7 @@ void mesh_build(Mesh& m, const rdst_mesh_desc* d, const rdst_mesh_geometry* g = 
 void build_partitions(Mesh& m, int maxCells);
 void mesh_upload(Mesh& m);
 StreamSet& mesh_stream(Mesh& m, bool fp32);  // the record stream, built and uploaded on first use
+TileSet& mesh_tiles(Mesh& m, bool fp32);     // the tiles and their record stream, likewise
 
 // ---------------------------------------------------------------------------
 // Device-side views passed to kernels by value.

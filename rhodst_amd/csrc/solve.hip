@@ -40,6 +40,9 @@ struct SolverWork {
     DBuf<double> partA, partB; // reduction partials
     DBuf<double> multi;        // classical Gram-Schmidt partials [nDirs+1][G]
     DBuf<uint8_t> st64, st32;  // the ILU(0) apply's record stream in FP64 / FP32
+    DBuf<double> ty64;         // natural-order sweeps by tiles: the forward result, unset between applies
+    DBuf<float> ty32;
+    DBuf<int> tickets;
     std::vector<double> hscal;
     // BiCGStab
     DBuf<double> p, ph, v, t, th, rw;
@@ -1003,22 +1006,43 @@ void stream_pack(Ctx& k, const StreamSet& ps, const T* LU, const T* Dinv) {
                        ps.d_src.p, ps.d_rowCell.p, ps.d_start.p, LU, Dinv, buf.p);
 }
 
-// x = M^-1 r from the record stream
+// x = M^-1 r from the record stream: one workgroup per partition, or the
+// natural-order sweeps by tiles (a mesh that is one tile is one partition)
+static DBuf<double>& tile_y(SolverWork& w, const double*) { return w.ty64; }
+static DBuf<float>& tile_y(SolverWork& w, const float*) { return w.ty32; }
 template <class TM, class TV, int KDU>
-void stream_launch(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV* r, TV* x) {
+void stream_launch(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV* r, TV* x, bool natural) {
     Mesh& m = k.m;
+    const TileSet& ts = m.tiles;
+    const int slots = natural ? ts.maxSlots : m.maxPartRows;
     // lanes read KDU + 1 blocks from wherever their row starts: room for them past a short partition's vector
-    const size_t shmem = stream_ring(sizeof(TM) == 4) +
-                         std::max(sizeof(TV) * 5 * (size_t)m.maxPartRows, sizeof(TM) * 25 * (KDU + 1));
-    hipLaunchKernelGGL((k_stream_apply<TM, TV, KDU>), dim3(m.nParts), dim3(STREAM_THREADS), shmem, k.s,
-                       m.d_partRowStart.p, m.d_partRows.p, ps.d_recBeg.p, ps.d_recMid.p, ps.d_hdr.p, ps.d_start.p,
-                       stream, r, x);
+    const size_t shmem = stream_ring(sizeof(TM) == 4) + std::max(sizeof(TV) * 5 * (size_t)slots, sizeof(TM) * 25 * (KDU + 1));
+    if (!natural || ts.nParts == 1) {
+        hipLaunchKernelGGL((k_stream_apply<TM, TV, KDU>), dim3(natural ? 1 : m.nParts), dim3(STREAM_THREADS), shmem, k.s,
+                           natural ? ts.d_rowStart.p : m.d_partRowStart.p, natural ? ts.d_rows.p : m.d_partRows.p,
+                           ps.d_recBeg.p, ps.d_recMid.p, ps.d_hdr.p, ps.d_start.p, stream, r, x);
+        return;
+    }
+    auto& ty = tile_y(k.w, (const TV*)nullptr);
+    const size_t n5 = 5 * (size_t)m.nC;
+    if (ty.n != n5) {
+        ty.alloc(n5);
+        k.w.tickets.alloc(2);
+        hipLaunchKernelGGL((k_fill_unset<TV>), dim3(RED_MAXG), dim3(256), 0, k.s, (long)n5, ty.p, k.w.tickets.p);
+    }
+    const int grid = std::min(ts.nParts, 256);
+    hipLaunchKernelGGL((k_tile_sweep<TM, TV, KDU, false>), dim3(grid), dim3(STREAM_THREADS), shmem, k.s, ts.nParts,
+                       k.w.tickets.p, ts.d_rowStart.p, ts.d_rows.p, ts.d_haloFStart.p, ts.d_haloF.p, ps.d_recBeg.p,
+                       ps.d_recMid.p, ps.d_hdr.p, ps.d_start.p, stream, r, ty.p, x);
+    hipLaunchKernelGGL((k_tile_sweep<TM, TV, KDU, true>), dim3(grid), dim3(STREAM_THREADS), shmem, k.s, ts.nParts,
+                       k.w.tickets.p, ts.d_rowStart.p, ts.d_rows.p, ts.d_haloBStart.p, ts.d_haloB.p, ps.d_recBeg.p,
+                       ps.d_recMid.p, ps.d_hdr.p, ps.d_start.p, stream, (const TV*)ty.p, x, ty.p);
 }
 template <class TM, class TV>
-void stream_apply(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV* r, TV* x) {
-    if (ps.kmax <= 3) stream_launch<TM, TV, 3>(k, ps, stream, r, x);
-    else if (ps.kmax <= 4) stream_launch<TM, TV, 4>(k, ps, stream, r, x);
-    else stream_launch<TM, TV, kStreamKD>(k, ps, stream, r, x);
+void stream_apply(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV* r, TV* x, bool natural) {
+    if (ps.kmax <= 3) stream_launch<TM, TV, 3>(k, ps, stream, r, x, natural);
+    else if (ps.kmax <= 4) stream_launch<TM, TV, 4>(k, ps, stream, r, x, natural);
+    else stream_launch<TM, TV, kStreamKD>(k, ps, stream, r, x, natural);
 }
 
 template <class T>
@@ -1047,6 +1071,8 @@ void ilu_factor(Ctx& k, const T* A, T* LU, T* Dinv) {
                                    fail);
             }
         }
+        const StreamSet& ps = mesh_tiles(m, sizeof(T) == 4).ps[sizeof(T) == 4];
+        if (ps.kmax > 0) stream_pack<T>(k, ps, LU, Dinv);
     } else if (k.c.st.precond == RDST_PRECOND_DIAG) {
         hipLaunchKernelGGL((k_diag_inv<T>), dim3(blocks_for(m.nC, 256)), dim3(256), 0, k.s, m.nC, m.d_slotDiag.p, A, Dinv,
                            fail);
@@ -1075,7 +1101,7 @@ void precondition(Ctx& k, const TM* LU, const TM* Dinv, const TV* r, TV* x, TV* 
         const size_t shmem = sizeof(TV) * 5 * (size_t)m.maxPartRows;
         const StreamSet& ps = m.ps[sizeof(TM) == 4];
         if (ps.kmax > 0) {
-            stream_apply<TM, TV>(k, ps, stream_buf(k.w, LU).p, r, x);
+            stream_apply<TM, TV>(k, ps, stream_buf(k.w, LU).p, r, x, false);
             return;
         }
         if (sizeof(TM) == 4)
@@ -1088,6 +1114,12 @@ void precondition(Ctx& k, const TM* LU, const TM* Dinv, const TV* r, TV* x, TV* 
                                m.d_cols.p, m.d_slotDiag.p, m.d_localCol.p, LU, Dinv, r, x);
         return;
     }
+    const StreamSet& ns = m.tiles.ps[sizeof(TM) == 4];
+    if (ns.kmax > 0) {
+        stream_apply<TM, TV>(k, ns, stream_buf(k.w, LU).p, r, x, true);
+        return;
+    }
+    // tiles too wide for LDS, or rows too long for the stream: level by level
     for (const LevelRun& g : m.runL) {
         if (g.fused) {
             hipLaunchKernelGGL((k_ilu_fwd_seg<TM, TV>), dim3(1), dim3(ILU_SEG_THREADS), 0, k.s, g.L0, g.L1,

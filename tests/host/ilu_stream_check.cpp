@@ -1,0 +1,156 @@
+// Host-side check of the ILU(0) record streams and of the tiles of the
+// natural-order sweeps: replays the streams on the CPU with one number per
+// block and compares with the plain sweeps over the block-CSR pattern.
+#include "../../rhodst_amd/csrc/mesh_host.cpp"
+
+#include <cstdio>
+
+namespace rdst {
+void set_error(const std::string&) {}
+}  // namespace rdst
+using namespace rdst;
+
+static std::string g_what;
+static int fail(const char* what, long a = 0, long b = 0) {
+    char s[200];
+    std::snprintf(s, sizeof s, "%s (%ld, %ld)", what, a, b);
+    g_what = s;
+    return 1;
+}
+static double coef(int s) { return 0.05 + 0.1 * ((s * 2654435761u) % 1000) / 1000.0; }
+static double dinv(int c) { return 0.5 + 0.3 * ((c * 40503u) % 1000) / 1000.0; }
+
+// one sweep's records over a partition's vector y (rows, then halo values)
+static int replay(const Mesh& m, const StreamSet& ps, bool fp32, int q0, int q1, bool bwd, int slots, std::vector<double>& y) {
+    const int blk = 25 * (fp32 ? 4 : 8);
+    for (int q = q0; q < q1; ++q) {
+        const int nr = ps.recRows[q + 1] - ps.recRows[q], b0 = ps.recBlk[q], nb = ps.recBlk[q + 1] - b0;
+        if ((int)(ps.hdr[q] & 0xffff) != nr || nr < 1 || nr > kStreamRows) return fail("rows of a record", q, nr);
+        if (nr * ps.ent + ((nb * blk + 15) & ~15) > stream_record(fp32)) return fail("record too large", q);
+        std::vector<double> nw(nr);
+        for (int j = 0; j < nr; ++j) {
+            const uint16_t* e = ps.entries.data() + (size_t)(ps.recRows[q] + j) * (ps.ent / 2);
+            const int t = e[0] / 5, cnt = e[1] >> 8;
+            int b = b0 + (e[1] & 0xff);
+            double a = y[t];
+            double d = 1.0;
+            if (bwd) {
+                if (ps.src[b] >= 0) return fail("no Dinv first", q, j);
+                d = dinv(-ps.src[b] - 1);
+                if (ps.rowCell[b] != -ps.src[b] - 1) return fail("row cell", q, j);
+                a *= d;
+                ++b;
+            }
+            for (int k = 0; k < cnt; ++k, ++b) {
+                if (b >= ps.recBlk[q + 1]) return fail("block outside its record", q, j);
+                if (e[2 + k] % 5 || e[2 + k] / 5 >= slots) return fail("column out of range", q, e[2 + k]);
+                if (bwd != (ps.rowCell[b] >= 0)) return fail("sweep of a block", q, j);
+                a -= d * coef(ps.src[b]) * y[e[2 + k] / 5];
+            }
+            nw[j] = a;
+        }
+        // rows of a record are independent: storing them together changes nothing
+        for (int j = 0; j < nr; ++j) y[ps.entries[(size_t)(ps.recRows[q] + j) * (ps.ent / 2)] / 5] = nw[j];
+    }
+    return 0;
+}
+
+static int check(const rdst_mesh_desc* desc, bool fp32, bool natural) {
+    Mesh m;
+    mesh_build(m, desc);
+    const int n = m.nC;
+    TileSet ts;
+    StreamSet ps;
+    std::vector<int32_t> part(m.part);
+    if (natural) {
+        build_tiles(m, ts);
+        build_stream(m, {ts.nParts, ts.rowStart, ts.rows, ts.levStart, ts.levPtr, ts.localCol}, ts.nParts > 1, fp32, ps);
+        std::fill(part.begin(), part.end(), 0);
+    } else {
+        build_stream(m, {m.nParts, m.partRowStart, m.partRows, m.partLevStart, m.partLevPtr, m.localCol}, false, fp32, ps);
+    }
+    if (ps.kmax == 0) return fail("not built");
+    const int nP = natural ? ts.nParts : m.nParts;
+    const std::vector<int32_t>&rowStart = natural ? ts.rowStart : m.partRowStart, &rows = natural ? ts.rows : m.partRows;
+    // what the loader relies on: partitions at 1 KB, records inside the ring, three of them at once
+    const int ring = stream_ring(fp32) / 16;
+    const bool split = natural && nP > 1;  // each sweep a launch of its own
+    for (int p = 0; p < nP; ++p)
+        for (int part2 = 0; part2 < (split ? 2 : 1); ++part2) {
+            const int q0 = part2 ? ps.recMid[p] : ps.recBeg[p], q1 = split && !part2 ? ps.recMid[p] : ps.recBeg[p + 1];
+            if (q0 == q1) continue;
+            const uint32_t base = ps.start[q0];
+            if (base % 64) return fail("start of a sweep", p);
+            // the last 1 KB piece ends inside the stream
+            if (16 * (size_t)(base + (ps.start[q1] - base + 63) / 64 * 64) > ps.bytes()) return fail("past the stream's end", p);
+            uint32_t off = 0;
+            for (int q = q0; q < q1; ++q) {
+                const int nr = ps.recRows[q + 1] - ps.recRows[q], nb = ps.recBlk[q + 1] - ps.recBlk[q];
+                const int len = (nr * ps.ent + ((nb * 25 * (fp32 ? 4 : 8) + 15) & ~15)) / 16;
+                if (off != ps.start[q] - base) return fail("distances do not add up", q);
+                off += ps.hdr[q] >> 16;
+                if ((int)((ps.start[q] - base) % ring) + len > ring) return fail("record crosses the ring's end", q);
+                // while record q + 1 is read, record q + 3 arrives
+                const uint32_t a = ps.start[std::min(q + 1, q1)] - base, b = ps.start[std::min(q + 4, q1)] - base;
+                if ((b + 63) / 64 > a / 64 + ring / 64) return fail("three records do not fit the ring", q);
+            }
+        }
+    // the plain sweeps
+    std::vector<double> r(n), y(n), x(n), yr(n), xr(n);
+    for (int i = 0; i < n; ++i) r[i] = std::sin(1.0 + 0.37 * i);
+    for (int i = 0; i < n; ++i) {
+        yr[i] = r[i];
+        for (int s = m.rowPtr[i]; s < m.slotDiag[i]; ++s)
+            if (part[m.cols[s]] == part[i]) yr[i] -= coef(s) * yr[m.cols[s]];
+    }
+    for (int i = n - 1; i >= 0; --i) {
+        double a = yr[i];
+        for (int s = m.slotDiag[i] + 1; s < m.rowPtr[i + 1]; ++s)
+            if (part[m.cols[s]] == part[i]) a -= coef(s) * xr[m.cols[s]];
+        xr[i] = dinv(i) * a;
+    }
+    // the streams, tiles in ticket order: a halo value must have been stored before it is read
+    std::vector<char> have(n, 0);
+    for (int sweep = 0; sweep < 2; ++sweep) {
+        std::fill(have.begin(), have.end(), 0);
+        for (int t = 0; t < nP; ++t) {
+            const int p = sweep ? nP - 1 - t : t;
+            const int rs = rowStart[p], nr = rowStart[p + 1] - rs;
+            std::vector<double> v(nr);
+            for (int q = 0; q < nr; ++q) v[q] = sweep ? y[rows[rs + q]] : r[rows[rs + q]];
+            if (natural) {
+                const std::vector<int32_t>&hs = sweep ? ts.haloBStart : ts.haloFStart, &h = sweep ? ts.haloB : ts.haloF;
+                for (int q = hs[p]; q < hs[p + 1]; ++q) {
+                    if (!have[h[q]]) return fail("a tile reads a cell of a later tile", p, h[q]);
+                    v.push_back((sweep ? x : y)[h[q]]);
+                }
+                if ((int)v.size() > ts.maxSlots) return fail("slots", p);
+            }
+            const int q0 = sweep ? ps.recMid[p] : ps.recBeg[p], q1 = sweep ? ps.recBeg[p + 1] : ps.recMid[p];
+            if (int e = replay(m, ps, fp32, q0, q1, sweep != 0, (int)v.size(), v)) return e;
+            for (int q = 0; q < nr; ++q) {
+                (sweep ? x : y)[rows[rs + q]] = v[q];
+                have[rows[rs + q]] = 1;
+            }
+        }
+        for (int i = 0; i < n; ++i)
+            if (!have[i]) return fail("a cell is in no partition", i);
+    }
+    double scale = 1e-300;
+    for (int i = 0; i < n; ++i) scale = std::max(scale, std::fabs(xr[i]));
+    for (int i = 0; i < n; ++i)
+        if (!(std::fabs(x[i] - xr[i]) <= 1e-12 * scale)) return fail("sweep result differs", i);
+    return 0;
+}
+
+extern "C" int ilu_stream_check(const rdst_mesh_desc* desc, int fp32, int natural, char* what, int len) {
+    g_what.clear();
+    int rc = 2;
+    try {
+        rc = check(desc, fp32 != 0, natural != 0);
+    } catch (const std::exception& e) {
+        g_what = e.what();
+    }
+    std::snprintf(what, len, "%s", g_what.c_str());
+    return rc;
+}

@@ -1,0 +1,76 @@
+"""The ILU(0) record streams and the tiles of the natural-order sweeps,
+replayed on the CPU (tests/host/ilu_stream_check.cpp) over meshes of every
+numbering: structured, curvilinear with a wake cut, hybrid, tetrahedra, and
+the same cells numbered at random."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from rhodst_amd import meshgen
+from rhodst_amd._abi import MeshDesc, rdst_mesh_desc
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def checker(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host") / "ilu_stream_check.so")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I", f"{rocm}/include",
+                    "-I", os.path.join(HERE, "..", "include"), os.path.join(HERE, "host", "ilu_stream_check.cpp"),
+                    "-L", f"{rocm}/lib", "-lamdhip64", f"-Wl,-rpath,{rocm}/lib", "-o", so], check=True)
+    lib = C.CDLL(so)
+    lib.ilu_stream_check.argtypes = [C.POINTER(rdst_mesh_desc), C.c_int, C.c_int, C.c_char_p, C.c_int]
+    return lib
+
+
+def shuffled(mesh, seed):
+    """The same cells in a random order (owner/neighbour of a face swapped to
+    keep the lower cell its owner, faces in upper-triangular order)."""
+    rng = np.random.default_rng(seed)
+    p = rng.permutation(mesh.n_cells)
+    own, nei = p[np.asarray(mesh.owner)], p[np.asarray(mesh.neighbour)]
+    nI = len(nei)
+    fp = [list(mesh.face_points[mesh.face_offsets[f]:mesh.face_offsets[f + 1]]) for f in range(len(own))]
+    for f in range(nI):
+        if own[f] > nei[f]:
+            own[f], nei[f] = nei[f], own[f]
+            fp[f] = fp[f][:1] + fp[f][:0:-1]
+    order = np.concatenate([np.lexsort((nei, own[:nI])), np.arange(nI, len(own))])
+    fp = [fp[f] for f in order]
+    import copy
+    m = copy.copy(mesh)
+    m.owner, m.neighbour = own[order].astype(np.int32), nei[order[:nI]].astype(np.int32)
+    m.face_points = np.concatenate([np.asarray(q) for q in fp]).astype(np.int32)
+    m.face_offsets = np.concatenate([[0], np.cumsum([len(q) for q in fp])]).astype(np.int32)
+    return m
+
+
+MESHES = {
+    "one cell": lambda: meshgen.box_2d(1, 1),
+    "line": lambda: meshgen.channel_1d(2500),
+    "box 33x31": lambda: meshgen.box_2d(33, 31, jitter=0.2),  # 1023 cells: one tile
+    "box 25x41": lambda: meshgen.box_2d(25, 41, jitter=0.2),  # 1025: several
+    "box 150x70": lambda: meshgen.box_2d(150, 70, jitter=0.2),
+    "step": lambda: meshgen.forward_step(120, 40),
+    "hybrid airfoil": lambda: meshgen.hybrid_airfoil(n_surf=80, n_layers=16, first_cell=2e-5, far=8.0),
+    "wing": lambda: meshgen.swept_wing(n_wake=13, n_surf=30, n_normal=21, n_span_wing=9, n_span_out=5, n_layers=8),
+    "wing tiles": lambda: meshgen.swept_wing(n_wake=6, n_surf=16, n_normal=16, n_span_wing=8, n_span_out=4, n_layers=8,
+                                             order="tiles"),
+    "tets": lambda: meshgen.tet_prism_box(11, 13, 12, prism_layers=3, jitter=0.1),
+    "box shuffled": lambda: shuffled(meshgen.box_2d(60, 45, jitter=0.2), 1),
+    "tets shuffled": lambda: shuffled(meshgen.tet_prism_box(7, 6, 8, prism_layers=3, jitter=0.1), 2),
+}
+
+
+@pytest.mark.parametrize("name", sorted(MESHES))
+def test_streams_and_tiles(checker, name):
+    md = MeshDesc(MESHES[name]())
+    what = C.create_string_buffer(256)
+    for fp32 in (0, 1):
+        for natural in (0, 1):
+            rc = checker.ilu_stream_check(C.byref(md.desc), fp32, natural, what, 256)
+            assert rc == 0, (name, fp32, natural, what.value.decode())
