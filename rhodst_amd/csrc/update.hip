@@ -13,6 +13,7 @@
 // T-derived enthalpy coefficients, from the new rho/U and the not-yet-
 // corrected p, T, psi; (2) the cell update; (3) h_b, T_b, psi_b, p_b (the
 // far-field pressure reads the corrected cell p and psi), rho_b, rhoU_b, rhoE_b.
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -428,6 +429,24 @@ __global__ void k_conserved_aos(int n, Fields F, double* out) {
     out[5 * (size_t)i + 4] = F.rhoE[i];
 }
 
+// ---------------------------------------------------------------- host arrays
+struct Comps {
+    double* p[9];
+};
+// entries [e0, e0 + cnt) of the interleaved array (entry k i + d is comps[d][i])
+__global__ __launch_bounds__(256) void k_interleave(Comps c, int k, size_t e0, size_t cnt, double* out) {
+    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < cnt; e += (size_t)gridDim.x * blockDim.x) {
+        const size_t q = e0 + e, i = q / k;
+        out[e] = c.p[q - i * k][i];
+    }
+}
+__global__ __launch_bounds__(256) void k_deinterleave(Comps c, int k, size_t e0, size_t cnt, const double* in) {
+    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < cnt; e += (size_t)gridDim.x * blockDim.x) {
+        const size_t q = e0 + e, i = q / k;
+        c.p[q - i * k][i] = in[e];
+    }
+}
+
 // ---------------------------------------------------------------- CFL ramp
 // per-block partial sums of |R_c|^2 (mag then square, timeDST.C:328-331)
 __global__ __launch_bounds__(256) void k_rnorm_partial(int n, const double* R, double* partial) {
@@ -485,6 +504,40 @@ __global__ void k_store_old(int n, Fields F) {
 }
 
 }  // namespace
+
+double* stage_buf(Case& c, size_t want) {
+    want = std::min(want, kStageDoubles);
+    if (c.stage.n < want) c.stage.alloc(want);
+    return c.stage.p;
+}
+
+void download_aos(Case& c, const double* const* comps, int k, size_t n, double* out) {
+    Comps cp{};
+    for (int d = 0; d < k; ++d) cp.p[d] = const_cast<double*>(comps[d]);
+    double* st = stage_buf(c, k * n);
+    for (size_t e = 0; e < k * n; e += kStageDoubles) {
+        const size_t cnt = std::min(kStageDoubles, k * n - e);
+        hipLaunchKernelGGL(k_interleave, dim3(std::min<long>(8192, blocks_for((long)cnt, 256))), dim3(256), 0, c.stream, cp,
+                           k, e, cnt, st);
+        RDST_HIP(hipGetLastError());
+        RDST_HIP(hipMemcpyAsync(out + e, st, cnt * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+        RDST_HIP(hipStreamSynchronize(c.stream));
+    }
+}
+
+void upload_aos(Case& c, double* const* comps, int k, size_t n, const double* in) {
+    Comps cp{};
+    for (int d = 0; d < k; ++d) cp.p[d] = comps[d];
+    double* st = stage_buf(c, k * n);
+    for (size_t e = 0; e < k * n; e += kStageDoubles) {
+        const size_t cnt = std::min(kStageDoubles, k * n - e);
+        RDST_HIP(hipMemcpyAsync(st, in + e, cnt * sizeof(double), hipMemcpyHostToDevice, c.stream));
+        hipLaunchKernelGGL(k_deinterleave, dim3(std::min<long>(8192, blocks_for((long)cnt, 256))), dim3(256), 0, c.stream,
+                           cp, k, e, cnt, st);
+        RDST_HIP(hipGetLastError());
+        RDST_HIP(hipStreamSynchronize(c.stream));
+    }
+}
 
 void set_steady_state_deltaT(Case& c) {
     MeshDev md = c.meshDev();
