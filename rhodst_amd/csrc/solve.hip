@@ -29,13 +29,14 @@ namespace rdst {
 
 struct SolverWork {
     int n = 0, n5 = 0, nDirs = 0, G = 0;
+    long ld = 0;               // stride of the Krylov basis: n5, in FP32 padded to a multiple of four
     bool mixed = false;
     DBuf<double> LU, Dinv;     // FP64 factors
     DBuf<float> LU32, Dinv32;  // FP32 factors
     DBuf<double> b, r, wA, tmp, x0;
     DBuf<double> dW;           // the correction of the deltaW / mixed forms
     DBuf<double> V;            // (nDirs+1) x n5 FP64 basis
-    DBuf<float> V32, w32, r32, t32;
+    DBuf<float> V32, w32, r32;
     DBuf<double> scal;         // device scalars
     DBuf<double> partA, partB; // reduction partials
     DBuf<double> multi;        // classical Gram-Schmidt partials [nDirs+1][G]
@@ -111,7 +112,7 @@ __global__ __launch_bounds__(RED_BS) void k_xref_final(const double* part, int G
         if (threadIdx.x == 0) xref[k] = t / n;
     }
 }
-// normFactor partials: sum |wA - pA| + |b - pA| (5-vector magnitudes)
+// normFactor partials: sum |wA - pA| + |b - pA| (5-vector magnitudes; null: zero)
 __global__ __launch_bounds__(RED_BS) void k_norm_partial(int n, const double* wA, const double* pA, const double* b,
                                                           double* part) {
     __shared__ double sh[16];
@@ -119,7 +120,8 @@ __global__ __launch_bounds__(RED_BS) void k_norm_partial(int n, const double* wA
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         double a = 0, c = 0;
         for (int k = 0; k < 5; ++k) {
-            double d1 = wA[5 * i + k] - pA[5 * i + k], d2 = b[5 * i + k] - pA[5 * i + k];
+            const double wv = wA ? wA[5 * i + k] : 0.0, pv = pA ? pA[5 * i + k] : 0.0;
+            double d1 = wv - pv, d2 = b[5 * i + k] - pv;
             a += d1 * d1;
             c += d2 * d2;
         }
@@ -147,18 +149,11 @@ __global__ void k_sub(long n, double* r, const double* b, const double* a) {
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) r[i] = b[i] - a[i];
 }
 template <class T>
-__global__ void k_acc(long n, T* y, const T* a) {
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) y[i] += a[i];
+__global__ void k_acc(long n, double* y, const T* a) {
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) y[i] += (double)a[i];
 }
 __global__ void k_add(long n, double* y, const double* a) {
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) y[i] += a[i];
-}
-// y = x / s[0]
-template <class T>
-__global__ void k_scale_div(long n, T* y, const T* x, const double* s) {
-    const double d = s[0];
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-        y[i] = (T)((double)x[i] / d);
 }
 // fused MGS step: h = reduce(partIn); w -= h Vj; partial dot(w, Vnext) -> partOut; block 0 stores h
 template <class T>
@@ -176,13 +171,45 @@ __global__ __launch_bounds__(RED_BS) void k_mgs_step(long n, T* w, const T* Vj, 
     double t = block_sum(s, sh);
     if (threadIdx.x == 0) partOut[blockIdx.x] = t;
 }
-// x += sum_i yh[i] V_i
-template <class TV, class TX>
-__global__ void k_update_x(long n, TX* x, const TV* V, const double* yh, int m) {
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        double xi = (double)x[i];
-        for (int k = 0; k < m; ++k) xi += yh[k] * (double)V[(size_t)k * n + i];
-        x[i] = (TX)xi;
+// x += sum_i yh[i] V_i (V_i at V + i ld), and for EXPAND the sum alone, rounded
+// to the basis' type, added to x (the correction of the mixed form).  The sum of
+// an entry runs in order i = 0, 1, ...; five vectors' entries of two places per
+// thread are in flight (one load at a time reached 2.2 TB/s).
+template <class TV, class TX, bool EXPAND>
+__global__ __launch_bounds__(RED_BS) void k_update_x(long n, long ld, TX* x, const TV* V, const double* yh, int m) {
+    constexpr int HC = RED_BS;
+    __shared__ double yc[HC];
+    for (int t = threadIdx.x; t < m && t < HC; t += blockDim.x) yc[t] = yh[t];
+    __syncthreads();
+    const long st = (long)gridDim.x * blockDim.x;
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += 2 * st) {
+        const bool two = i + st < n;
+        const long i1 = two ? i + st : i;
+        double a0 = EXPAND ? 0.0 : (double)x[i], a1 = EXPAND ? 0.0 : (double)x[i1];
+        int k = 0;
+        for (; k + 5 <= m; k += 5) {
+            TV v0[5], v1[5];
+#pragma unroll
+            for (int q = 0; q < 5; ++q) { v0[q] = V[(size_t)(k + q) * ld + i]; v1[q] = V[(size_t)(k + q) * ld + i1]; }
+#pragma unroll
+            for (int q = 0; q < 5; ++q) {
+                const double h = k + q < HC ? yc[k + q] : yh[k + q];
+                a0 += h * (double)v0[q];
+                a1 += h * (double)v1[q];
+            }
+        }
+        for (; k < m; ++k) {
+            const double h = k < HC ? yc[k] : yh[k];
+            a0 += h * (double)V[(size_t)k * ld + i];
+            a1 += h * (double)V[(size_t)k * ld + i1];
+        }
+        if (EXPAND) {
+            x[i] += (TX)(TV)a0;
+            if (two) x[i1] += (TX)(TV)a1;
+        } else {
+            x[i] = (TX)a0;
+            if (two) x[i1] = (TX)a1;
+        }
     }
 }
 
@@ -192,40 +219,85 @@ __device__ inline void givens(double h, double beta, double& c, double& s) {
     else if (fabs(beta) > fabs(h)) { double tau = -h / beta; s = 1.0 / sqrt(1.0 + tau * tau); c = s * tau; }
     else { double tau = -beta / h; c = 1.0 / sqrt(1.0 + tau * tau); s = c * tau; }
 }
-// beta = sqrt(reduce(part)); rotate column i, new rotation, update bh
-__global__ __launch_bounds__(RED_BS) void k_gmres_column(double* sc, const double* part, int G, int i, int m) {
+// The step between two Krylov vectors, one launch: beta = sqrt(reduce(part)) in
+// every block, y = x / beta (entries n .. ld - 1 zero); block 0 also applies the
+// rotations to column i, forms the new one and updates bh (i = -1: the start of
+// a cycle, bh = (beta, 0, ..)).  The scalar work is one thread's, on a column
+// staged in LDS: read from memory step by step it took up to 11 us of a 30-vector
+// cycle's every iteration, in a launch of its own.
+constexpr int GMRES_COL = 256;  // longest column staged
+template <class T>
+__global__ __launch_bounds__(RED_BS) void k_gmres_next(long n, long ld, T* y, const T* x, double* sc, const double* part,
+                                                       int G, int i, int m) {
     __shared__ double sh[16];
-    const double beta = sqrt(reduce_partials(part, G, sh));
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    __shared__ double hc[GMRES_COL + 1], cc[GMRES_COL], ss[GMRES_COL];
     double* H = sc + S_H;
     double* cs = H + m * m;
     double* sn = cs + m;
     double* bh = sn + m;
-    for (int j = 0; j < i; ++j) {
-        const double Hji = H[j * m + i];
-        H[j * m + i] = cs[j] * Hji - sn[j] * H[(j + 1) * m + i];
-        H[(j + 1) * m + i] = sn[j] * Hji + cs[j] * H[(j + 1) * m + i];
+    const bool lds = i < GMRES_COL;
+    if (blockIdx.x == 0 && lds)
+        for (int j = threadIdx.x; j <= i; j += blockDim.x) {
+            hc[j] = H[j * m + i];
+            cc[j] = cs[j];
+            ss[j] = sn[j];
+        }
+    const double beta = sqrt(reduce_partials(part, G, sh));
+    if (y) {
+        for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < ld; e += (long)gridDim.x * blockDim.x)
+            y[e] = e < n ? (T)((double)x[e] / beta) : T(0);
     }
-    givens(H[i * m + i], beta, cs[i], sn[i]);
-    const double bhi = bh[i];
-    bh[i] = cs[i] * bhi - sn[i] * bh[i + 1];
-    bh[i + 1] = sn[i] * bhi + cs[i] * bh[i + 1];
-    H[i * m + i] = cs[i] * H[i * m + i] - sn[i] * beta;
+    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    if (i < 0) {
+        for (int k = 1; k <= m; ++k) bh[k] = 0.0;
+        bh[0] = beta;
+        return;
+    }
+    double h;
+    if (lds) {
+        h = hc[0];
+        for (int j = 0; j < i; ++j) {
+            const double Hji = h, hn = hc[j + 1];
+            H[j * m + i] = cc[j] * Hji - ss[j] * hn;
+            h = ss[j] * Hji + cc[j] * hn;
+        }
+    } else {
+        h = H[i];
+        for (int j = 0; j < i; ++j) {
+            const double Hji = h, hn = H[(j + 1) * m + i];
+            H[j * m + i] = cs[j] * Hji - sn[j] * hn;
+            h = sn[j] * Hji + cs[j] * hn;
+        }
+    }
+    double c, s;
+    givens(h, beta, c, s);
+    cs[i] = c;
+    sn[i] = s;
+    const double bhi = bh[i], bh1 = bh[i + 1];
+    bh[i] = c * bhi - s * bh1;
+    bh[i + 1] = s * bhi + c * bh1;
+    H[i * m + i] = c * h - s * beta;
 }
-__global__ void k_gmres_start(double* sc, int m) {
-    double* H = sc + S_H;
-    double* bh = H + m * m + 2 * m;
-    for (int k = 0; k <= m; ++k) bh[k] = 0.0;
-    bh[0] = sc[S_BETA];
-}
-__global__ void k_gmres_backsub(double* sc, int m) {
+// back-substitution, one thread on a triangle staged in LDS (m <= GMRES_TRI)
+constexpr int GMRES_TRI = 80;
+__global__ __launch_bounds__(256) void k_gmres_backsub(double* sc, int m) {
+    extern __shared__ double tri[];
     double* H = sc + S_H;
     double* bh = H + m * m + 2 * m;
     double* yh = bh + m + 1;
+    const double* A = H;
+    if (m <= GMRES_TRI) {
+        for (int e = threadIdx.x; e < m * m + m; e += blockDim.x) tri[e] = e < m * m ? H[e] : bh[e - m * m];
+        A = tri;
+        __syncthreads();
+    }
+    if (threadIdx.x != 0) return;
+    double* yl = m <= GMRES_TRI ? tri + m * m : yh;
     for (int i = m - 1; i >= 0; --i) {
-        double s = bh[i];
-        for (int j = i + 1; j < m; ++j) s -= H[i * m + j] * yh[j];
-        yh[i] = s / H[i * m + i];
+        double s = m <= GMRES_TRI ? yl[i] : bh[i];
+        for (int j = i + 1; j < m; ++j) s -= A[i * m + j] * yl[j];
+        yl[i] = s / A[i * m + i];
+        yh[i] = yl[i];
     }
 }
 
@@ -287,19 +359,21 @@ __global__ __launch_bounds__(64) void k_sell_spmv(int n, const int64_t* sellPtr,
 }
 
 // ---------------------------------------------------------------- classical Gram-Schmidt
-// partial dots of w with NACC consecutive basis vectors V_j0 .. V_j0+NACC-1
-// (cnt of them valid).  Each thread walks its grid-stride elements four at a
+// partial dots of w with the tot basis vectors (V_j at V + j ld), NACC consecutive
+// ones V_j0 .. per blockIdx.y: one launch for all of them, so a short basis or
+// vector still fills the chip.  Each thread walks its grid-stride elements four at a
 // time so that 4 (NACC+1) loads are in flight; the accumulation order per
 // thread is the plain grid-stride order, so the partials do not depend on it.
 template <class T, int NACC>
-__global__ __launch_bounds__(RED_BS) void k_multidot_partial(long n, const T* w, const T* V, int j0, int cnt,
+__global__ __launch_bounds__(RED_BS) void k_multidot_partial(long n, long ld, const T* w, const T* V, int tot,
                                                              double* part) {
     __shared__ double sh[16];
+    const int j0 = NACC * (int)blockIdx.y, cnt = min(NACC, tot - j0);
     double acc[NACC];
     for (int q = 0; q < NACC; ++q) acc[q] = 0.0;
     const long st = (long)gridDim.x * blockDim.x;
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const T* Vb = V + (size_t)j0 * n;
+    const T* Vb = V + (size_t)j0 * ld;
     for (; i + 3 * st < n; i += 4 * st) {
         double wi[4];
         T v[4][NACC];
@@ -309,7 +383,7 @@ __global__ __launch_bounds__(RED_BS) void k_multidot_partial(long n, const T* w,
         for (int q = 0; q < NACC; ++q)
             if (q < cnt)
 #pragma unroll
-                for (int u = 0; u < 4; ++u) v[u][q] = Vb[(size_t)q * n + i + u * st];
+                for (int u = 0; u < 4; ++u) v[u][q] = Vb[(size_t)q * ld + i + u * st];
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
@@ -320,7 +394,7 @@ __global__ __launch_bounds__(RED_BS) void k_multidot_partial(long n, const T* w,
         const double wi = (double)w[i];
 #pragma unroll
         for (int q = 0; q < NACC; ++q)
-            if (q < cnt) acc[q] += wi * (double)Vb[(size_t)q * n + i];
+            if (q < cnt) acc[q] += wi * (double)Vb[(size_t)q * ld + i];
     }
 #pragma unroll
     for (int q = 0; q < NACC; ++q) {
@@ -329,21 +403,22 @@ __global__ __launch_bounds__(RED_BS) void k_multidot_partial(long n, const T* w,
         if (threadIdx.x == 0) part[(size_t)(j0 + q) * gridDim.x + blockIdx.x] = t;
     }
 }
-// the same for an FP32 basis whose length is a multiple of four: each thread
+// the same for an FP32 basis (padded with zeros to a multiple of four): each thread
 // reads four consecutive entries per 16-byte load (twice the bytes in flight
 // of the scalar form); per thread the entries are summed in grid-stride order
 // of their float4 groups
 template <int NACC>
-__global__ __launch_bounds__(RED_BS) void k_multidot_partial4(long n, const float* w, const float* V, int j0, int cnt,
+__global__ __launch_bounds__(RED_BS) void k_multidot_partial4(long ld, const float* w, const float* V, int tot,
                                                               double* part) {
     __shared__ double sh[16];
+    const int j0 = NACC * (int)blockIdx.y, cnt = min(NACC, tot - j0);
     double acc[NACC];
     for (int q = 0; q < NACC; ++q) acc[q] = 0.0;
-    const long n4 = n / 4;
+    const long n4 = ld / 4;
     const long st = (long)gridDim.x * blockDim.x;
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const float4* w4 = reinterpret_cast<const float4*>(w);
-    const float4* Vb = reinterpret_cast<const float4*>(V + (size_t)j0 * n);
+    const float4* Vb = reinterpret_cast<const float4*>(V + (size_t)j0 * ld);
     for (; i + st < n4; i += 2 * st) {
         float4 wi[2], v[2][NACC];
 #pragma unroll
@@ -430,11 +505,11 @@ __global__ __launch_bounds__(RED_BS) void k_cgs_update(long n, T* w, const T* V,
     if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
-// the same for an FP32 basis whose length is a multiple of four: 16-byte
+// the same for an FP32 basis padded with zeros to ld, a multiple of four: 16-byte
 // loads, two float4 groups per thread and two basis vectors per pass; each
 // entry is updated in the same order (j ascending) as above, so w is
 // unchanged; the |w|^2 partials are summed per float4 group
-__global__ __launch_bounds__(RED_BS) void k_cgs_update4(long n, float* w, const float* V, const double* H, int m, int col,
+__global__ __launch_bounds__(RED_BS) void k_cgs_update4(long n, long ld, float* w, const float* V, const double* H, int m, int col,
                                                         int cnt, double* part) {
     constexpr int HC = RED_BS;
     __shared__ double sh[16];
@@ -442,7 +517,7 @@ __global__ __launch_bounds__(RED_BS) void k_cgs_update4(long n, float* w, const 
     for (int t = threadIdx.x; t < cnt && t < HC; t += blockDim.x) hc[t] = H[t * m + col];
     __syncthreads();
     double s = 0.0;
-    const long n4 = n / 4;
+    const long n4 = ld / 4;
     const long st = (long)gridDim.x * blockDim.x;
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     float4* w4 = reinterpret_cast<float4*>(w);
@@ -477,7 +552,11 @@ __global__ __launch_bounds__(RED_BS) void k_cgs_update4(long n, float* w, const 
             if (two) upd(a[1], h0, Vj[i + st]);
         }
         for (int u = 0; u < (two ? 2 : 1); ++u) {
-            const float4 o = make_float4((float)a[u][0], (float)a[u][1], (float)a[u][2], (float)a[u][3]);
+            float4 o = make_float4((float)a[u][0], (float)a[u][1], (float)a[u][2], (float)a[u][3]);
+            if (4 * (i + u * st) + 3 >= n) {  // the padding stays zero
+                const long e = 4 * (i + u * st);
+                o.y = e + 1 < n ? o.y : 0.f; o.z = e + 2 < n ? o.z : 0.f; o.w = 0.f;
+            }
             w4[i + u * st] = o;
             s += (double)o.x * (double)o.x + (double)o.y * (double)o.y + (double)o.z * (double)o.z +
                  (double)o.w * (double)o.w;
@@ -917,13 +996,15 @@ static void ensure_work(Case& c) {
     if (mixed) {
         w->LU32.alloc(nn);
         w->Dinv32.alloc(25 * (size_t)m.nC);
-        w->V32.alloc((size_t)(w->nDirs + 1) * n5);
-        w->w32.alloc(n5);
+        w->ld = (long)((n5 + 3) & ~(size_t)3);
+        w->V32.alloc((size_t)(w->nDirs + 1) * w->ld);
+        w->w32.alloc(w->ld);
+        w->w32.zero(c.stream);
         w->r32.alloc(n5);
-        w->t32.alloc(n5);
     } else {
         w->LU.alloc(nn);
         w->Dinv.alloc(25 * (size_t)m.nC);
+        w->ld = (long)n5;
         w->V.alloc((size_t)(w->nDirs + 1) * n5);
     }
     w->b.alloc(n5);
@@ -1197,10 +1278,12 @@ void read_scalars(Ctx& k, int from, int count, double* dst) {
 }
 
 // one left-preconditioned GMRES(m) restart cycle on A z = rhs from z
-// (z updated in place); TV/TM = basis/matrix type
+// (z updated in place; z FP64 with an FP32 basis: the correction, added to z);
+// TV/TM = basis/matrix type
 template <class TM, class TV>
-void gmres_cycle(Ctx& k, const TM* A, const TM* LU, const TM* Dinv, TV* z, const TV* rres, TV* wv, TV* rv, TV* V, TV* ytmp) {
-    const long n5 = k.w.n5;
+void gmres_cycle(Ctx& k, const TM* A, const TM* LU, const TM* Dinv, double* z, const TV* rres, TV* wv, TV* rv, TV* V, TV* ytmp) {
+    constexpr bool EXPAND = sizeof(TV) == 4;
+    const long n5 = k.w.n5, ld = k.w.ld;
     const int m = k.w.nDirs;
     const int G = k.G;
     double* sc = k.w.scal.p;
@@ -1209,11 +1292,12 @@ void gmres_cycle(Ctx& k, const TM* A, const TM* LU, const TM* Dinv, TV* z, const
     // wA = M^-1 rA (right: rA); beta = |wA|
     if (k.right) hipLaunchKernelGGL((k_copy<TV, TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, wv, rres);
     else precondition(k, LU, Dinv, rres, wv, ytmp);
-    dot(k, n5, wv, wv, sc + S_BETA, 1);
-    hipLaunchKernelGGL(k_gmres_start, dim3(1), dim3(1), 0, k.s, sc, m);
+    double* pin = k.w.partA.p;
+    double* pout = k.w.partB.p;
+    hipLaunchKernelGGL((k_dot_partial<TV, TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, wv, wv, pin);
+    hipLaunchKernelGGL((k_gmres_next<TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, ld, V, wv, sc, pin, G, -1, m);
     for (int i = 0; i < m; ++i) {
-        TV* Vi = V + (size_t)i * n5;
-        hipLaunchKernelGGL((k_scale_div<TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, Vi, wv, sc + S_BETA);
+        TV* Vi = V + (size_t)i * ld;
         if (k.right) {
             precondition(k, LU, Dinv, Vi, rv, ytmp);
             spmv(k, A, rv, wv);
@@ -1221,74 +1305,81 @@ void gmres_cycle(Ctx& k, const TM* A, const TM* LU, const TM* Dinv, TV* z, const
             spmv(k, A, Vi, rv);
             precondition(k, LU, Dinv, rv, wv, ytmp);
         }
-        double* pin = k.w.partA.p;
-        double* pout = k.w.partB.p;
         if (k.c.st.gram_schmidt == RDST_GS_CLASSICAL) {
             // all projections from one multi-dot, then one fused update (+ |w|^2 partials)
-            for (int j0 = 0; j0 <= i; j0 += 8) {
-                if constexpr (sizeof(TV) == 4) {
-                    if (n5 % 4 == 0) {
-                        hipLaunchKernelGGL((k_multidot_partial4<8>), dim3(G), dim3(RED_BS), 0, k.s, n5, (const float*)wv,
-                                           (const float*)V, j0, std::min(8, i + 1 - j0), k.w.multi.p);
-                        continue;
-                    }
-                }
-                hipLaunchKernelGGL((k_multidot_partial<TV, 8>), dim3(G), dim3(RED_BS), 0, k.s, n5, wv, V, j0,
-                                   std::min(8, i + 1 - j0), k.w.multi.p);
-            }
+            const dim3 grid(G, (i + 8) / 8);
+            if constexpr (sizeof(TV) == 4)
+                hipLaunchKernelGGL((k_multidot_partial4<8>), grid, dim3(RED_BS), 0, k.s, ld, wv, V, i + 1, k.w.multi.p);
+            else
+                hipLaunchKernelGGL((k_multidot_partial<TV, 8>), grid, dim3(RED_BS), 0, k.s, n5, ld, wv, V, i + 1,
+                                   k.w.multi.p);
             hipLaunchKernelGGL(k_multidot_final, dim3(i + 1), dim3(RED_BS), 0, k.s, k.w.multi.p, G, i + 1, H, m, i);
-            bool done = false;
-            if constexpr (sizeof(TV) == 4) {
-                if (n5 % 4 == 0) {
-                    hipLaunchKernelGGL(k_cgs_update4, dim3(G), dim3(RED_BS), 0, k.s, n5, (float*)wv, (const float*)V, H,
-                                       m, i, i + 1, pin);
-                    done = true;
-                }
-            }
-            if (!done)
+            if constexpr (sizeof(TV) == 4)
+                hipLaunchKernelGGL(k_cgs_update4, dim3(G), dim3(RED_BS), 0, k.s, n5, ld, wv, V, H, m, i, i + 1, pin);
+            else
                 hipLaunchKernelGGL((k_cgs_update<TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, wv, V, H, m, i, i + 1, pin);
         } else {
             // partial dot(w, V0), then the fused MGS steps
             hipLaunchKernelGGL((k_dot_partial<TV, TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, wv, V, pin);
             for (int j = 0; j <= i; ++j) {
-                const TV* Vj = V + (size_t)j * n5;
-                const TV* Vn = (j < i) ? V + (size_t)(j + 1) * n5 : wv;
+                const TV* Vj = V + (size_t)j * ld;
+                const TV* Vn = (j < i) ? V + (size_t)(j + 1) * ld : wv;
                 hipLaunchKernelGGL((k_mgs_step<TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, wv, Vj, Vn, pin, G, pout,
                                    H + j * m + i);
                 std::swap(pin, pout);
             }
         }
-        // pin holds partials of |w|^2; rotations, and beta = |w| for the next V
-        hipLaunchKernelGGL(k_gmres_column, dim3(1), dim3(RED_BS), 0, k.s, sc, pin, G, i, m);
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(RED_BS), 0, k.s, pin, G, sc + S_BETA, 1);
+        // pin holds partials of |w|^2: the next V, the rotations
+        hipLaunchKernelGGL((k_gmres_next<TV>), dim3(i + 1 < m ? G : 1), dim3(RED_BS), 0, k.s, n5, ld,
+                           i + 1 < m ? V + (size_t)(i + 1) * ld : (TV*)nullptr, (const TV*)wv, sc, pin, G, i, m);
     }
-    hipLaunchKernelGGL(k_gmres_backsub, dim3(1), dim3(1), 0, k.s, sc, m);
+    hipLaunchKernelGGL(k_gmres_backsub, dim3(1), dim3(256), m <= GMRES_TRI ? sizeof(double) * (m * m + m) : 0, k.s, sc, m);
     if (k.right) {
         // z += M^-1 (V y)
         RDST_HIP(hipMemsetAsync(wv, 0, sizeof(TV) * n5, k.s));
-        hipLaunchKernelGGL((k_update_x<TV, TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, wv, V, yh, m);
+        hipLaunchKernelGGL((k_update_x<TV, TV, false>), dim3(G), dim3(RED_BS), 0, k.s, n5, ld, wv, V, yh, m);
         precondition(k, LU, Dinv, wv, rv, ytmp);
         hipLaunchKernelGGL((k_acc<TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, z, rv);
     } else {
-        hipLaunchKernelGGL((k_update_x<TV, TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, z, V, yh, m);
+        hipLaunchKernelGGL((k_update_x<TV, double, EXPAND>), dim3(G), dim3(RED_BS), 0, k.s, n5, ld, z, V, yh, m);
     }
 }
 
-rdst_solver_perf gmres_fp64(Ctx& k, const double* A, double* x, const double* b) {
+// norm factor, b - A x and its normalised magnitude.  fromZero: x is zero, so
+// A x, xRef and A xRef are, and the three products are left out
+template <class TA>
+void initial_residual(Ctx& k, const TA* A, const double* x, const double* b, bool fromZero, rdst_solver_perf& perf) {
+    SolverWork& w = k.w;
+    const long n5 = w.n5;
+    double* sc = w.scal.p;
+    if (fromZero) {
+        const int g = std::max(1, std::min(RED_MAXG, blocks_for(k.m.nC, RED_BS)));
+        hipLaunchKernelGGL(k_norm_partial, dim3(g), dim3(RED_BS), 0, k.s, k.m.nC, (const double*)nullptr,
+                           (const double*)nullptr, b, w.partA.p);
+        hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(RED_BS), 0, k.s, w.partA.p, g, sc + S_NORM);
+        cmptmag(k, b, sc + S_INIT, sc + S_NORM);
+    } else {
+        norm_factor(k, A, x, b);
+        spmv(k, A, x, w.wA.p);
+        hipLaunchKernelGGL(k_sub, dim3(k.G), dim3(RED_BS), 0, k.s, n5, w.r.p, b, w.wA.p);
+        cmptmag(k, w.r.p, sc + S_INIT, sc + S_NORM);
+    }
+    read_scalars(k, S_INIT, 5, perf.initial_residual);
+    for (int q = 0; q < 5; ++q) perf.final_residual[q] = perf.initial_residual[q];
+}
+
+rdst_solver_perf gmres_fp64(Ctx& k, const double* A, double* x, const double* b, bool fromZero) {
     SolverWork& w = k.w;
     const long n5 = w.n5;
     rdst_solver_perf perf{};
-    norm_factor(k, A, x, b);
-    spmv(k, A, x, w.wA.p);
-    hipLaunchKernelGGL(k_sub, dim3(k.G), dim3(RED_BS), 0, k.s, n5, w.r.p, b, w.wA.p);
-    cmptmag(k, w.r.p, w.scal.p + S_INIT, w.scal.p + S_NORM);
-    read_scalars(k, S_INIT, 5, perf.initial_residual);
-    for (int q = 0; q < 5; ++q) perf.final_residual[q] = perf.initial_residual[q];
+    initial_residual(k, A, x, b, fromZero, perf);
     if (converged(k.c.st, perf)) return perf;
+    const double* r = fromZero ? b : w.r.p;
     do {
-        gmres_cycle<double, double>(k, A, w.LU.p, w.Dinv.p, x, w.r.p, w.wA.p, w.tmp.p, w.V.p, w.x0.p);
+        gmres_cycle<double, double>(k, A, w.LU.p, w.Dinv.p, x, r, w.wA.p, w.tmp.p, w.V.p, w.x0.p);
         spmv(k, A, x, w.wA.p);
         hipLaunchKernelGGL(k_sub, dim3(k.G), dim3(RED_BS), 0, k.s, n5, w.r.p, b, w.wA.p);
+        r = w.r.p;
         cmptmag(k, w.r.p, w.scal.p + S_FIN, w.scal.p + S_NORM);
         read_scalars(k, S_FIN, 5, perf.final_residual);
         perf.n_iterations++;
@@ -1298,30 +1389,21 @@ rdst_solver_perf gmres_fp64(Ctx& k, const double* A, double* x, const double* b)
 
 // mixed precision: FP64 outer defect correction r = b - Aout x (Aout FP32
 // promoted for the implicit step, FP64 for the adjoint), inner FP32 GMRES
-// cycle on A e = r with the FP32 matrix, FP32 ILU and FP32 basis
+// cycle on A e = r with the FP32 matrix, FP32 ILU and FP32 basis; x += e in FP64
 template <class TO>
-rdst_solver_perf gmres_mixed(Ctx& k, const TO* Aout, const float* A, double* x, const double* b) {
+rdst_solver_perf gmres_mixed(Ctx& k, const TO* Aout, const float* A, double* x, const double* b, bool fromZero) {
     SolverWork& w = k.w;
     const long n5 = w.n5;
     rdst_solver_perf perf{};
-    norm_factor(k, Aout, x, b);
-    spmv(k, Aout, x, w.wA.p);
-    hipLaunchKernelGGL(k_sub, dim3(k.G), dim3(RED_BS), 0, k.s, n5, w.r.p, b, w.wA.p);
-    cmptmag(k, w.r.p, w.scal.p + S_INIT, w.scal.p + S_NORM);
-    read_scalars(k, S_INIT, 5, perf.initial_residual);
-    for (int q = 0; q < 5; ++q) perf.final_residual[q] = perf.initial_residual[q];
+    initial_residual(k, Aout, x, b, fromZero, perf);
     if (converged(k.c.st, perf)) return perf;
+    const double* r = fromZero ? b : w.r.p;
     do {
-        hipLaunchKernelGGL((k_copy<float, double>), dim3(k.G), dim3(RED_BS), 0, k.s, n5, w.r32.p, w.r.p);
-        RDST_HIP(hipMemsetAsync(w.t32.p, 0, sizeof(float) * n5, k.s));
-        // correction e (t32) from zero
-        gmres_cycle<float, float>(k, A, w.LU32.p, w.Dinv32.p, w.t32.p, w.r32.p, w.w32.p, w.r32.p, w.V32.p,
-                                  (float*)w.tmp.p);
-        // x += e in FP64
-        hipLaunchKernelGGL((k_copy<double, float>), dim3(k.G), dim3(RED_BS), 0, k.s, n5, w.wA.p, w.t32.p);
-        hipLaunchKernelGGL(k_add, dim3(k.G), dim3(RED_BS), 0, k.s, n5, x, w.wA.p);
+        hipLaunchKernelGGL((k_copy<float, double>), dim3(k.G), dim3(RED_BS), 0, k.s, n5, w.r32.p, r);
+        gmres_cycle<float, float>(k, A, w.LU32.p, w.Dinv32.p, x, w.r32.p, w.w32.p, w.r32.p, w.V32.p, (float*)w.tmp.p);
         spmv(k, Aout, x, w.wA.p);
         hipLaunchKernelGGL(k_sub, dim3(k.G), dim3(RED_BS), 0, k.s, n5, w.r.p, b, w.wA.p);
+        r = w.r.p;
         cmptmag(k, w.r.p, w.scal.p + S_FIN, w.scal.p + S_NORM);
         read_scalars(k, S_FIN, 5, perf.final_residual);
         perf.n_iterations++;
@@ -1407,13 +1489,13 @@ void block_solve(Case& c, rdst_solver_perf* perfOut) {
         // sourceW = A.W + s; solve A.W = sourceW from W (fvBlockMatrixDST.C:112-123)
         spmv(k, (const double*)c.A64.p, (const double*)W, w.b.p);
         hipLaunchKernelGGL(k_add, dim3(k.G), dim3(RED_BS), 0, k.s, n5, w.b.p, c.src.p);
-        perf = (c.st.solver == RDST_SOLVER_GMRES) ? gmres_fp64(k, c.A64.p, W, w.b.p) : bicgstab_fp64(k, W, w.b.p);
+        perf = (c.st.solver == RDST_SOLVER_GMRES) ? gmres_fp64(k, c.A64.p, W, w.b.p, false) : bicgstab_fp64(k, W, w.b.p);
     } else {
         // A.dW = s from 0, W += dW (deltaW mode; the mixed form always solves for the correction)
         double* dW = w.dW.p;
         RDST_HIP(hipMemsetAsync(dW, 0, sizeof(double) * n5, k.s));
-        if (mixed) perf = gmres_mixed<float>(k, c.A32.p, c.A32.p, dW, c.src.p);
-        else perf = (c.st.solver == RDST_SOLVER_GMRES) ? gmres_fp64(k, c.A64.p, dW, c.src.p) : bicgstab_fp64(k, dW, c.src.p);
+        if (mixed) perf = gmres_mixed<float>(k, c.A32.p, c.A32.p, dW, c.src.p, true);
+        else perf = (c.st.solver == RDST_SOLVER_GMRES) ? gmres_fp64(k, c.A64.p, dW, c.src.p, true) : bicgstab_fp64(k, dW, c.src.p);
         hipLaunchKernelGGL(k_add, dim3(k.G), dim3(RED_BS), 0, k.s, n5, W, dW);
         RDST_HIP(hipStreamSynchronize(k.s));
     }
@@ -1490,19 +1572,19 @@ void ldu_solve(Case& c, const double* diag, const double* upper, const double* l
     rdst_solver_perf perf{};
     double* X = c.lduX.p;
     if (mode == RDST_LDU_PLAIN && !mixed) {
-        perf = (c.st.solver == RDST_SOLVER_GMRES) ? gmres_fp64(k, c.A64.p, X, c.lduB.p) : bicgstab_fp64(k, X, c.lduB.p);
+        perf = (c.st.solver == RDST_SOLVER_GMRES) ? gmres_fp64(k, c.A64.p, X, c.lduB.p, false) : bicgstab_fp64(k, X, c.lduB.p);
     } else if (mode == RDST_LDU_PLAIN) {
-        perf = gmres_mixed<double>(k, c.A64.p, c.A32.p, X, c.lduB.p);
+        perf = gmres_mixed<double>(k, c.A64.p, c.A32.p, X, c.lduB.p, false);
     } else if (mode == RDST_LDU_W && !mixed) {
         spmv(k, (const double*)c.A64.p, (const double*)X, w.b.p);
         hipLaunchKernelGGL(k_add, dim3(k.G), dim3(RED_BS), 0, k.s, (long)n5, w.b.p, c.lduB.p);
-        perf = (c.st.solver == RDST_SOLVER_GMRES) ? gmres_fp64(k, c.A64.p, X, w.b.p) : bicgstab_fp64(k, X, w.b.p);
+        perf = (c.st.solver == RDST_SOLVER_GMRES) ? gmres_fp64(k, c.A64.p, X, w.b.p, false) : bicgstab_fp64(k, X, w.b.p);
     } else {
         // deltaW, and the W form in mixed precision (A x' = A x + b is A (x' - x) = b)
         double* dW = w.dW.p;
         RDST_HIP(hipMemsetAsync(dW, 0, sizeof(double) * n5, k.s));
-        if (mixed) perf = gmres_mixed<double>(k, c.A64.p, c.A32.p, dW, c.lduB.p);
-        else perf = (c.st.solver == RDST_SOLVER_GMRES) ? gmres_fp64(k, c.A64.p, dW, c.lduB.p) : bicgstab_fp64(k, dW, c.lduB.p);
+        if (mixed) perf = gmres_mixed<double>(k, c.A64.p, c.A32.p, dW, c.lduB.p, true);
+        else perf = (c.st.solver == RDST_SOLVER_GMRES) ? gmres_fp64(k, c.A64.p, dW, c.lduB.p, true) : bicgstab_fp64(k, dW, c.lduB.p);
         hipLaunchKernelGGL(k_add, dim3(k.G), dim3(RED_BS), 0, k.s, (long)n5, X, dW);
     }
     RDST_HIP(hipGetLastError());
@@ -1575,22 +1657,22 @@ void adjoint_solve(Case& c, const double* g, double* lambda, const rdst_adjoint_
             ilu_factor<float>(k, c.adjJT32.p, k.w.LU32.p, k.w.Dinv32.p);
             const double* outer = c.adjWide ? c.adjWT.p : c.adjJT.p;
             if (as.inner_operator == 1) {
-                p = gmres_mixed<double>(k, outer, c.adjJT32.p, lambda, g);
+                p = gmres_mixed<double>(k, outer, c.adjJT32.p, lambda, g, false);
             } else if (c.adjWide) {
                 const size_t nw = c.adjWT.n;
                 if (c.adjWT32.n != nw) c.adjWT32.alloc(nw);
                 hipLaunchKernelGGL((k_cast<double, float>), dim3(std::min(4096, blocks_for((long)nw, 256))), dim3(256),
                                    0, c.stream, (long)nw, c.adjWT.p, c.adjWT32.p);
-                p = gmres_mixed<double>(k, outer, c.adjWT32.p, lambda, g);
+                p = gmres_mixed<double>(k, outer, c.adjWT32.p, lambda, g, false);
             } else {
                 if (PT != c.adjJT.p)
                     hipLaunchKernelGGL((k_cast<double, float>), dim3(gb), dim3(256), 0, c.stream, (long)nn, c.adjJT.p,
                                        c.adjJT32.p);
-                p = gmres_mixed<double>(k, outer, c.adjJT32.p, lambda, g);
+                p = gmres_mixed<double>(k, outer, c.adjJT32.p, lambda, g, false);
             }
         } else {
             ilu_factor<double>(k, PT, k.w.LU.p, k.w.Dinv.p);
-            p = gmres_fp64(k, c.adjWide ? c.adjWT.p : c.adjJT.p, lambda, g);
+            p = gmres_fp64(k, c.adjWide ? c.adjWT.p : c.adjJT.p, lambda, g, false);
         }
         RDST_HIP(hipStreamSynchronize(c.stream));
         if (perf) *perf = p;
