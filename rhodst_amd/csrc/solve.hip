@@ -223,6 +223,12 @@ __device__ inline void givens(double h, double beta, double& c, double& s) {
 // every block, y = x / beta (entries n .. ld - 1 zero); block 0 also applies the
 // rotations to column i, forms the new one and updates bh (i = -1: the start of
 // a cycle, bh = (beta, 0, ..)).  The scalar work is one thread's, on a column
+// (x, y) rotated, with the contraction written out: left to the compiler it
+// changes with the code around it, and so does the last bit of every iterate
+__device__ inline void rotate(double c, double s, double x, double y, double& xr, double& yr) {
+    xr = __builtin_fma(c, x, -(s * y));
+    yr = __builtin_fma(s, x, c * y);
+}
 // staged in LDS: read from memory step by step it took up to 11 us of a 30-vector
 // cycle's every iteration, in a launch of its own.
 constexpr int GMRES_COL = 256;  // longest column staged
@@ -258,25 +264,22 @@ __global__ __launch_bounds__(RED_BS) void k_gmres_next(long n, long ld, T* y, co
         h = hc[0];
         for (int j = 0; j < i; ++j) {
             const double Hji = h, hn = hc[j + 1];
-            H[j * m + i] = cc[j] * Hji - ss[j] * hn;
-            h = ss[j] * Hji + cc[j] * hn;
+            rotate(cc[j], ss[j], Hji, hn, H[j * m + i], h);
         }
     } else {
         h = H[i];
         for (int j = 0; j < i; ++j) {
             const double Hji = h, hn = H[(j + 1) * m + i];
-            H[j * m + i] = cs[j] * Hji - sn[j] * hn;
-            h = sn[j] * Hji + cs[j] * hn;
+            rotate(cs[j], sn[j], Hji, hn, H[j * m + i], h);
         }
     }
     double c, s;
     givens(h, beta, c, s);
     cs[i] = c;
     sn[i] = s;
-    const double bhi = bh[i], bh1 = bh[i + 1];
-    bh[i] = c * bhi - s * bh1;
-    bh[i + 1] = s * bhi + c * bh1;
-    H[i * m + i] = c * h - s * beta;
+    rotate(c, s, bh[i], bh[i + 1], bh[i], bh[i + 1]);
+    double below;
+    rotate(c, s, h, beta, H[i * m + i], below);
 }
 // back-substitution, one thread on a triangle staged in LDS (m <= GMRES_TRI)
 constexpr int GMRES_TRI = 80;
