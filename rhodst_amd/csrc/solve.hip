@@ -219,16 +219,16 @@ __device__ inline void givens(double h, double beta, double& c, double& s) {
     else if (fabs(beta) > fabs(h)) { double tau = -h / beta; s = 1.0 / sqrt(1.0 + tau * tau); c = s * tau; }
     else { double tau = -beta / h; c = 1.0 / sqrt(1.0 + tau * tau); s = c * tau; }
 }
-// The step between two Krylov vectors, one launch: beta = sqrt(reduce(part)) in
-// every block, y = x / beta (entries n .. ld - 1 zero); block 0 also applies the
-// rotations to column i, forms the new one and updates bh (i = -1: the start of
-// a cycle, bh = (beta, 0, ..)).  The scalar work is one thread's, on a column
 // (x, y) rotated, with the contraction written out: left to the compiler it
 // changes with the code around it, and so does the last bit of every iterate
 __device__ inline void rotate(double c, double s, double x, double y, double& xr, double& yr) {
     xr = __builtin_fma(c, x, -(s * y));
     yr = __builtin_fma(s, x, c * y);
 }
+// The step between two Krylov vectors, one launch: beta = sqrt(reduce(part)) in
+// every block, y = x / beta (entries n .. ld - 1 zero); block 0 also applies the
+// rotations to column i, forms the new one and updates bh (i = -1: the start of
+// a cycle, bh = (beta, 0, ..)).  The scalar work is one thread's, on a column
 // staged in LDS: read from memory step by step it took up to 11 us of a 30-vector
 // cycle's every iteration, in a launch of its own.
 constexpr int GMRES_COL = 256;  // longest column staged
