@@ -435,9 +435,10 @@ __global__ __launch_bounds__(64) void k_stream_entries(int ent, const int32_t* r
 // Scatter the factor into the stream, one wavefront per record and one thread
 // per (block, block row).  src[b]: block-CSR slot, or -(cell + 1) for the
 // row's Dinv; in a backward record (rowCell[b] >= 0) the slots' blocks are
-// stored as Dinv U, formed in FP64.
+// stored as Dinv U, formed in FP64.  uOnly: Dinv and the forward records are
+// in place already (k_ilu_chain), and LU is the matrix itself.
 template <class T>
-__global__ __launch_bounds__(256) void k_stream_pack(int nRec, int ent, const int32_t* recRows, const int32_t* recBlk,
+__global__ __launch_bounds__(256) void k_stream_pack(int nRec, int ent, int uOnly, const int32_t* recRows, const int32_t* recBlk,
                                                     const int32_t* src, const int32_t* rowCell, const uint32_t* start,
                                                     const T* LU, const T* Dinv, uint8_t* stream) {
     const int q = 4 * blockIdx.x + (threadIdx.x >> 6);
@@ -448,6 +449,7 @@ __global__ __launch_bounds__(256) void k_stream_pack(int nRec, int ent, const in
         const int b = e / 5, r = e - 5 * b, sl = src[b0 + b], cell = rowCell[b0 + b];
         T* dst = val + 5 * e;
         if (sl < 0 || cell < 0) {
+            if (uOnly) continue;
             const T* Bk = sl < 0 ? Dinv + 25 * (size_t)(-sl - 1) + 5 * r : LU + 25 * (size_t)sl + 5 * r;
             for (int c = 0; c < 5; ++c) dst[c] = Bk[c];
         } else {

@@ -90,6 +90,7 @@ static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp3
     ps.recRows.assign(1, 0);
     ps.recBlk.assign(1, 0);
     size_t pos = 0;
+    std::vector<uint32_t> lDst(m.nnzb, 0), dDst(m.nC, 0);  // of forward blocks and Dinv, 4-byte units
     auto size_of = [&](int nr, int nb) { return nr * ps.ent + ((nb * blk + 15) & ~15); };
     for (int p = 0; p < pv.nParts; ++p) {
         const int rs = pv.rowStart[p];
@@ -135,7 +136,9 @@ static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp3
                         uint16_t* e = ps.entries.data() + e0;
                         e[0] = (uint16_t)(5 * w.t);
                         e[1] = (uint16_t)(first | w.cnt << 8);
+                        const size_t at = (pos + (size_t)nr * ps.ent + (size_t)blk * first) / 4;
                         if (sweep) {
+                            dDst[w.i] = (uint32_t)at;
                             ps.src.push_back(-(w.i + 1));
                             ps.rowCell.push_back(w.i);
                         }
@@ -144,6 +147,7 @@ static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp3
                                   s1 = sweep ? m.rowPtr[w.i + 1] : m.slotDiag[w.i];
                         for (int s = s0; s < s1; ++s)
                             if (pv.localCol[s] >= 0) {
+                                if (!sweep) lDst[s] = (uint32_t)(at + (size_t)blk / 4 * (k - 2));
                                 ps.src.push_back(s);
                                 ps.rowCell.push_back(sweep ? w.i : -1);
                                 e[k++] = (uint16_t)(5 * pv.localCol[s]);
@@ -166,6 +170,51 @@ static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp3
     ps.start.push_back((uint32_t)(pos / 16));
     ps.nRec = (int)ps.hdr.size();
     ps.kmax = kmax;
+    // the factor as a chain: a bipartite mesh has no triangle, any other is looked through
+    int K = 1;
+    bool tri = pos / 4 > 0xffffffffull;
+    for (int i = 0; i < m.nC && !tri; ++i) {
+        int lo = 0;
+        for (int p = m.rowPtr[i]; p < m.slotDiag[i]; ++p) {
+            if (pv.localCol[p] < 0) continue;
+            ++lo;
+            if (m.nCellColours <= 2) continue;
+            const int k = m.cols[p];
+            for (int q = m.slotDiag[k] + 1; q < m.rowPtr[k + 1] && !tri; ++q)
+                if (pv.localCol[q] >= 0 && m.cols[q] != i)
+                    for (int s = m.rowPtr[i]; s < m.rowPtr[i + 1]; ++s)
+                        if (m.cols[s] == m.cols[q] && pv.localCol[s] >= 0) tri = true;
+        }
+        K = std::max(K, lo);
+    }
+    if (tri || K > 4) return;
+    ps.chainK = K <= 3 ? 3 : 4;
+    const int stride = 4 + 4 * ps.chainK;
+    ps.chain.assign((size_t)stride * pv.rows.size(), 0);
+    std::vector<int32_t> trans(m.nnzb, 0);
+    for (int f = 0; f < m.nI; ++f) {
+        trans[m.slotUpper[f]] = m.slotLower[f];
+        trans[m.slotLower[f]] = m.slotUpper[f];
+    }
+    for (size_t t = 0; t < pv.rows.size(); ++t) {
+        const int i = pv.rows[t];
+        int32_t* e = ps.chain.data() + stride * t;
+        e[0] = i;
+        e[2] = m.slotDiag[i];
+        e[3] = (int32_t)dDst[i];
+        for (int k = 0; k < ps.chainK; ++k) {  // unused places read the diagonal
+            e[4 + 4 * k] = e[5 + 4 * k] = m.slotDiag[i];
+            e[6 + 4 * k] = i;
+        }
+        for (int s = m.rowPtr[i]; s < m.slotDiag[i]; ++s) {
+            if (pv.localCol[s] < 0) continue;
+            int32_t* q = e + 4 + 4 * e[1]++;
+            q[0] = s;
+            q[1] = trans[s];
+            q[2] = m.cols[s];
+            q[3] = (int32_t)lDst[s];
+        }
+    }
 }
 
 void StreamSet::upload() {
@@ -179,6 +228,7 @@ void StreamSet::upload() {
     d_start.upload(start);
     d_src.upload(src);
     d_rowCell.upload(rowCell);
+    d_chain.upload(chain);
 }
 
 StreamSet& mesh_stream(Mesh& m, bool fp32) {
@@ -355,6 +405,7 @@ static void build_tiles(const Mesh& m, TileSet& ts) {
     order_partitions(m, tile, nT, ts);
     // columns outside the tile: halo cells, each once per tile and sweep
     ts.haloFStart.assign(1, 0);
+    ts.predStart.assign(1, 0);
     ts.haloBStart.assign(1, 0);
     std::vector<int32_t> seen(n, -1), slot(n, 0);
     for (int sweep = 0; sweep < 2; ++sweep) {
@@ -376,6 +427,13 @@ static void build_tiles(const Mesh& m, TileSet& ts) {
                     ts.localCol[s] = slot[j];
                 }
             }
+            if (!sweep) {
+                const size_t p0 = ts.pred.size();
+                for (int q = hs.back(); q < (int)h.size(); ++q) ts.pred.push_back(tile[h[q]]);
+                std::sort(ts.pred.begin() + p0, ts.pred.end());
+                ts.pred.erase(std::unique(ts.pred.begin() + p0, ts.pred.end()), ts.pred.end());
+                ts.predStart.push_back((int32_t)ts.pred.size());
+            }
             hs.push_back((int32_t)h.size());
             ts.maxSlots = std::max(ts.maxSlots, nr + hs[t + 1] - hs[t]);
         }
@@ -392,8 +450,13 @@ TileSet& mesh_tiles(Mesh& m, bool fp32) {
         ts.d_haloF.upload(ts.haloF);
         ts.d_haloBStart.upload(ts.haloBStart);
         ts.d_haloB.upload(ts.haloB);
-        // the tile's vector and its halo next to the ring in 160 KB of LDS, 16-bit columns
-        ts.ok = 40 * (size_t)ts.maxSlots + stream_ring(false) + 4096 <= 160 * 1024;
+        ts.d_predStart.upload(ts.predStart);
+        ts.d_pred.upload(ts.pred);
+        ts.d_levStart.upload(ts.levStart);
+        ts.d_levPtr.upload(ts.levPtr);
+        // the tile's vector and its halo, and where the vector's entries belong, next to the
+        // ring in 160 KB of LDS; 16-bit columns
+        ts.ok = 40 * (size_t)ts.maxSlots + 20 * kTileCells + stream_ring(false) + 4096 <= 160 * 1024;
         ts.tried = true;
     }
     StreamSet& ps = ts.ps[fp32];

@@ -104,7 +104,15 @@ struct StreamSet {
     std::vector<uint16_t> entries;          // [rows][ent / 2]
     std::vector<uint32_t> hdr, start;       // [nRec]; [nRec + 1] first 16-byte unit
     std::vector<int32_t> src, rowCell;      // [blocks] block-CSR slot, or -(cell + 1) for Dinv; the row's cell in a backward record, else -1
-    DBuf<int32_t> d_recBeg, d_recMid, d_recRows, d_recBlk, d_src, d_rowCell;
+    // The factor as a chain of diagonal blocks (no three coupled cells are
+    // coupled pairwise): per row, in the partitions' row order, cell, lower
+    // blocks, diagonal slot, where Dinv goes in the stream (4-byte units); per
+    // lower block its slot, the transposed coupling's slot, its cell, where L
+    // goes.  chainK: places per row, 0 when the factor has other updates.
+    int chainK = 0;
+    std::vector<int32_t> chain;
+    DBuf<int32_t> d_chain;
+    DBuf<int32_t> d_recBeg, d_recMid, d_recRows, d_recBlk, d_need, d_src, d_rowCell;
     DBuf<uint16_t> d_entries;
     DBuf<uint32_t> d_hdr, d_start;
     size_t bytes() const { return 16 * (size_t)start.back(); }
@@ -138,7 +146,8 @@ struct TileSet : PartSet {
     bool tried = false, ok = false;
     int maxSlots = 0;  // most rows + halo cells of a tile
     std::vector<int32_t> haloFStart, haloF, haloBStart, haloB;
-    DBuf<int32_t> d_haloFStart, d_haloF, d_haloBStart, d_haloB;
+    std::vector<int32_t> predStart, pred;  // the tiles whose factor a tile's needs
+    DBuf<int32_t> d_haloFStart, d_haloF, d_haloBStart, d_haloB, d_predStart, d_pred;
     StreamSet ps[2];   // FP64, FP32
 };
 constexpr int kTileCells = 512;  // most rows of a tile

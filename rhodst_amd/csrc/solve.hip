@@ -24,6 +24,7 @@
 #include "rdst_internal.hpp"
 #include "reduce.hpp"
 #include "ilu_stream.hpp"
+#include "ilu_factor.hpp"
 
 namespace rdst {
 
@@ -43,7 +44,10 @@ struct SolverWork {
     DBuf<uint8_t> st64, st32;  // the ILU(0) apply's record stream in FP64 / FP32
     DBuf<double> ty64;         // natural-order sweeps by tiles: the forward result, unset between applies
     DBuf<float> ty32;
-    DBuf<int> tickets;
+    DBuf<int> tickets;         // of the two sweeps
+    DBuf<int> factorState;     // zero-pivot flag and tile ticket of a factor
+    DBuf<int> tileDone;        // factor epoch of each tile
+    int epoch = 0;
     std::vector<double> hscal;
     // BiCGStab
     DBuf<double> p, ph, v, t, th, rw;
@@ -995,9 +999,8 @@ static void ensure_work(Case& c) {
     w->nDirs = std::max(1, c.st.n_directions);
     w->mixed = mixed;
     w->G = grid_for(w->n5);
-    const size_t n5 = w->n5, nn = (size_t)m.nnzb * 25;
+    const size_t n5 = w->n5;
     if (mixed) {
-        w->LU32.alloc(nn);
         w->Dinv32.alloc(25 * (size_t)m.nC);
         w->ld = (long)((n5 + 3) & ~(size_t)3);
         w->V32.alloc((size_t)(w->nDirs + 1) * w->ld);
@@ -1005,7 +1008,6 @@ static void ensure_work(Case& c) {
         w->w32.zero(c.stream);
         w->r32.alloc(n5);
     } else {
-        w->LU.alloc(nn);
         w->Dinv.alloc(25 * (size_t)m.nC);
         w->ld = (long)n5;
         w->V.alloc((size_t)(w->nDirs + 1) * n5);
@@ -1079,15 +1081,47 @@ static DBuf<uint8_t>& stream_buf(SolverWork& w, const double*) { return w.st64; 
 static DBuf<uint8_t>& stream_buf(SolverWork& w, const float*) { return w.st32; }
 
 template <class T>
-void stream_pack(Ctx& k, const StreamSet& ps, const T* LU, const T* Dinv) {
-    DBuf<uint8_t>& buf = stream_buf(k.w, LU);
+uint8_t* stream_alloc(Ctx& k, const StreamSet& ps) {
+    DBuf<uint8_t>& buf = stream_buf(k.w, (const T*)nullptr);
     if (buf.n != ps.bytes()) {
         buf.alloc(ps.bytes());
         hipLaunchKernelGGL(k_stream_entries, dim3(ps.nRec), dim3(64), 0, k.s, ps.ent, ps.d_recRows.p,
                            reinterpret_cast<const uint4*>(ps.d_entries.p), ps.d_start.p, buf.p);
     }
-    hipLaunchKernelGGL((k_stream_pack<T>), dim3(blocks_for(ps.nRec, 4)), dim3(256), 0, k.s, ps.nRec, ps.ent, ps.d_recRows.p, ps.d_recBlk.p,
-                       ps.d_src.p, ps.d_rowCell.p, ps.d_start.p, LU, Dinv, buf.p);
+    return buf.p;
+}
+template <class T>
+void stream_pack(Ctx& k, const StreamSet& ps, const T* LU, const T* Dinv, bool uOnly) {
+    uint8_t* st = stream_alloc<T>(k, ps);
+    hipLaunchKernelGGL((k_stream_pack<T>), dim3(blocks_for(ps.nRec, 4)), dim3(256), 0, k.s, ps.nRec, ps.ent, uOnly ? 1 : 0,
+                       ps.d_recRows.p, ps.d_recBlk.p, ps.d_src.p, ps.d_rowCell.p, ps.d_start.p, LU, Dinv, st);
+}
+
+// The factor straight into the record stream.  Taken wherever the couplings of
+// the partitions or tiles form no triangle and a row has at most four lower
+// neighbours (structured and box-like meshes; prisms and tetrahedra mostly):
+// the general kernels below, with a copy of A and a full pack, took 5.8 / 9.5 /
+// 0.52 ms (FP32 partitions of 2 M cells, FP64 natural order of 23.5 k and 252
+// cells), this takes 2.2 / 4.5 / 0.20 ms.
+template <class T, int K>
+void chain_launch(Ctx& k, const StreamSet& ps, const T* A, T* Dinv, bool natural, int* fail) {
+    Mesh& m = k.m;
+    const TileSet& ts = m.tiles;
+    uint8_t* st = stream_alloc<T>(k, ps);
+    if (natural && ts.nParts > 1) {
+        if (k.w.tileDone.n != (size_t)ts.nParts) {
+            k.w.tileDone.alloc(ts.nParts);
+            k.w.tileDone.zero(k.s);
+        }
+        hipLaunchKernelGGL((k_ilu_chain_tiles<T, K>), dim3(std::min(ts.nParts, 512)), dim3(CHAIN_THREADS), 0, k.s,
+                           ts.nParts, fail + 1, k.w.tileDone.p, ++k.w.epoch, ts.d_predStart.p, ts.d_pred.p,
+                           ts.d_levStart.p, ts.d_levPtr.p, ps.d_chain.p, A, Dinv, st, fail);
+    } else {
+        hipLaunchKernelGGL((k_ilu_chain<T, K>), dim3(natural ? 1 : m.nParts), dim3(CHAIN_THREADS), 0, k.s,
+                           natural ? ts.d_levStart.p : m.d_partLevStart.p, natural ? ts.d_levPtr.p : m.d_partLevPtr.p,
+                           ps.d_chain.p, A, Dinv, st, fail);
+    }
+    stream_pack<T>(k, ps, A, (const T*)Dinv, true);
 }
 
 // x = M^-1 r from the record stream: one workgroup per partition, or the
@@ -1129,18 +1163,35 @@ void stream_apply(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV* 
     else stream_launch<TM, TV, kStreamKD>(k, ps, stream, r, x, natural);
 }
 
+static DBuf<double>& factor_buf(SolverWork& w, const double*) { return w.LU; }
+static DBuf<float>& factor_buf(SolverWork& w, const float*) { return w.LU32; }
+
 template <class T>
-void ilu_factor(Ctx& k, const T* A, T* LU, T* Dinv) {
+void ilu_factor(Ctx& k, const T* A, T* Dinv) {
     Mesh& m = k.m;
-    RDST_HIP(hipMemcpyAsync(LU, A, sizeof(T) * 25 * (size_t)m.nnzb, hipMemcpyDeviceToDevice, k.s));
-    int* fail = (int*)(k.w.partB.p);  // scratch int
-    RDST_HIP(hipMemsetAsync(fail, 0, sizeof(int), k.s));
-    if (k.c.st.precond == RDST_PRECOND_ILU0 && k.c.st.ilu_order == RDST_ILU_PARTITIONED) {
+    constexpr bool F = sizeof(T) == 4;
+    if (!k.w.factorState.p) k.w.factorState.alloc(2);
+    int* fail = k.w.factorState.p;
+    RDST_HIP(hipMemsetAsync(fail, 0, 2 * sizeof(int), k.s));
+    const bool ilu = k.c.st.precond == RDST_PRECOND_ILU0, natural = k.c.st.ilu_order == RDST_ILU_NATURAL;
+    const StreamSet* ps = ilu ? (natural ? &mesh_tiles(m, F).ps[F] : &mesh_stream(m, F)) : nullptr;
+    const bool chain = ps && ps->kmax > 0 && ps->chainK > 0;
+    T* LU = nullptr;
+    if (ilu && !chain) {
+        // updates beyond the diagonal, or rows too long for the stream: a factor matrix
+        DBuf<T>& lu = factor_buf(k.w, (const T*)nullptr);
+        if (lu.n != 25 * (size_t)m.nnzb) lu.alloc(25 * (size_t)m.nnzb);
+        LU = lu.p;
+        RDST_HIP(hipMemcpyAsync(LU, A, sizeof(T) * 25 * (size_t)m.nnzb, hipMemcpyDeviceToDevice, k.s));
+    }
+    if (chain) {
+        if (ps->chainK == 3) chain_launch<T, 3>(k, *ps, A, Dinv, natural, fail);
+        else chain_launch<T, 4>(k, *ps, A, Dinv, natural, fail);
+    } else if (ilu && !natural) {
         hipLaunchKernelGGL((k_pilu_factor<T>), dim3(m.nParts), dim3(PILU_FACTOR_THREADS), 0, k.s, m.d_partLevStart.p, m.d_partLevPtr.p,
                            m.d_partRows.p, m.d_rowPtr.p, m.d_cols.p, m.d_slotDiag.p, m.d_localCol.p, LU, Dinv, fail);
-        const StreamSet& ps = mesh_stream(m, sizeof(T) == 4);
-        if (ps.kmax > 0) stream_pack<T>(k, ps, LU, Dinv);
-    } else if (k.c.st.precond == RDST_PRECOND_ILU0) {
+        if (ps->kmax > 0) stream_pack<T>(k, *ps, LU, Dinv, false);
+    } else if (ilu) {
         for (const LevelRun& g : m.runL) {
             if (g.fused) {
                 hipLaunchKernelGGL((k_ilu_factor_seg<T>), dim3(1), dim3(ILU_SEG_FACTOR_THREADS), 0, k.s, g.L0, g.L1,
@@ -1155,8 +1206,7 @@ void ilu_factor(Ctx& k, const T* A, T* LU, T* Dinv) {
                                    fail);
             }
         }
-        const StreamSet& ps = mesh_tiles(m, sizeof(T) == 4).ps[sizeof(T) == 4];
-        if (ps.kmax > 0) stream_pack<T>(k, ps, LU, Dinv);
+        if (ps->kmax > 0) stream_pack<T>(k, *ps, LU, Dinv, false);
     } else if (k.c.st.precond == RDST_PRECOND_DIAG) {
         hipLaunchKernelGGL((k_diag_inv<T>), dim3(blocks_for(m.nC, 256)), dim3(256), 0, k.s, m.nC, m.d_slotDiag.p, A, Dinv,
                            fail);
@@ -1480,10 +1530,10 @@ void block_solve(Case& c, rdst_solver_perf* perfOut) {
     // exact operator A (Newton-Krylov)
     const bool newton = c.st.jacobian == RDST_JACOBIAN_EXACT;
     if (mixed) {
-        ilu_factor<float>(k, newton ? c.P32.p : c.A32.p, w.LU32.p, w.Dinv32.p);
+        ilu_factor<float>(k, newton ? c.P32.p : c.A32.p, w.Dinv32.p);
         if (!c.sellFresh) build_sell<float>(k, c.A32.p, c.S32);
     } else {
-        ilu_factor<double>(k, newton ? c.P64.p : c.A64.p, w.LU.p, w.Dinv.p);
+        ilu_factor<double>(k, newton ? c.P64.p : c.A64.p, w.Dinv.p);
         if (!c.sellFresh) build_sell<double>(k, c.A64.p, c.S64);
     }
     rdst_solver_perf perf{};
@@ -1565,11 +1615,11 @@ void ldu_solve(Case& c, const double* diag, const double* upper, const double* l
         if (c.A32.n != nn) c.A32.alloc(nn);
         hipLaunchKernelGGL((k_cast<double, float>), dim3(std::min(4096, blocks_for((long)nn, 256))), dim3(256), 0, c.stream,
                            (long)nn, c.A64.p, c.A32.p);
-        ilu_factor<float>(k, c.A32.p, w.LU32.p, w.Dinv32.p);
+        ilu_factor<float>(k, c.A32.p, w.Dinv32.p);
         build_sell<float>(k, c.A32.p, c.S32);
         c.S64.release();  // the FP64 outer products read the block-CSR A64, never a stale sliced copy
     } else {
-        ilu_factor<double>(k, c.A64.p, w.LU.p, w.Dinv.p);
+        ilu_factor<double>(k, c.A64.p, w.Dinv.p);
         build_sell<double>(k, c.A64.p, c.S64);
     }
     rdst_solver_perf perf{};
@@ -1657,7 +1707,7 @@ void adjoint_solve(Case& c, const double* g, double* lambda, const rdst_adjoint_
             if (c.adjJT32.n != nn) c.adjJT32.alloc(nn);
             const int gb = std::min(4096, blocks_for((long)nn, 256));
             hipLaunchKernelGGL((k_cast<double, float>), dim3(gb), dim3(256), 0, c.stream, (long)nn, PT, c.adjJT32.p);
-            ilu_factor<float>(k, c.adjJT32.p, k.w.LU32.p, k.w.Dinv32.p);
+            ilu_factor<float>(k, c.adjJT32.p, k.w.Dinv32.p);
             const double* outer = c.adjWide ? c.adjWT.p : c.adjJT.p;
             if (as.inner_operator == 1) {
                 p = gmres_mixed<double>(k, outer, c.adjJT32.p, lambda, g, false);
@@ -1674,7 +1724,7 @@ void adjoint_solve(Case& c, const double* g, double* lambda, const rdst_adjoint_
                 p = gmres_mixed<double>(k, outer, c.adjJT32.p, lambda, g, false);
             }
         } else {
-            ilu_factor<double>(k, PT, k.w.LU.p, k.w.Dinv.p);
+            ilu_factor<double>(k, PT, k.w.Dinv.p);
             p = gmres_fp64(k, c.adjWide ? c.adjWT.p : c.adjJT.p, lambda, g, false);
         }
         RDST_HIP(hipStreamSynchronize(c.stream));

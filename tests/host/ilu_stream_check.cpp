@@ -95,6 +95,46 @@ static int check(const rdst_mesh_desc* desc, bool fp32, bool natural) {
                 if ((b + 63) / 64 > a / 64 + ring / 64) return fail("three records do not fit the ring", q);
             }
         }
+    // the factor chain: each row's blocks, their transposed couplings and their places in the stream
+    if (ps.chainK) {
+        std::vector<uint32_t> place(m.nnzb, 0), placeD(n, 0);
+        for (int q = 0; q < ps.nRec; ++q) {
+            const size_t v = 16 * (size_t)ps.start[q] + (size_t)ps.ent * (ps.recRows[q + 1] - ps.recRows[q]);
+            for (int b = ps.recBlk[q]; b < ps.recBlk[q + 1]; ++b) {
+                const uint32_t at = (uint32_t)((v + (size_t)(25 * (fp32 ? 4 : 8)) * (b - ps.recBlk[q])) / 4);
+                if (ps.src[b] < 0) placeD[-ps.src[b] - 1] = at;
+                else if (ps.rowCell[b] < 0) place[ps.src[b]] = at;
+            }
+        }
+        const int stride = 4 + 4 * ps.chainK;
+        std::vector<int> rowOf(m.nnzb);
+        for (int i = 0; i < n; ++i)
+            for (int s = m.rowPtr[i]; s < m.rowPtr[i + 1]; ++s) rowOf[s] = i;
+        for (size_t t = 0; t < rows.size(); ++t) {
+            const int32_t* e = ps.chain.data() + stride * t;
+            const int i = rows[t];
+            int cnt = 0;
+            if (e[0] != i || e[2] != m.slotDiag[i] || (uint32_t)e[3] != placeD[i]) return fail("chain row", i);
+            for (int s = m.rowPtr[i]; s < m.slotDiag[i]; ++s) {
+                if (part[m.cols[s]] != part[i]) continue;
+                const int32_t* q = e + 4 + 4 * cnt++;
+                if (q[0] != s || rowOf[q[1]] != m.cols[s] || m.cols[q[1]] != i || q[2] != m.cols[s] ||
+                    (uint32_t)q[3] != place[s])
+                    return fail("chain block", i, cnt);
+            }
+            if (cnt != e[1] || cnt > ps.chainK) return fail("chain count", i, cnt);
+        }
+    }
+    // a chain must be all of the factor: no lower neighbour shares another neighbour with the row
+    for (int i = 0; i < n && ps.chainK; ++i)
+        for (int p = m.rowPtr[i]; p < m.slotDiag[i]; ++p) {
+            const int k = m.cols[p];
+            if (part[k] != part[i]) continue;
+            for (int q = m.slotDiag[k] + 1; q < m.rowPtr[k + 1]; ++q)
+                for (int s = m.rowPtr[i]; s < m.rowPtr[i + 1]; ++s)
+                    if (m.cols[q] != i && m.cols[s] == m.cols[q] && part[m.cols[s]] == part[i])
+                        return fail("an update beyond the diagonal", i, k);
+        }
     // the plain sweeps
     std::vector<double> r(n), y(n), x(n), yr(n), xr(n);
     for (int i = 0; i < n; ++i) r[i] = std::sin(1.0 + 0.37 * i);
