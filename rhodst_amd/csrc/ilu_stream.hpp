@@ -105,6 +105,32 @@ __device__ __forceinline__ double dot5(const double* v, const double* y) {
     return __builtin_fma(v[4], y[4], __builtin_fma(v[3], y[3], __builtin_fma(v[2], y[2], __builtin_fma(v[0], y[0], v[1] * y[1]))));
 }
 
+// "not there yet" in a vector whose entries other workgroups wait for: a NaN of
+// its own; a result with that bit pattern is stored as another NaN
+template <class T>
+struct Unset;
+template <>
+struct Unset<double> {
+    using U = unsigned long long;
+    static constexpr U bits = 0x7ffc5ad3e1b0972full;
+};
+template <>
+struct Unset<float> {
+    using U = unsigned int;
+    static constexpr U bits = 0x7fe5ad3eu;
+};
+template <class T>
+__device__ __forceinline__ typename Unset<T>::U load_dev(const T* p) {
+    return __hip_atomic_load(reinterpret_cast<const typename Unset<T>::U*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ __forceinline__ void store_dev(T* p, T v) {
+    using U = typename Unset<T>::U;
+    U u = __builtin_bit_cast(U, v);
+    if (u == Unset<T>::bits) u ^= 1;  // a NaN either way
+    __hip_atomic_store(reinterpret_cast<U*>(p), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Records [0, n) of the list starting at r0; the first nF are forward ones
 // (y -= L y), the others backward ones (y = Dinv y - sum (Dinv U) y).  y holds
 // the partition's rows (and, behind them, the values of rows outside it).
@@ -112,9 +138,11 @@ __device__ __forceinline__ double dot5(const double* v, const double* y) {
 // the compute wavefronts, while the loader runs stream_load.  Per record: the
 // row entries are read two records ahead and the values one ahead, so between
 // two barriers only y's gather, the products and y's store depend on the
-// barrier before.
-template <class TM, class TV, int KDU, int RING>
-__device__ __forceinline__ void stream_compute(const uint32_t* hdr, int r0, int nF, int n, const uint8_t* ring, TV* y) {
+// barrier before.  PUB: each result also goes to out[to[its place in y]] at
+// once, for the workgroups that wait for it.
+template <class TM, class TV, int KDU, int RING, bool PUB>
+__device__ __forceinline__ void stream_compute(const uint32_t* hdr, int r0, int nF, int n, const uint8_t* ring, TV* y,
+                                               const int* to, TV* out) {
     constexpr int MASK = RING - 1, ENT = stream_entry(KDU), BLK = 25 * (int)sizeof(TM);
     struct Ent {
         uint32_t w[ENT / 4];
@@ -147,6 +175,8 @@ __device__ __forceinline__ void stream_compute(const uint32_t* hdr, int r0, int 
         if ((s & 63) == 63) {
             ha = hb;
             hb = s + 65 + lane < n ? hp[s + 65 + lane] : 0u;
+            // waited for here (vmcnt 0), not by the next records behind their stores
+            if constexpr (PUB) __builtin_amdgcn_s_waitcnt(0x0f70);
         }
     };
     auto entry = [&](Ent& E) {
@@ -174,10 +204,12 @@ __device__ __forceinline__ void stream_compute(const uint32_t* hdr, int r0, int 
     };
     struct Gat {
         TV a, d[5], v[KDU][5];
+        int to;
     };
     auto gather = [&](const Ent& E, Gat& G) {
         const TV* yr = y + (E.w[0] & 0xffff);
         G.a = yr[r];
+        if constexpr (PUB) G.to = to[(E.w[0] & 0xffff) + r];
 #pragma unroll
         for (int c = 0; c < 5; ++c) G.d[c] = yr[c];
 #pragma unroll
@@ -197,7 +229,10 @@ __device__ __forceinline__ void stream_compute(const uint32_t* hdr, int r0, int 
             const TV dot = dot5(V.v[k], G.v[k]);
             acc = k < cnt ? acc - dot : acc;
         }
-        if (E.row) y[(E.w[0] & 0xffff) + r] = acc;
+        if (E.row) {
+            y[(E.w[0] & 0xffff) + r] = acc;
+            if constexpr (PUB) store_dev(out + G.to, acc);
+        }
     };
     Ent e0, e1, e2;
     Val A, B;
@@ -300,7 +335,7 @@ __global__ __launch_bounds__(STREAM_THREADS) void k_stream_apply(const int32_t* 
     }
     const int rs = rowStart[pt], nl5 = (rowStart[pt + 1] - rs) * 5;
     gather_rows(rows + rs, nl5, r, y);
-    stream_compute<TM, TV, KDU, RING>(hdr, r0, rm - r0, r1 - r0, ring, y);
+    stream_compute<TM, TV, KDU, RING, false>(hdr, r0, rm - r0, r1 - r0, ring, y, nullptr, (TV*)nullptr);
     scatter_rows(rows + rs, nl5, y, x);
 }
 
@@ -309,35 +344,16 @@ __global__ __launch_bounds__(STREAM_THREADS) void k_stream_apply(const int32_t* 
 // tiles in an order that respects their dependencies (a ticket counter), so a
 // tile only waits for tiles that running workgroups already hold, and the
 // launch ends whatever number of workgroups is resident.  A value another tile
-// needs is its own flag: the vector is filled with kUnset before the sweep, a
-// reader polls until the value has arrived (device-scope loads and stores), a
-// result with that bit pattern is stored as another NaN.
-// Against one launch per level (8-10 us each, or 3.3 us per level in a
-// single-workgroup run of small levels) a level costs 0.35 us inside a tile and
-// a tile about 4 us of waiting.  Measured per apply (both sweeps): see stream_launch.
-template <class T>
-struct Unset;
-template <>
-struct Unset<double> {
-    using U = unsigned long long;
-    static constexpr U bits = 0x7ffc5ad3e1b0972full;
-};
-template <>
-struct Unset<float> {
-    using U = unsigned int;
-    static constexpr U bits = 0x7fe5ad3eu;
-};
-template <class T>
-__device__ __forceinline__ typename Unset<T>::U load_dev(const T* p) {
-    return __hip_atomic_load(reinterpret_cast<const typename Unset<T>::U*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <class T>
-__device__ __forceinline__ void store_dev(T* p, T v) {
-    using U = typename Unset<T>::U;
-    U u = __builtin_bit_cast(U, v);
-    if (u == Unset<T>::bits) u ^= 1;  // a NaN either way
-    __hip_atomic_store(reinterpret_cast<U*>(p), u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
+// needs is its own flag: the vector is filled with Unset before the sweep, a
+// row's result is stored the moment it is computed, and a wavefront of its own
+// polls for the halo values (device-scope loads and stores) in the order in
+// which the records read them.  A tile so runs a few levels behind the ones it
+// depends on, and a sweep costs about the levels of the whole mesh, not tiles
+// in a row times levels of a tile: with every halo value awaited at a tile's
+// start the sweeps took 365 us (RAE2822, 23.5 k cells, 27 tiles in a row) and 765
+// (wing, 321 k, 32 in a row), now 212 and 460.  By one launch per level (8-10 us
+// each, or 3.3 us per level in a single-workgroup run of small levels) it was
+// 1.5 ms and 2.3 ms.
 template <class T>
 __global__ __launch_bounds__(256) void k_fill_unset(long n, T* y, int* tickets) {
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
@@ -345,34 +361,79 @@ __global__ __launch_bounds__(256) void k_fill_unset(long n, T* y, int* tickets) 
     if (blockIdx.x == 0 && threadIdx.x < 2) tickets[threadIdx.x] = 0;
 }
 
-// Values of the halo cells into LDS, each awaited.
+// The halo wavefront: the values of the cells outside the tile into LDS, each
+// as soon as it has arrived, in step with the records (barriers as in
+// stream_load): before record s starts, the first need[s] are there.  A window
+// of 256 values is asked for at a time; what has not arrived is asked for again.
 template <class TV>
-__device__ __forceinline__ void await_rows(const int32_t* cells, int n5, const TV* x, TV* y) {
-    constexpr int U = 4, ST = 64 * STREAM_WAVES;
-    for (int b = 0; b < n5; b += U * ST) {
-        int i[U];
-        typename Unset<TV>::U v[U];
+__device__ __forceinline__ void stream_halo(const int32_t* cells, int nh5, const int32_t* need_, int n, const TV* x, TV* y) {
+    constexpr int U = 4, W = 64 * U;
+    const __attribute__((address_space(4))) int32_t* need = (const __attribute__((address_space(4))) int32_t*)need_;
+    const int lane = threadIdx.x & 63;
+    int b = 0, have = 0, i[U];
+    typename Unset<TV>::U v[U];
+    auto ask = [&]() {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int t = min(b + u * ST + (int)threadIdx.x, n5 - 1);
+            const int t = min(b + 64 * u + lane, nh5 - 1);
             i[u] = 5 * cells[t / 5] + t % 5;
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) v[u] = load_dev(x + i[u]);
-        for (;;) {
-            bool wait = false;
+    };
+    auto until = [&](int k) {
+        while (have < k) {
+            int first = min(b + W, nh5);
 #pragma unroll
-            for (int u = 0; u < U; ++u) wait |= v[u] == Unset<TV>::bits;
-            if (!__any(wait)) break;
-            __builtin_amdgcn_s_sleep(1);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (v[u] == Unset<TV>::bits) v[u] = load_dev(x + i[u]);
+            for (int u = U - 1; u >= 0; --u) {
+                const int t = b + 64 * u + lane;
+                const bool ok = v[u] != Unset<TV>::bits;
+                if (ok && t < nh5) y[t] = __builtin_bit_cast(TV, v[u]);
+                const unsigned long long miss = __ballot(!ok && t < nh5);
+                if (miss) first = b + 64 * u + (int)__builtin_ctzll(miss);
+                if (!ok) v[u] = load_dev(x + i[u]);
+            }
+            have = first;
+            if (first == b + W && first < nh5) {
+                b += W;
+                ask();
+            }
         }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the values in LDS
+    };
+    if (nh5 > 0) ask();
+    barrier_raw();
+    until(need[0]);
+    barrier_raw();
+    for (int s = 0; s < n; ++s) {
+        until(need[min(s + 1, n - 1)]);
+        barrier_raw();
+    }
+}
+
+// The tile's part of `in` into LDS, where each entry belongs in the vectors, and
+// `reset` made unset (it may be `in`: each thread resets what it has read).
+template <class TV>
+__device__ __forceinline__ void gather_tile(const int32_t* rows, int nl5, const TV* in, TV* y, int* to, TV* reset) {
+    constexpr int U = 10, ST = 64 * STREAM_WAVES;
+    for (int b = 0; b < nl5; b += U * ST) {
+        int i[U];
+        TV v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int t = min(b + u * ST + (int)threadIdx.x, nl5 - 1);
+            i[u] = 5 * rows[t / 5] + t % 5;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = in[i[u]];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int t = b + u * ST + (int)threadIdx.x;
-            if (t < n5) y[t] = __builtin_bit_cast(TV, v[u]);
+            if (t < nl5) {
+                y[t] = v[u];
+                to[t] = i[u];
+                reinterpret_cast<typename Unset<TV>::U*>(reset)[i[u]] = Unset<TV>::bits;
+            }
         }
     }
 }
@@ -380,23 +441,26 @@ __device__ __forceinline__ void await_rows(const int32_t* cells, int n5, const T
 // One sweep.  Forward: out = y from in = r, reset = x for the backward sweep.
 // Backward: out = x from in = y, reset = y for the next forward sweep.  Each
 // resets the other's ticket counter (the launches are ordered).
+constexpr int TILE_THREADS = STREAM_THREADS + 64;  // + the halo wavefront
 template <class TM, class TV, int KDU, bool BWD>
-__global__ __launch_bounds__(STREAM_THREADS) void k_tile_sweep(int nT, int* tickets, const int32_t* __restrict__ rowStart,
-                                                               const int32_t* __restrict__ rows,
-                                                               const int32_t* __restrict__ haloStart,
-                                                               const int32_t* __restrict__ halo,
-                                                               const int32_t* __restrict__ recBeg,
-                                                               const int32_t* __restrict__ recMid,
-                                                               const uint32_t* __restrict__ hdr,
-                                                               const uint32_t* __restrict__ start,
-                                                               const uint8_t* __restrict__ stream, const TV* in, TV* out,
-                                                               TV* reset) {
-    constexpr int RING = stream_ring(sizeof(TM) == 4), ST = 64 * STREAM_WAVES;
+__global__ __launch_bounds__(TILE_THREADS) void k_tile_sweep(int nT, int* tickets, const int32_t* __restrict__ rowStart,
+                                                             const int32_t* __restrict__ rows,
+                                                             const int32_t* __restrict__ haloStart,
+                                                             const int32_t* __restrict__ halo,
+                                                             const int32_t* __restrict__ recBeg,
+                                                             const int32_t* __restrict__ recMid,
+                                                             const int32_t* __restrict__ need,
+                                                             const uint32_t* __restrict__ hdr,
+                                                             const uint32_t* __restrict__ start,
+                                                             const uint8_t* __restrict__ stream, const TV* in, TV* out,
+                                                             TV* reset) {
+    constexpr int RING = stream_ring(sizeof(TM) == 4);
     extern __shared__ __align__(1024) unsigned char smem_raw[];
     __shared__ int next[2];
     uint8_t* ring = smem_raw;
-    TV* y = reinterpret_cast<TV*>(smem_raw + RING);
-    const bool loader = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == STREAM_WAVES;
+    int* to = reinterpret_cast<int*>(smem_raw + RING);
+    TV* y = reinterpret_cast<TV*>(smem_raw + RING + 20 * kTileCells);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (threadIdx.x == 0) next[0] = atomicAdd(tickets + BWD, 1);
     __syncthreads();
     for (int round = 0;; ++round) {
@@ -404,22 +468,17 @@ __global__ __launch_bounds__(STREAM_THREADS) void k_tile_sweep(int nT, int* tick
         if (ticket >= nT) break;
         const int tl = BWD ? nT - 1 - ticket : ticket;
         const int r0 = BWD ? recMid[tl] : recBeg[tl], r1 = BWD ? recBeg[tl + 1] : recMid[tl];
-        if (loader) {
-            if (r1 > r0) stream_load<RING>(stream, start, r0, r1, ring);
+        const int rs = rowStart[tl], nl5 = (rowStart[tl + 1] - rs) * 5;
+        if (wave == STREAM_WAVES) {
+            stream_load<RING>(stream, start, r0, r1, ring);
             if ((threadIdx.x & 63) == 0) next[(round + 1) & 1] = atomicAdd(tickets + BWD, 1);
+        } else if (wave > STREAM_WAVES) {
+            const int h0 = haloStart[tl];
+            stream_halo(halo + h0, (haloStart[tl + 1] - h0) * 5, need + r0, r1 - r0, (const TV*)out, y + nl5);
         } else {
             if (ticket == 0 && threadIdx.x == 0) tickets[!BWD] = 0;
-            const int rs = rowStart[tl], nl5 = (rowStart[tl + 1] - rs) * 5;
-            const int h0 = haloStart[tl], nh5 = (haloStart[tl + 1] - h0) * 5;
-            gather_rows(rows + rs, nl5, in, y);
-            await_rows(halo + h0, nh5, (const TV*)out, y + nl5);
-            if (r1 > r0) stream_compute<TM, TV, KDU, RING>(hdr, r0, BWD ? 0 : r1 - r0, r1 - r0, ring, y);
-            // (no record: every thread stores the entries that it gathered itself)
-            for (int t = threadIdx.x; t < nl5; t += ST) {
-                const size_t i = 5 * (size_t)rows[rs + t / 5] + t % 5;
-                store_dev(out + i, y[t]);
-                reinterpret_cast<typename Unset<TV>::U*>(reset)[i] = Unset<TV>::bits;
-            }
+            gather_tile(rows + rs, nl5, in, y, to, reset);
+            stream_compute<TM, TV, KDU, RING, true>(hdr, r0, BWD ? 0 : r1 - r0, r1 - r0, ring, y, to, out);
         }
         __syncthreads();
     }

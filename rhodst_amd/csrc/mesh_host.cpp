@@ -93,7 +93,7 @@ static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp3
     std::vector<uint32_t> lDst(m.nnzb, 0), dDst(m.nC, 0);  // of forward blocks and Dinv, 4-byte units
     auto size_of = [&](int nr, int nb) { return nr * ps.ent + ((nb * blk + 15) & ~15); };
     for (int p = 0; p < pv.nParts; ++p) {
-        const int rs = pv.rowStart[p];
+        const int rs = pv.rowStart[p], nOwn = pv.rowStart[p + 1] - rs;
         const int l0 = pv.levStart[p], nl = pv.levStart[p + 1] - l0 - 1;
         size_t base = pos;
         for (int sweep = 0; sweep < 2; ++sweep) {
@@ -101,6 +101,7 @@ static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp3
                 ps.recMid.push_back((int32_t)ps.hdr.size());
                 if (split) base = pos = (pos + 1023) & ~(size_t)1023;
             }
+            int need = 0;  // halo cells read so far
             for (int li = 0; li < nl; ++li) {
                 const int L = sweep ? nl - 1 - li : li;
                 rows.clear();
@@ -109,7 +110,7 @@ static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp3
                     const int s0 = sweep ? m.slotDiag[i] + 1 : m.rowPtr[i], s1 = sweep ? m.rowPtr[i + 1] : m.slotDiag[i];
                     int cnt = 0;
                     for (int s = s0; s < s1; ++s) cnt += pv.localCol[s] >= 0;
-                    if (sweep || cnt) rows.push_back({t - rs, i, cnt});  // forward: y = r on a row without L
+                    if (sweep || cnt || split) rows.push_back({t - rs, i, cnt});  // forward: y = r on a row without L
                 }
                 // rows of one block count together: a wavefront's rows run the same products
                 std::stable_sort(rows.begin(), rows.end(), [](const Row& a, const Row& b) { return a.cnt > b.cnt; });
@@ -151,6 +152,7 @@ static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp3
                                 ps.src.push_back(s);
                                 ps.rowCell.push_back(sweep ? w.i : -1);
                                 e[k++] = (uint16_t)(5 * pv.localCol[s]);
+                                need = std::max(need, pv.localCol[s] - nOwn + 1);
                             }
                         first += w.cnt + sweep;
                     }
@@ -158,6 +160,7 @@ static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp3
                     ps.hdr.push_back((uint32_t)nr | (uint32_t)(bytes / 16) << 16);
                     ps.recRows.push_back(ps.recRows.back() + nr);
                     ps.recBlk.push_back((int32_t)ps.src.size());
+                    if (split) ps.need.push_back(5 * need);
                     pos += bytes;
                     r0 = r1;
                 }
@@ -226,6 +229,7 @@ void StreamSet::upload() {
     d_entries.upload(entries);
     d_hdr.upload(hdr);
     d_start.upload(start);
+    d_need.upload(need);
     d_src.upload(src);
     d_rowCell.upload(rowCell);
     d_chain.upload(chain);
@@ -413,8 +417,8 @@ static void build_tiles(const Mesh& m, TileSet& ts) {
         std::fill(seen.begin(), seen.end(), -1);
         for (int t = 0; t < nT; ++t) {
             const int rs = ts.rowStart[t], nr = ts.rowStart[t + 1] - rs;
-            for (int q = rs; q < rs + nr; ++q) {
-                const int i = ts.rows[q];
+            for (int q0 = 0; q0 < nr; ++q0) {  // in the sweep's order of levels
+                const int i = ts.rows[sweep ? rs + nr - 1 - q0 : rs + q0];
                 const int s0 = sweep ? m.slotDiag[i] + 1 : m.rowPtr[i], s1 = sweep ? m.rowPtr[i + 1] : m.slotDiag[i];
                 for (int s = s0; s < s1; ++s) {
                     const int j = m.cols[s];

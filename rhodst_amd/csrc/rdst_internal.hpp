@@ -83,7 +83,9 @@ static constexpr uint32_t ELL_IDX_MASK = 0x3fffffffu;
 // 16.  The forward records hold each row's in-partition L blocks (rows without
 // one are left out); the backward ones, which follow them, hold per row Dinv
 // first (its column is the row itself) and then Dinv U for each in-partition U
-// block, so x = Dinv y - sum (Dinv U) x needs no separate diagonal solve.
+// block, so x = Dinv y - sum (Dinv U) x needs no separate diagonal solve.  In a
+// tile's stream (TileSet) every row has a forward entry, since that is where
+// its result is handed on.
 constexpr int kStreamKD = 8;     // most off-diagonal blocks of a row in one sweep
 constexpr int kStreamRows = 48;  // rows of a record: 4 wavefronts x 12 rows of 5 lanes
 // Ring bytes.  With the partition's vector (at most 1024 rows) that leaves
@@ -103,6 +105,7 @@ struct StreamSet {
     std::vector<int32_t> recRows, recBlk;   // [nRec + 1] first row entry, first block
     std::vector<uint16_t> entries;          // [rows][ent / 2]
     std::vector<uint32_t> hdr, start;       // [nRec]; [nRec + 1] first 16-byte unit
+    std::vector<int32_t> need;              // [nRec] halo values (5 x cells) the tile must have before this record (tiles only)
     std::vector<int32_t> src, rowCell;      // [blocks] block-CSR slot, or -(cell + 1) for Dinv; the row's cell in a backward record, else -1
     // The factor as a chain of diagonal blocks (no three coupled cells are
     // coupled pairwise): per row, in the partitions' row order, cell, lower
@@ -141,7 +144,7 @@ struct PartSet {
 // only ever wait for tiles taken before (backward: in reverse).  As a PartSet,
 // with localCol numbering the cells outside the tile that a row reads behind
 // the tile's own: halo cell q of tile t's forward sweep is haloF[haloFStart[t]
-// + q], column nRows(t) + q.
+// + q], column nRows(t) + q, in the order in which the sweep's levels read them.
 struct TileSet : PartSet {
     bool tried = false, ok = false;
     int maxSlots = 0;  // most rows + halo cells of a tile

@@ -1149,12 +1149,13 @@ void stream_launch(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV*
         hipLaunchKernelGGL((k_fill_unset<TV>), dim3(RED_MAXG), dim3(256), 0, k.s, (long)n5, ty.p, k.w.tickets.p);
     }
     const int grid = std::min(ts.nParts, 256);
-    hipLaunchKernelGGL((k_tile_sweep<TM, TV, KDU, false>), dim3(grid), dim3(STREAM_THREADS), shmem, k.s, ts.nParts,
+    const size_t tshmem = shmem + 20 * kTileCells;
+    hipLaunchKernelGGL((k_tile_sweep<TM, TV, KDU, false>), dim3(grid), dim3(TILE_THREADS), tshmem, k.s, ts.nParts,
                        k.w.tickets.p, ts.d_rowStart.p, ts.d_rows.p, ts.d_haloFStart.p, ts.d_haloF.p, ps.d_recBeg.p,
-                       ps.d_recMid.p, ps.d_hdr.p, ps.d_start.p, stream, r, ty.p, x);
-    hipLaunchKernelGGL((k_tile_sweep<TM, TV, KDU, true>), dim3(grid), dim3(STREAM_THREADS), shmem, k.s, ts.nParts,
+                       ps.d_recMid.p, ps.d_need.p, ps.d_hdr.p, ps.d_start.p, stream, r, ty.p, x);
+    hipLaunchKernelGGL((k_tile_sweep<TM, TV, KDU, true>), dim3(grid), dim3(TILE_THREADS), tshmem, k.s, ts.nParts,
                        k.w.tickets.p, ts.d_rowStart.p, ts.d_rows.p, ts.d_haloBStart.p, ts.d_haloB.p, ps.d_recBeg.p,
-                       ps.d_recMid.p, ps.d_hdr.p, ps.d_start.p, stream, (const TV*)ty.p, x, ty.p);
+                       ps.d_recMid.p, ps.d_need.p, ps.d_hdr.p, ps.d_start.p, stream, (const TV*)ty.p, x, ty.p);
 }
 template <class TM, class TV>
 void stream_apply(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV* r, TV* x, bool natural) {

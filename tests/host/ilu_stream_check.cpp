@@ -21,13 +21,19 @@ static double coef(int s) { return 0.05 + 0.1 * ((s * 2654435761u) % 1000) / 100
 static double dinv(int c) { return 0.5 + 0.3 * ((c * 40503u) % 1000) / 1000.0; }
 
 // one sweep's records over a partition's vector y (rows, then halo values)
-static int replay(const Mesh& m, const StreamSet& ps, bool fp32, int q0, int q1, bool bwd, int slots, std::vector<double>& y) {
+static int replay(const Mesh& m, const StreamSet& ps, bool fp32, int q0, int q1, bool bwd, int own, int slots,
+                  std::vector<double>& y) {
     const int blk = 25 * (fp32 ? 4 : 8);
+    const bool tiles = !ps.need.empty();
+    int need = 0;
+    std::vector<char> done(own, 0);
     for (int q = q0; q < q1; ++q) {
         const int nr = ps.recRows[q + 1] - ps.recRows[q], b0 = ps.recBlk[q], nb = ps.recBlk[q + 1] - b0;
         if ((int)(ps.hdr[q] & 0xffff) != nr || nr < 1 || nr > kStreamRows) return fail("rows of a record", q, nr);
         if (nr * ps.ent + ((nb * blk + 15) & ~15) > stream_record(fp32)) return fail("record too large", q);
         std::vector<double> nw(nr);
+        if (tiles && (ps.need[q] < need || ps.need[q] > 5 * (slots - own))) return fail("halo count", q, ps.need[q]);
+        if (tiles) need = ps.need[q];
         for (int j = 0; j < nr; ++j) {
             const uint16_t* e = ps.entries.data() + (size_t)(ps.recRows[q] + j) * (ps.ent / 2);
             const int t = e[0] / 5, cnt = e[1] >> 8;
@@ -44,14 +50,21 @@ static int replay(const Mesh& m, const StreamSet& ps, bool fp32, int q0, int q1,
             for (int k = 0; k < cnt; ++k, ++b) {
                 if (b >= ps.recBlk[q + 1]) return fail("block outside its record", q, j);
                 if (e[2 + k] % 5 || e[2 + k] / 5 >= slots) return fail("column out of range", q, e[2 + k]);
+                if (e[2 + k] >= 5 * own && e[2 + k] - 5 * own >= need) return fail("a halo value before it is there", q, j);
                 if (bwd != (ps.rowCell[b] >= 0)) return fail("sweep of a block", q, j);
                 a -= d * coef(ps.src[b]) * y[e[2 + k] / 5];
             }
             nw[j] = a;
         }
         // rows of a record are independent: storing them together changes nothing
-        for (int j = 0; j < nr; ++j) y[ps.entries[(size_t)(ps.recRows[q] + j) * (ps.ent / 2)] / 5] = nw[j];
+        for (int j = 0; j < nr; ++j) {
+            const int t = ps.entries[(size_t)(ps.recRows[q] + j) * (ps.ent / 2)] / 5;
+            y[t] = nw[j];
+            ++done[t];
+        }
     }
+    for (int t = 0; t < own && tiles; ++t)
+        if (done[t] != 1) return fail("a tile's row is not in one record", t);
     return 0;
 }
 
@@ -167,7 +180,7 @@ static int check(const rdst_mesh_desc* desc, bool fp32, bool natural) {
                 if ((int)v.size() > ts.maxSlots) return fail("slots", p);
             }
             const int q0 = sweep ? ps.recMid[p] : ps.recBeg[p], q1 = sweep ? ps.recBeg[p + 1] : ps.recMid[p];
-            if (int e = replay(m, ps, fp32, q0, q1, sweep != 0, (int)v.size(), v)) return e;
+            if (int e = replay(m, ps, fp32, q0, q1, sweep != 0, nr, natural && nP > 1 ? (int)v.size() : nr, v)) return e;
             for (int q = 0; q < nr; ++q) {
                 (sweep ? x : y)[rows[rs + q]] = v[q];
                 have[rows[rs + q]] = 1;
