@@ -350,8 +350,8 @@ __global__ __launch_bounds__(STREAM_THREADS) void k_stream_apply(const int32_t* 
 // which the records read them.  A tile so runs a few levels behind the ones it
 // depends on, and a sweep costs about the levels of the whole mesh, not tiles
 // in a row times levels of a tile: with every halo value awaited at a tile's
-// start the sweeps took 365 us (RAE2822, 23.5 k cells, 27 tiles in a row) and 765
-// (wing, 321 k, 32 in a row), now 212 and 460.  By one launch per level (8-10 us
+// start the sweeps took 365 us (RAE2822, 23.5 k cells, 431 levels) and 765 (wing,
+// 321 k, 260 levels), now 180 and 232.  By one launch per level (8-10 us
 // each, or 3.3 us per level in a single-workgroup run of small levels) it was
 // 1.5 ms and 2.3 ms.
 template <class T>

@@ -372,7 +372,11 @@ static void build_tiles(const Mesh& m, TileSet& ts) {
             for (int c = 0; c < 3; ++c) x[3 * (size_t)i + c] = std::max(x[3 * (size_t)i + c], x[3 * (size_t)j + c] + (c == cl ? 1 : 0));
             lev[i] = std::max(lev[i], lev[j] + 1);
         }
-    const int T[3] = {three ? 8 : 16, three ? 8 : 16, 8};
+    // Box sides.  Small boxes hand on sooner, but more of them cross more halos (1-2 us
+    // each) and the whole mesh's worth must be held by 256 workgroups.  Measured, step
+    // of a 321 k wing: 8x8x8 45.9 ms, 6x6x6 38.1, 8x8x4 35.7, 8x4x2 32.6, 4x4x4 31.0,
+    // 8x4x4 30.9; RAE2822 (two classes): 16x16 and 8x8 20.8, 16x8 18.9.
+    const int T[3] = {three ? 8 : 16, three ? 4 : 8, 4};
     std::vector<int32_t> tile(n, 0);
     int nT = 0;
     if (n <= kPartCells) {
