@@ -559,12 +559,24 @@ __device__ inline int seed_of(const int32_t* color, int i, int col, int comp) {
     return (col >= 0 && color[i] == col) ? comp : -1;
 }
 
+// Forward-mode passes are numbered 5 x colour + component; a launch does
+// gridDim.y of them from pass0 on (pass0 < 0: one without a seed, values only),
+// each with scratch of its own.
+__device__ inline void pass_of(int pass0, int& col, int& comp) {
+    const int p = pass0 + (int)blockIdx.y;
+    col = pass0 < 0 ? -1 : p / 5;
+    comp = pass0 < 0 ? 0 : p - 5 * col;
+}
+
 // fvc::grad(U) of every cell, value and tangent: gd[q n + c], gd[(9 + q) n + c]
 __global__ __launch_bounds__(256) void k_av_grad(MeshDev m, Fields F, const BcPatchDev* bc, Thermo th, Bounds bd,
-                                                 const int32_t* color, int col, int comp, double* gd) {
+                                                 const int32_t* color, int pass0, double* gd) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= m.nC) return;
     const int n = m.nC;
+    int col, comp;
+    pass_of(pass0, col, comp);
+    gd += (size_t)blockIdx.y * 18 * n;
     const size_t E = (size_t)m.ellW * m.nC;
     const Prim<D1> Pc = seeded(F.W, c, seed_of(color, c, col, comp), th, bd);
     D1 g[9];
@@ -607,20 +619,24 @@ __global__ __launch_bounds__(256) void k_av_grad(MeshDev m, Fields F, const BcPa
     }
 }
 
-// the residual (inviscid flux + viscous terms) of every cell, value Rv and
-// tangent Jv [n][5], and the tangent of the cell's share of the force
+// the residual (inviscid flux + viscous terms) of every cell, value Rv [n][5],
+// its tangent where row c of the second-neighbour matrix Jw couples with the
+// one column of the pass's colour (column comp of that block), and the tangent of the cell's share of the force
 // objective (its faces on the patch: pressure and viscous force . dir / q)
 template <int S>
 __global__ __launch_bounds__(256) void k_av_resid(MeshDev m, Fields F, const BcPatchDev* bc, Thermo th, Bounds bd,
                                                   int lowMach, double Mainf, double lapPsi, double snPsi, int heat,
-                                                  const int32_t* color, int col, int comp, const double* gd,
-                                                  double* Rv, double* Jv, int patch, double dx, double dy, double dz,
+                                                  const int32_t* color, int pass0, const double* gd, double* Rv,
+                                                  const int32_t* wRowPtr, const int32_t* wCols, double* Jw, int patch, double dx, double dy, double dz,
                                                   double rq, double pRef, double* objd, double* objv) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= m.nC) return;
     const int n = m.nC;
     const size_t E = (size_t)m.ellW * m.nC;
     const double gamma = th.gamma;
+    int col, comp;
+    pass_of(pass0, col, comp);
+    gd += (size_t)blockIdx.y * 18 * n;
     const Prim<D1> Pc = seeded(F.W, c, seed_of(color, c, col, comp), th, bd);
     const SideT<D1> sc = side_of(Pc, gamma);
     D1 gC[9], tauC[9];
@@ -742,33 +758,27 @@ __global__ __launch_bounds__(256) void k_av_resid(MeshDev m, Fields F, const BcP
     r[3] = a[3] / V - (lz / V + tz / V);
     r[4] = a[4] / V - sd / V;
     if (heat) r[4] -= hq / V;
-    for (int q = 0; q < 5; ++q) {
-        if (Rv) Rv[5 * (size_t)c + q] = r[q].v;
-        if (Jv) Jv[5 * (size_t)c + q] = r[q].d;
-    }
-    if (objd) objd[c] = ob.d;
+    if (Rv)
+        for (int q = 0; q < 5; ++q) Rv[5 * (size_t)c + q] = r[q].v;
+    if (Jw)
+        for (int e = wRowPtr[c]; e < wRowPtr[c + 1]; ++e)
+            if (color[wCols[e]] == col) {
+                for (int q = 0; q < 5; ++q) Jw[25 * (size_t)e + 5 * q + comp] = r[q].d;
+                break;
+            }
+    if (objd) objd[(size_t)blockIdx.y * n + c] = ob.d;
     if (objv) objv[c] = ob.v;
-}
-
-// column comp of the blocks of this pass's colour: row r's tangent is the
-// block (r, j) of the one column j of the colour in row r
-__global__ void k_av_scatter(int n, const int32_t* rowPtr, const int32_t* cols, const int32_t* color, int col,
-                             int comp, const double* Jv, double* Jw) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n) return;
-    for (int e = rowPtr[r]; e < rowPtr[r + 1]; ++e)
-        if (color[cols[e]] == col) {
-            for (int q = 0; q < 5; ++q) Jw[25 * (size_t)e + 5 * q + comp] = Jv[5 * (size_t)r + q];
-            return;
-        }
 }
 
 // dJ/dW of the cells of this pass's colour: the objective share of a cell
 // depends on the cell and its face neighbours, so cell j collects the
 // tangents of itself and of its neighbours
-__global__ void k_av_obj_gather(MeshDev m, const int32_t* color, int col, int comp, const double* objd, double* g) {
+__global__ void k_av_obj_gather(MeshDev m, const int32_t* color, int pass0, const double* objd, double* g) {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    int col, comp;
+    pass_of(pass0, col, comp);
     if (j >= m.nC || color[j] != col) return;
+    objd += (size_t)blockIdx.y * m.nC;
     double s = objd[j];
     for (int ke = 0; ke < m.ellW; ++ke) {
         const size_t e = (size_t)ke * m.nC + j;
@@ -834,39 +844,61 @@ void launch_res(Case& c, double* R) {
                        bounds_of(c), c.st.low_mach, c.st.Mainf, R);
 }
 
+// where the residual of a launch goes (null: not wanted)
+struct AvOut {
+    double* Rv = nullptr;    // values
+    double* Jw = nullptr;    // tangents, into the second-neighbour matrix
+    double* objd = nullptr;  // tangents and values of the objective's shares
+    double* objv = nullptr;
+    int patch = -1;
+    const double* dir = nullptr;
+    double rq = 0.0, pRef = 0.0;
+};
+
 template <int S>
-void launch_av_resid(Case& c, int col, int comp, double* Rv, double* Jv, int patch, const double* dir, double rq,
-                     double* objd, double pRef = 0.0, double* objv = nullptr) {
+void launch_av_resid(Case& c, int pass0, int nPass, const AvOut& o) {
     const Mesh& m = *c.mesh;
-    const int nb = blocks_for(m.nC, 256);
-    hipLaunchKernelGGL((k_av_resid<S>), dim3(nb), dim3(256), 0, c.stream, c.meshDev(), c.f, c.d_bc.p, c.th, bounds_of(c),
+    const dim3 grid(blocks_for(m.nC, 256), nPass);
+    hipLaunchKernelGGL((k_av_resid<S>), grid, dim3(256), 0, c.stream, c.meshDev(), c.f, c.d_bc.p, c.th, bounds_of(c),
                        c.st.low_mach, c.st.Mainf, sngrad_psi(c.st.laplacian_sngrad, c.st.laplacian_limit),
-                       sngrad_psi(c.st.sngrad, c.st.sngrad_limit), c.st.heat_conduction, m.d_wideColor.p, col, comp,
-                       c.avGrad.p, Rv, Jv, patch, dir ? dir[0] : 0.0, dir ? dir[1] : 0.0, dir ? dir[2] : 0.0, rq, pRef,
-                       objd, objv);
+                       sngrad_psi(c.st.sngrad, c.st.sngrad_limit), c.st.heat_conduction, m.d_wideColor.p, pass0,
+                       c.avGrad.p, o.Rv, m.d_wideRowPtr.p, m.d_wideCols.p, o.Jw, o.patch, o.dir ? o.dir[0] : 0.0,
+                       o.dir ? o.dir[1] : 0.0, o.dir ? o.dir[2] : 0.0, o.rq, o.pRef, o.objd, o.objv);
 }
 
-// one forward-mode pass: gradient, then residual (and objective) tangents
-// of the seed (colour col, component comp); col < 0: values only
-void av_pass(Case& c, int col, int comp, double* Rv, double* Jv, int patch, const double* dir, double rq, double* objd) {
+// nPass forward-mode passes from pass0 on: gradient, then residual (and
+// objective) tangents of the seeds; pass0 < 0: values only
+void av_pass(Case& c, int pass0, int nPass, const AvOut& o) {
     const Mesh& m = *c.mesh;
-    hipLaunchKernelGGL(k_av_grad, dim3(blocks_for(m.nC, 256)), dim3(256), 0, c.stream, c.meshDev(), c.f, c.d_bc.p, c.th,
-                       bounds_of(c), m.d_wideColor.p, col, comp, c.avGrad.p);
+    hipLaunchKernelGGL(k_av_grad, dim3(blocks_for(m.nC, 256), nPass), dim3(256), 0, c.stream, c.meshDev(), c.f, c.d_bc.p,
+                       c.th, bounds_of(c), m.d_wideColor.p, pass0, c.avGrad.p);
     switch (c.st.flux_scheme) {
-        case RDST_FLUX_AUSMPLUS: launch_av_resid<RDST_FLUX_AUSMPLUS>(c, col, comp, Rv, Jv, patch, dir, rq, objd); break;
-        case RDST_FLUX_AUSMPLUSUP: launch_av_resid<RDST_FLUX_AUSMPLUSUP>(c, col, comp, Rv, Jv, patch, dir, rq, objd); break;
-        case RDST_FLUX_HLL: launch_av_resid<RDST_FLUX_HLL>(c, col, comp, Rv, Jv, patch, dir, rq, objd); break;
-        case RDST_FLUX_HLLC: launch_av_resid<RDST_FLUX_HLLC>(c, col, comp, Rv, Jv, patch, dir, rq, objd); break;
-        default: launch_av_resid<RDST_FLUX_KURGANOV>(c, col, comp, Rv, Jv, patch, dir, rq, objd); break;
+        case RDST_FLUX_AUSMPLUS: launch_av_resid<RDST_FLUX_AUSMPLUS>(c, pass0, nPass, o); break;
+        case RDST_FLUX_AUSMPLUSUP: launch_av_resid<RDST_FLUX_AUSMPLUSUP>(c, pass0, nPass, o); break;
+        case RDST_FLUX_HLL: launch_av_resid<RDST_FLUX_HLL>(c, pass0, nPass, o); break;
+        case RDST_FLUX_HLLC: launch_av_resid<RDST_FLUX_HLLC>(c, pass0, nPass, o); break;
+        default: launch_av_resid<RDST_FLUX_KURGANOV>(c, pass0, nPass, o); break;
     }
     RDST_HIP(hipGetLastError());
 }
 
+// Passes of one launch: one pass over a mesh of a few hundred blocks leaves most
+// of the chip idle (a block per CU, one wavefront per SIMD), so several go
+// together until there are some AV_BLOCKS blocks; a mesh of that many blocks by
+// itself takes one pass at a time, with the scratch it always had.  The scratch of a
+// launch stays below 19 doubles x 256 x AV_BLOCKS (160 MB).
+constexpr int AV_BLOCKS = 4096;
+int av_batch(const Mesh& m) { return std::max(1, std::min(5 * m.wideColors, AV_BLOCKS / std::max(1, blocks_for(m.nC, 256)))); }
+// passes [0, 5 x colours) in batches: f(pass0, nPass)
+template <class Fn>
+void av_batches(const Mesh& m, Fn f) {
+    const int total = 5 * m.wideColors, step = av_batch(m);
+    for (int p = 0; p < total; p += step) f(p, std::min(step, total - p));
+}
+
 void av_buffers(Case& c) {
-    const size_t n = (size_t)c.mesh->nC;
+    const size_t n = (size_t)c.mesh->nC * av_batch(*c.mesh);
     if (c.avGrad.n != 18 * n) c.avGrad.alloc(18 * n);
-    if (c.avR.n != 5 * n) c.avR.alloc(5 * n);
-    if (c.avJv.n != 5 * n) c.avJv.alloc(5 * n);
     if (c.avObj.n != n) c.avObj.alloc(n);
 }
 
@@ -943,13 +975,9 @@ void viscous_linearise(Case& c) {
     const size_t nnz = m.wideCols.size();
     if (c.adjW.n != 25 * nnz) c.adjW.alloc(25 * nnz);
     if (c.adjWT.n != 25 * nnz) c.adjWT.alloc(25 * nnz);
-    const int nb = blocks_for(m.nC, 256);
-    for (int col = 0; col < m.wideColors; ++col)
-        for (int comp = 0; comp < 5; ++comp) {
-            av_pass(c, col, comp, nullptr, c.avJv.p, -1, nullptr, 0.0, nullptr);
-            hipLaunchKernelGGL(k_av_scatter, dim3(nb), dim3(256), 0, c.stream, m.nC, m.d_wideRowPtr.p, m.d_wideCols.p,
-                               m.d_wideColor.p, col, comp, c.avJv.p, c.adjW.p);
-        }
+    AvOut out;
+    out.Jw = c.adjW.p;
+    av_batches(m, [&](int p0, int np) { av_pass(c, p0, np, out); });
     const int gb = std::min(4096, blocks_for((long)nnz, 256));
     hipLaunchKernelGGL(k_wide_transpose, dim3(gb), dim3(256), 0, c.stream, (long)nnz, m.d_wideT.p, c.adjW.p, c.adjWT.p);
     const size_t nn = 25 * (size_t)m.nnzb;
@@ -1059,7 +1087,9 @@ void adjoint_residual(Case& c, double* R) {
     if (c.st.viscous) {
         build_wide(*c.mesh);
         av_buffers(c);
-        av_pass(c, -1, 0, R, nullptr, -1, nullptr, 0.0, nullptr);
+        AvOut out;
+        out.Rv = R;
+        av_pass(c, -1, 1, out);
         return;
     }
     switch (c.st.flux_scheme) {
@@ -1080,12 +1110,16 @@ void adjoint_objective_gradient(Case& c, int patch, const double* dir, double q,
         Mesh& m = *c.mesh;
         build_wide(m);
         av_buffers(c);
-        for (int col = 0; col < m.wideColors; ++col)
-            for (int comp = 0; comp < 5; ++comp) {
-                av_pass(c, col, comp, nullptr, nullptr, patch, dir, 1.0 / q, c.avObj.p);
-                hipLaunchKernelGGL(k_av_obj_gather, dim3(blocks_for(m.nC, 256)), dim3(256), 0, c.stream, c.meshDev(),
-                                   m.d_wideColor.p, col, comp, c.avObj.p, g);
-            }
+        AvOut out;
+        out.patch = patch;
+        out.dir = dir;
+        out.rq = 1.0 / q;
+        out.objd = c.avObj.p;
+        av_batches(m, [&](int p0, int np) {
+            av_pass(c, p0, np, out);
+            hipLaunchKernelGGL(k_av_obj_gather, dim3(blocks_for(m.nC, 256), np), dim3(256), 0, c.stream, c.meshDev(),
+                               m.d_wideColor.p, p0, c.avObj.p, g);
+        });
         RDST_HIP(hipGetLastError());
         return;
     }
@@ -1103,24 +1137,13 @@ void adjoint_objective_cells(Case& c, int patch, const double* dir, double q, do
     if (c.st.viscous) {
         build_wide(m);
         av_buffers(c);
-        hipLaunchKernelGGL(k_av_grad, dim3(blocks_for(m.nC, 256)), dim3(256), 0, c.stream, c.meshDev(), c.f, c.d_bc.p,
-                           c.th, bounds_of(c), m.d_wideColor.p, -1, 0, c.avGrad.p);
-        switch (c.st.flux_scheme) {
-            case RDST_FLUX_AUSMPLUS:
-                launch_av_resid<RDST_FLUX_AUSMPLUS>(c, -1, 0, nullptr, nullptr, patch, dir, 1.0 / q, nullptr, pRef, o);
-                break;
-            case RDST_FLUX_AUSMPLUSUP:
-                launch_av_resid<RDST_FLUX_AUSMPLUSUP>(c, -1, 0, nullptr, nullptr, patch, dir, 1.0 / q, nullptr, pRef, o);
-                break;
-            case RDST_FLUX_HLL:
-                launch_av_resid<RDST_FLUX_HLL>(c, -1, 0, nullptr, nullptr, patch, dir, 1.0 / q, nullptr, pRef, o);
-                break;
-            case RDST_FLUX_HLLC:
-                launch_av_resid<RDST_FLUX_HLLC>(c, -1, 0, nullptr, nullptr, patch, dir, 1.0 / q, nullptr, pRef, o);
-                break;
-            default:
-                launch_av_resid<RDST_FLUX_KURGANOV>(c, -1, 0, nullptr, nullptr, patch, dir, 1.0 / q, nullptr, pRef, o);
-        }
+        AvOut out;
+        out.patch = patch;
+        out.dir = dir;
+        out.rq = 1.0 / q;
+        out.pRef = pRef;
+        out.objv = o;
+        av_pass(c, -1, 1, out);
     } else {
         hipLaunchKernelGGL(k_adj_objective_cells, dim3(blocks_for(m.nC, 256)), dim3(256), 0, c.stream, c.meshDev(), c.f,
                            c.d_bc.p, c.th, bounds_of(c), patch, dir[0], dir[1], dir[2], 1.0 / q, pRef, o);

@@ -399,7 +399,7 @@ struct Case {
     DBuf<double> adjW, adjWT;
     DBuf<double> adjPT;  // the preconditioner's matrix with a pseudo-time shift
     DBuf<float> adjWT32;
-    DBuf<double> avGrad, avR, avJv, avObj;  // scratch of the forward-mode passes
+    DBuf<double> avGrad, avObj;             // scratch of the forward-mode passes
     bool adjWide = false;                   // the last linearisation is the second-neighbour one
 
     MeshDev meshDev() const;
