@@ -13,7 +13,7 @@
 // straight into the sweeps' record stream: no copy of A, no factor matrix.
 // Measured, this kernel with its pack against thread per row, copy and pack:
 // FP32 partitions 2 M cells 2.16 / 5.8 ms, 24 k cells 0.25 / 0.52 ms; FP64 natural
-// order 252 cells 0.20 / 0.52 ms, 23.5 k 4.5 / 9.5 ms, 321 k 5.5 / 9.9 ms.
+// order 252 cells 0.19 / 0.52 ms, 23.5 k 2.2 / 9.5 ms, 321 k 2.1 / 9.9 ms.
 #pragma once
 #include "rdst_internal.hpp"
 
@@ -86,59 +86,61 @@ __device__ __forceinline__ int inv5_lanes(T (&a)[5], T (&b)[5], int base, int r)
 
 constexpr int CHAIN_THREADS = 256;  // 4 wavefronts x 12 rows of 5 lanes
 
-// A row of the chain and its part of A, row r of each block in this lane.
+// A row of the chain (row entry t of StreamSet::chain) and its part of A, row r
+// of each block in this lane.
+template <int K>
+struct ChainEntry {
+    int4 h, n[K];
+};
 template <class T, int K>
 struct ChainRegs {
-    int cell, cnt, lk[K];
+    int cell, cnt, lk[K];  // lk: the neighbour's cell, or its column in the tile
     uint32_t dDst, lDst[K];
     T d[5], a[K][5], u[K][5];
 };
-template <class T, int K>
-__device__ __forceinline__ void chain_load(const int32_t* __restrict__ rows, long t, int r, const T* __restrict__ A,
-                                           ChainRegs<T, K>& R) {
+template <int K>
+__device__ __forceinline__ void chain_entry(const int32_t* __restrict__ rows, long t, ChainEntry<K>& E) {
     const int4* e = reinterpret_cast<const int4*>(rows + (4 + 4 * K) * (size_t)t);
-    const int4 h = e[0];
-    int4 n[K];
+    E.h = e[0];
 #pragma unroll
-    for (int k = 0; k < K; ++k) n[k] = e[1 + k];
-    R.cell = h.x;
-    R.cnt = h.y;
-    R.dDst = (uint32_t)h.w;
-    const T* p = A + 25 * (size_t)h.z + 5 * r;
+    for (int k = 0; k < K; ++k) E.n[k] = e[1 + k];
+}
+template <class T, int K>
+__device__ __forceinline__ void chain_load(const ChainEntry<K>& E, int r, const T* __restrict__ A, ChainRegs<T, K>& R) {
+    R.cell = E.h.x;
+    R.cnt = E.h.y;
+    R.dDst = (uint32_t)E.h.w;
+    const T* p = A + 25 * (size_t)E.h.z + 5 * r;
 #pragma unroll
     for (int c = 0; c < 5; ++c) R.d[c] = p[c];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        R.lk[k] = n[k].z;
-        R.lDst[k] = (uint32_t)n[k].w;
-        const T* pa = A + 25 * (size_t)n[k].x + 5 * r;
-        const T* pu = A + 25 * (size_t)n[k].y + 5 * r;
+        R.lk[k] = E.n[k].z;
+        R.lDst[k] = (uint32_t)E.n[k].w;
+        const T* pa = A + 25 * (size_t)E.n[k].x + 5 * r;
+        const T* pu = A + 25 * (size_t)E.n[k].y + 5 * r;
 #pragma unroll
         for (int c = 0; c < 5; ++c) { R.a[k][c] = pa[c]; R.u[k][c] = pu[c]; }
     }
 }
-template <class T, int K>
-__device__ __forceinline__ void chain_row(const ChainRegs<T, K>& R, bool on, int base, int r, T* Dinv, uint8_t* stream,
-                                          int* fail) {
-    T d[5];
+// own: the row's place in LDS (TILE), where the tile's Dinv and its halo's are
+// kept; outside it they are read from Dinv itself.
+template <class T, int K, bool TILE>
+__device__ __forceinline__ void chain_row(const ChainRegs<T, K>& R, bool on, int base, int r, T* Dinv, T* lds, int own,
+                                          uint8_t* stream, int* fail) {
+    T d[5], l[K][5];
 #pragma unroll
     for (int c = 0; c < 5; ++c) d[c] = R.d[c];
 #pragma unroll
     for (int k = 0; k < K; ++k)
         if (k < R.cnt) {
-            const T* Dk = Dinv + 25 * (size_t)R.lk[k];
-            T l[5];
+            const T* Dk = (TILE ? lds : Dinv) + 25 * (size_t)R.lk[k];
 #pragma unroll
             for (int j = 0; j < 5; ++j) {
                 T s = 0;
 #pragma unroll
                 for (int q = 0; q < 5; ++q) s += R.a[k][q] * Dk[5 * q + j];
-                l[j] = s;
-            }
-            if (on) {
-                T* o = reinterpret_cast<T*>(stream + 4 * (size_t)R.lDst[k]) + 5 * r;
-#pragma unroll
-                for (int j = 0; j < 5; ++j) o[j] = l[j];
+                l[k][j] = s;
             }
             T u[5][5];
 #pragma unroll
@@ -149,48 +151,87 @@ __device__ __forceinline__ void chain_row(const ChainRegs<T, K>& R, bool on, int
             for (int j = 0; j < 5; ++j) {
                 T s = 0;
 #pragma unroll
-                for (int q = 0; q < 5; ++q) s += l[q] * u[q][j];
+                for (int q = 0; q < 5; ++q) s += l[k][q] * u[q][j];
                 d[j] -= s;
             }
         }
     T b[5];
-    const int row = inv5_lanes(d, b, base, r);
+    int row = inv5_lanes(d, b, base, r);
+    // the next pass's blocks have arrived by now: waited for here (vmcnt 0), so
+    // that using them does not wait behind the stores below
+    __builtin_amdgcn_s_waitcnt(0x0f70);
     if (!on) return;
-    if (row < 0) {
+    if (row < 0) {  // the caller fails; whoever waits for this block goes on
         atomicExch(fail, 1);
-        return;
+        row = r;
+#pragma unroll
+        for (int c = 0; c < 5; ++c) b[c] = T(0);
     }
     T* g = Dinv + 25 * (size_t)R.cell + 5 * row;
     T* o = reinterpret_cast<T*>(stream + 4 * (size_t)R.dDst) + 5 * row;
 #pragma unroll
-    for (int c = 0; c < 5; ++c) { g[c] = b[c]; o[c] = b[c]; }
+    for (int c = 0; c < 5; ++c) {
+        if constexpr (TILE) {
+            lds[25 * own + 5 * row + c] = b[c];
+            store_dev(g + c, b[c]);
+        } else {
+            g[c] = b[c];
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 5; ++c) o[c] = b[c];
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        if (k < R.cnt) {
+            T* p = reinterpret_cast<T*>(stream + 4 * (size_t)R.lDst[k]) + 5 * r;
+#pragma unroll
+            for (int j = 0; j < 5; ++j) p[j] = l[k][j];
+        }
 }
 
-// One partition's (or tile's) rows level by level; the rows of the pass after
-// this one are loaded before this one is computed.
-template <class T, int K>
+// One partition's (or tile's) rows level by level, NW wavefronts, for a tile two
+// barriers before the first level, and one after each.  A pass is 12 NW rows of a
+// level; the blocks of the pass after this one are loaded before this one is
+// computed, and the entries of the one after that.
+template <class T, int K, int NW, bool TILE>
 __device__ __forceinline__ void chain_levels(int l0, int l1, const int32_t* __restrict__ levPtr,
-                                             const int32_t* __restrict__ rows, const T* __restrict__ A, T* Dinv,
+                                             const int32_t* __restrict__ rows, const T* __restrict__ A, T* Dinv, T* lds,
                                              uint8_t* stream, int* fail) {
     const int lane = threadIdx.x & 63, g = lane / 5, r = lane - 5 * g, base = lane - r;
-    const int w12 = 12 * (int)(threadIdx.x >> 6), slot = g < 12 ? w12 + g : 1 << 20;
-    int L = l0, s = levPtr[l0], e = levPtr[l0 + 1];
+    const int w12 = 12 * (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), slot = g < 12 ? w12 + g : 1 << 20;
+    struct Pass {
+        int L, s, e;  // level, its rows from this pass on
+    };
+    auto after = [&](Pass p) {
+        if (p.s + 12 * NW < p.e) return Pass{p.L, p.s + 12 * NW, p.e};
+        return Pass{p.L + 1, p.e, p.L + 2 < l1 ? levPtr[p.L + 2] : p.e};
+    };
+    // lanes without a row (past the last level: all) work on the last row there is and store nothing
+    auto row_of = [&](Pass p) { return max(min(p.s + slot, p.e - 1), p.s - 1); };
+    Pass p0 = {l0, levPtr[l0], levPtr[l0 + 1]};
+    const int first = p0.s;
+    Pass p1 = after(p0);
     ChainRegs<T, K> cur, nxt;
-    // lanes without a row work on the pass's last row and store nothing
-    chain_load<T, K>(rows, min(s + slot, e - 1), r, A, cur);
-    while (L + 1 < l1) {
-        int nL = L, ns = s + CHAIN_THREADS / 64 * 12, ne = e;
-        if (ns >= e) {
-            nL = L + 1;
-            ns = e;
-            ne = nL + 1 < l1 ? levPtr[nL + 1] : e;
-        }
-        const bool more = nL + 1 < l1;
-        if (more) chain_load<T, K>(rows, min(ns + slot, ne - 1), r, A, nxt);
-        if (s + w12 < e) chain_row<T, K>(cur, s + slot < e, base, r, Dinv, stream, fail);
-        if (nL != L) __syncthreads();  // rows of a later level read what this one stored
-        L = nL; s = ns; e = ne;
-        if (more) cur = nxt;
+    ChainEntry<K> ent;
+    chain_entry<K>(rows, row_of(p0), ent);
+    chain_load<T, K>(ent, r, A, cur);
+    chain_entry<K>(rows, row_of(p1), ent);
+    if constexpr (TILE) {
+        barrier_lds();
+        barrier_lds();
+    }
+    while (p0.L + 1 < l1) {
+        const Pass p2 = p1.L + 1 < l1 ? after(p1) : p1;
+        chain_load<T, K>(ent, r, A, nxt);
+        chain_entry<K>(rows, row_of(p2), ent);
+        if (p0.s + w12 < p0.e)
+            chain_row<T, K, TILE>(cur, p0.s + slot < p0.e, base, r, Dinv, lds, row_of(p0) - first, stream, fail);
+        else
+            __builtin_amdgcn_s_waitcnt(0x0f70);  // as in chain_row, or the next pass waits for its stores
+        if (p1.L != p0.L) barrier_lds();  // rows of a later level read what this one stored
+        p0 = p1;
+        p1 = p2;
+        cur = nxt;
     }
 }
 
@@ -200,41 +241,48 @@ __global__ __launch_bounds__(CHAIN_THREADS) void k_ilu_chain(const int32_t* __re
                                                              const int32_t* __restrict__ rows, const T* __restrict__ A,
                                                              T* Dinv, uint8_t* stream, int* fail) {
     const int p = blockIdx.x;
-    chain_levels<T, K>(levStart[p], levStart[p + 1], levPtr, rows, A, Dinv, stream, fail);
+    chain_levels<T, K, CHAIN_THREADS / 64, false>(levStart[p], levStart[p + 1], levPtr, rows, A, Dinv, (T*)nullptr, stream, fail);
 }
 
 // The natural-order factor by tiles, taken by ticket in an order that respects
-// their dependencies (see k_tile_sweep); done[t] = epoch releases tile t's Dinv.
+// their dependencies and pipelined as k_tile_sweep's: Dinv is unset before, each
+// row's is stored as it is computed, and a wavefront of its own polls for the
+// halo's.  The tile's Dinv and its halo's are kept in LDS.  A level costs 4.6 us,
+// nearly all of it the dependent instructions of a row.  With tiles that waited for
+// their predecessors to end, and Dinv read back from memory, the factor took 3.9 ms
+// (RAE2822, 23.5 k cells) and 4.35 (wing, 321 k), now 2.07 and 1.79.
+// Three wavefronts compute (a level of a tile has 10-20 rows): with the halo's one
+// per SIMD, so that all of a pass and the next one stay in registers.
+constexpr int CHAIN_TILE_WAVES = 3, CHAIN_TILE_THREADS = 64 * (CHAIN_TILE_WAVES + 1);
 template <class T, int K>
-__global__ __launch_bounds__(CHAIN_THREADS) void k_ilu_chain_tiles(int nT, int* ticket, int* done, int epoch,
-                                                                   const int32_t* __restrict__ predStart,
-                                                                   const int32_t* __restrict__ pred,
-                                                                   const int32_t* __restrict__ levStart,
-                                                                   const int32_t* __restrict__ levPtr,
-                                                                   const int32_t* __restrict__ rows,
-                                                                   const T* __restrict__ A, T* Dinv, uint8_t* stream,
-                                                                   int* fail) {
+__global__ __launch_bounds__(CHAIN_TILE_THREADS) void k_ilu_chain_tiles(int nT, int* ticket,
+                                                                        const int32_t* __restrict__ rowStart,
+                                                                        const int32_t* __restrict__ haloStart,
+                                                                        const int32_t* __restrict__ halo,
+                                                                        const int32_t* __restrict__ need,
+                                                                        const int32_t* __restrict__ levStart,
+                                                                        const int32_t* __restrict__ levPtr,
+                                                                        const int32_t* __restrict__ rows,
+                                                                        const T* __restrict__ A, T* Dinv,
+                                                                        uint8_t* stream, int* fail) {
+    extern __shared__ __align__(16) unsigned char chain_raw[];
+    T* lds = reinterpret_cast<T*>(chain_raw);
     __shared__ int cur;
     if (threadIdx.x == 0) cur = atomicAdd(ticket, 1);
     __syncthreads();
     for (;;) {
         const int t = __builtin_amdgcn_readfirstlane(cur);
         if (t >= nT) break;
-        for (int q = predStart[t] + (int)threadIdx.x; q < predStart[t + 1]; q += CHAIN_THREADS)
-            while (__hip_atomic_load(done + pred[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch)
-                __builtin_amdgcn_s_sleep(2);
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        __syncthreads();
-        chain_levels<T, K>(levStart[t], levStart[t + 1], levPtr, rows, A, Dinv, stream, fail);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        __syncthreads();
-        // Flag and next ticket under one condition, the barrier behind it: split
-        // over the loop's end, with no barrier between, the compiler joins the two
-        // across the back edge and lane 0 leaves its wavefront to loop without it.
-        if (threadIdx.x == 0) {
-            __hip_atomic_store(done + t, epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-            cur = atomicAdd(ticket, 1);
+        const int l0 = levStart[t], l1 = levStart[t + 1];
+        if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == CHAIN_TILE_WAVES) {
+            const int h0 = haloStart[t];
+            stream_halo<T, 25, 12>(halo + h0, haloStart[t + 1] - h0, need + l0, l1 - l0 - 1, (const T*)Dinv,
+                                   lds + 25 * (rowStart[t + 1] - rowStart[t]));
+        } else {
+            chain_levels<T, K, CHAIN_TILE_WAVES, true>(l0, l1, levPtr, rows, A, Dinv, lds, stream, fail);
         }
+        __syncthreads();  // every wavefront has read cur
+        if (threadIdx.x == 0) cur = atomicAdd(ticket, 1);
         __syncthreads();
     }
 }

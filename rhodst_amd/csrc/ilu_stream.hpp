@@ -361,52 +361,58 @@ __global__ __launch_bounds__(256) void k_fill_unset(long n, T* y, int* tickets) 
     if (blockIdx.x == 0 && threadIdx.x < 2) tickets[threadIdx.x] = 0;
 }
 
-// The halo wavefront: the values of the cells outside the tile into LDS, each
-// as soon as it has arrived, in step with the records (barriers as in
-// stream_load): before record s starts, the first need[s] are there.  A window
-// of 256 values is asked for at a time; what has not arrived is asked for again.
-template <class TV>
-__device__ __forceinline__ void stream_halo(const int32_t* cells, int nh5, const int32_t* need_, int n, const TV* x, TV* y) {
-    constexpr int U = 4, W = 64 * U;
+// The halo wavefront: the NV values of each cell outside the tile into LDS, each
+// as soon as it has arrived, in step with the n records (barriers as in
+// stream_load): before record s starts, those of the first need[s] cells are
+// there.  A window of 64 U values is asked for at a time; what has not arrived is
+// asked for again.
+template <class TV, int NV, int U>
+__device__ __forceinline__ void stream_halo(const int32_t* cells, int nh, const int32_t* need_, int n, const TV* x, TV* y) {
+    constexpr int W = 64 * U;
     const __attribute__((address_space(4))) int32_t* need = (const __attribute__((address_space(4))) int32_t*)need_;
-    const int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63, nv = NV * nh;
     int b = 0, have = 0, i[U];
     typename Unset<TV>::U v[U];
     auto ask = [&]() {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int t = min(b + 64 * u + lane, nh5 - 1);
-            i[u] = 5 * cells[t / 5] + t % 5;
+            const int t = min(b + 64 * u + lane, nv - 1);
+            i[u] = t / NV;
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = load_dev(x + i[u]);
+        for (int u = 0; u < U; ++u) i[u] = cells[i[u]];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            i[u] = NV * i[u] + min(b + 64 * u + lane, nv - 1) % NV;
+            v[u] = load_dev(x + i[u]);
+        }
     };
     auto until = [&](int k) {
         while (have < k) {
-            int first = min(b + W, nh5);
+            int first = min(b + W, nv);
 #pragma unroll
             for (int u = U - 1; u >= 0; --u) {
                 const int t = b + 64 * u + lane;
                 const bool ok = v[u] != Unset<TV>::bits;
-                if (ok && t < nh5) y[t] = __builtin_bit_cast(TV, v[u]);
-                const unsigned long long miss = __ballot(!ok && t < nh5);
+                if (ok && t < nv) y[t] = __builtin_bit_cast(TV, v[u]);
+                const unsigned long long miss = __ballot(!ok && t < nv);
                 if (miss) first = b + 64 * u + (int)__builtin_ctzll(miss);
                 if (!ok) v[u] = load_dev(x + i[u]);
             }
             have = first;
-            if (first == b + W && first < nh5) {
+            if (first == b + W && first < nv) {
                 b += W;
                 ask();
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the values in LDS
     };
-    if (nh5 > 0) ask();
+    if (nv > 0) ask();
     barrier_raw();
-    until(need[0]);
+    until(NV * need[0]);
     barrier_raw();
     for (int s = 0; s < n; ++s) {
-        until(need[min(s + 1, n - 1)]);
+        until(NV * need[min(s + 1, n - 1)]);
         barrier_raw();
     }
 }
@@ -474,7 +480,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_sweep(int nT, int* ticket
             if ((threadIdx.x & 63) == 0) next[(round + 1) & 1] = atomicAdd(tickets + BWD, 1);
         } else if (wave > STREAM_WAVES) {
             const int h0 = haloStart[tl];
-            stream_halo(halo + h0, (haloStart[tl + 1] - h0) * 5, need + r0, r1 - r0, (const TV*)out, y + nl5);
+            stream_halo<TV, 5, 4>(halo + h0, haloStart[tl + 1] - h0, need + r0, r1 - r0, (const TV*)out, y + nl5);
         } else {
             if (ticket == 0 && threadIdx.x == 0) tickets[!BWD] = 0;
             gather_tile(rows + rs, nl5, in, y, to, reset);

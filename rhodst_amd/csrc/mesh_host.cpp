@@ -67,11 +67,12 @@ struct PartView {
 };
 
 // The record stream of an ILU(0) apply, in the layout StreamSet describes.
-// split: the two sweeps of a partition are read by separate launches, so the
-// backward records start a ring of their own.  Left empty (kmax = 0) when a row
+// tiles: the set is a TileSet; if it is more than one tile, the two sweeps are
+// read by separate launches, so the backward records start a ring of their own.  Left empty (kmax = 0) when a row
 // has more than kStreamKD off-diagonal blocks in one sweep or the stream passes
 // 64 GiB.
-static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp32, StreamSet& ps) {
+static void build_stream(const Mesh& m, const PartView& pv, bool tiles, bool fp32, StreamSet& ps) {
+    const bool split = tiles && pv.nParts > 1;
     int kmax = 1;
     for (int i = 0; i < m.nC; ++i) {
         int lo = 0, up = 0;
@@ -160,7 +161,7 @@ static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp3
                     ps.hdr.push_back((uint32_t)nr | (uint32_t)(bytes / 16) << 16);
                     ps.recRows.push_back(ps.recRows.back() + nr);
                     ps.recBlk.push_back((int32_t)ps.src.size());
-                    if (split) ps.need.push_back(5 * need);
+                    if (split) ps.need.push_back(need);
                     pos += bytes;
                     r0 = r1;
                 }
@@ -207,14 +208,14 @@ static void build_stream(const Mesh& m, const PartView& pv, bool split, bool fp3
         e[3] = (int32_t)dDst[i];
         for (int k = 0; k < ps.chainK; ++k) {  // unused places read the diagonal
             e[4 + 4 * k] = e[5 + 4 * k] = m.slotDiag[i];
-            e[6 + 4 * k] = i;
+            e[6 + 4 * k] = tiles ? 0 : i;
         }
         for (int s = m.rowPtr[i]; s < m.slotDiag[i]; ++s) {
             if (pv.localCol[s] < 0) continue;
             int32_t* q = e + 4 + 4 * e[1]++;
             q[0] = s;
             q[1] = trans[s];
-            q[2] = m.cols[s];
+            q[2] = tiles ? pv.localCol[s] : m.cols[s];
             q[3] = (int32_t)lDst[s];
         }
     }
@@ -413,7 +414,7 @@ static void build_tiles(const Mesh& m, TileSet& ts) {
     order_partitions(m, tile, nT, ts);
     // columns outside the tile: halo cells, each once per tile and sweep
     ts.haloFStart.assign(1, 0);
-    ts.predStart.assign(1, 0);
+    ts.needF.assign(ts.levPtr.size(), 0);
     ts.haloBStart.assign(1, 0);
     std::vector<int32_t> seen(n, -1), slot(n, 0);
     for (int sweep = 0; sweep < 2; ++sweep) {
@@ -435,15 +436,16 @@ static void build_tiles(const Mesh& m, TileSet& ts) {
                     ts.localCol[s] = slot[j];
                 }
             }
-            if (!sweep) {
-                const size_t p0 = ts.pred.size();
-                for (int q = hs.back(); q < (int)h.size(); ++q) ts.pred.push_back(tile[h[q]]);
-                std::sort(ts.pred.begin() + p0, ts.pred.end());
-                ts.pred.erase(std::unique(ts.pred.begin() + p0, ts.pred.end()), ts.pred.end());
-                ts.predStart.push_back((int32_t)ts.pred.size());
-            }
             hs.push_back((int32_t)h.size());
             ts.maxSlots = std::max(ts.maxSlots, nr + hs[t + 1] - hs[t]);
+            if (sweep) continue;
+            int need = 0;
+            for (int L = ts.levStart[t]; L + 1 < ts.levStart[t + 1]; ++L) {
+                for (int q = ts.levPtr[L]; q < ts.levPtr[L + 1]; ++q)
+                    for (int s = m.rowPtr[ts.rows[q]]; s < m.slotDiag[ts.rows[q]]; ++s)
+                        need = std::max(need, ts.localCol[s] - nr + 1);
+                ts.needF[L] = need;
+            }
         }
     }
 }
@@ -458,8 +460,7 @@ TileSet& mesh_tiles(Mesh& m, bool fp32) {
         ts.d_haloF.upload(ts.haloF);
         ts.d_haloBStart.upload(ts.haloBStart);
         ts.d_haloB.upload(ts.haloB);
-        ts.d_predStart.upload(ts.predStart);
-        ts.d_pred.upload(ts.pred);
+        ts.d_needF.upload(ts.needF);
         ts.d_levStart.upload(ts.levStart);
         ts.d_levPtr.upload(ts.levPtr);
         // the tile's vector and its halo, and where the vector's entries belong, next to the
@@ -469,7 +470,7 @@ TileSet& mesh_tiles(Mesh& m, bool fp32) {
     }
     StreamSet& ps = ts.ps[fp32];
     if (!ps.tried && ts.ok) {
-        build_stream(m, {ts.nParts, ts.rowStart, ts.rows, ts.levStart, ts.levPtr, ts.localCol}, ts.nParts > 1, fp32, ps);
+        build_stream(m, {ts.nParts, ts.rowStart, ts.rows, ts.levStart, ts.levPtr, ts.localCol}, true, fp32, ps);
         ps.upload();
     }
     ps.tried = true;

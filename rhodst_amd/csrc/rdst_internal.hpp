@@ -105,13 +105,13 @@ struct StreamSet {
     std::vector<int32_t> recRows, recBlk;   // [nRec + 1] first row entry, first block
     std::vector<uint16_t> entries;          // [rows][ent / 2]
     std::vector<uint32_t> hdr, start;       // [nRec]; [nRec + 1] first 16-byte unit
-    std::vector<int32_t> need;              // [nRec] halo values (5 x cells) the tile must have before this record (tiles only)
+    std::vector<int32_t> need;              // [nRec] halo cells whose values must be there before this record (tiles only)
     std::vector<int32_t> src, rowCell;      // [blocks] block-CSR slot, or -(cell + 1) for Dinv; the row's cell in a backward record, else -1
     // The factor as a chain of diagonal blocks (no three coupled cells are
     // coupled pairwise): per row, in the partitions' row order, cell, lower
     // blocks, diagonal slot, where Dinv goes in the stream (4-byte units); per
-    // lower block its slot, the transposed coupling's slot, its cell, where L
-    // goes.  chainK: places per row, 0 when the factor has other updates.
+    // lower block its slot, the transposed coupling's slot, its cell (in a tile's
+    // stream the column in the tile), where L goes.  chainK: places per row, 0 when the factor has other updates.
     int chainK = 0;
     std::vector<int32_t> chain;
     DBuf<int32_t> d_chain;
@@ -149,8 +149,8 @@ struct TileSet : PartSet {
     bool tried = false, ok = false;
     int maxSlots = 0;  // most rows + halo cells of a tile
     std::vector<int32_t> haloFStart, haloF, haloBStart, haloB;
-    std::vector<int32_t> predStart, pred;  // the tiles whose factor a tile's needs
-    DBuf<int32_t> d_haloFStart, d_haloF, d_haloBStart, d_haloB, d_predStart, d_pred;
+    std::vector<int32_t> needF;  // beside levPtr: forward halo cells that a level (and those before) reads
+    DBuf<int32_t> d_haloFStart, d_haloF, d_haloBStart, d_haloB, d_needF;
     StreamSet ps[2];   // FP64, FP32
 };
 constexpr int kTileCells = 512;  // most rows of a tile

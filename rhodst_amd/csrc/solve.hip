@@ -46,8 +46,6 @@ struct SolverWork {
     DBuf<float> ty32;
     DBuf<int> tickets;         // of the two sweeps
     DBuf<int> factorState;     // zero-pivot flag and tile ticket of a factor
-    DBuf<int> tileDone;        // factor epoch of each tile
-    int epoch = 0;
     std::vector<double> hscal;
     // BiCGStab
     DBuf<double> p, ph, v, t, th, rw;
@@ -1097,29 +1095,32 @@ void stream_pack(Ctx& k, const StreamSet& ps, const T* LU, const T* Dinv, bool u
                        ps.d_recRows.p, ps.d_recBlk.p, ps.d_src.p, ps.d_rowCell.p, ps.d_start.p, LU, Dinv, st);
 }
 
+// LDS of a tile of the natural-order factor: Dinv of its rows and of its halo
+template <class T>
+size_t chain_lds(const TileSet& ts) { return 25 * sizeof(T) * (size_t)ts.maxSlots; }
+
 // The factor straight into the record stream.  Taken wherever the couplings of
 // the partitions or tiles form no triangle and a row has at most four lower
 // neighbours (structured and box-like meshes; prisms and tetrahedra mostly):
 // the general kernels below, with a copy of A and a full pack, took 5.8 / 9.5 /
 // 0.52 ms (FP32 partitions of 2 M cells, FP64 natural order of 23.5 k and 252
-// cells), this takes 2.2 / 4.5 / 0.20 ms.
+// cells), this takes 2.2 / 2.2 / 0.19 ms.  In natural order a tile's Dinv and its
+// halo's must fit in LDS; where they do not, one launch per level.
 template <class T, int K>
 void chain_launch(Ctx& k, const StreamSet& ps, const T* A, T* Dinv, bool natural, int* fail) {
     Mesh& m = k.m;
     const TileSet& ts = m.tiles;
     uint8_t* st = stream_alloc<T>(k, ps);
-    if (natural && ts.nParts > 1) {
-        if (k.w.tileDone.n != (size_t)ts.nParts) {
-            k.w.tileDone.alloc(ts.nParts);
-            k.w.tileDone.zero(k.s);
-        }
-        hipLaunchKernelGGL((k_ilu_chain_tiles<T, K>), dim3(std::min(ts.nParts, 512)), dim3(CHAIN_THREADS), 0, k.s,
-                           ts.nParts, fail + 1, k.w.tileDone.p, ++k.w.epoch, ts.d_predStart.p, ts.d_pred.p,
-                           ts.d_levStart.p, ts.d_levPtr.p, ps.d_chain.p, A, Dinv, st, fail);
+    if (natural) {
+        const long nd = 25 * (long)m.nC;
+        hipLaunchKernelGGL((k_fill_unset<T>), dim3(std::min(RED_MAXG, blocks_for((int)std::min(nd, 1L << 30), 256))), dim3(256),
+                           0, k.s, nd, Dinv, fail);
+        hipLaunchKernelGGL((k_ilu_chain_tiles<T, K>), dim3(std::min(ts.nParts, 512)), dim3(CHAIN_TILE_THREADS),
+                           chain_lds<T>(ts), k.s, ts.nParts, fail + 1, ts.d_rowStart.p, ts.d_haloFStart.p, ts.d_haloF.p,
+                           ts.d_needF.p, ts.d_levStart.p, ts.d_levPtr.p, ps.d_chain.p, A, Dinv, st, fail);
     } else {
-        hipLaunchKernelGGL((k_ilu_chain<T, K>), dim3(natural ? 1 : m.nParts), dim3(CHAIN_THREADS), 0, k.s,
-                           natural ? ts.d_levStart.p : m.d_partLevStart.p, natural ? ts.d_levPtr.p : m.d_partLevPtr.p,
-                           ps.d_chain.p, A, Dinv, st, fail);
+        hipLaunchKernelGGL((k_ilu_chain<T, K>), dim3(m.nParts), dim3(CHAIN_THREADS), 0, k.s, m.d_partLevStart.p,
+                           m.d_partLevPtr.p, ps.d_chain.p, A, Dinv, st, fail);
     }
     stream_pack<T>(k, ps, A, (const T*)Dinv, true);
 }
@@ -1176,7 +1177,7 @@ void ilu_factor(Ctx& k, const T* A, T* Dinv) {
     RDST_HIP(hipMemsetAsync(fail, 0, 2 * sizeof(int), k.s));
     const bool ilu = k.c.st.precond == RDST_PRECOND_ILU0, natural = k.c.st.ilu_order == RDST_ILU_NATURAL;
     const StreamSet* ps = ilu ? (natural ? &mesh_tiles(m, F).ps[F] : &mesh_stream(m, F)) : nullptr;
-    const bool chain = ps && ps->kmax > 0 && ps->chainK > 0;
+    const bool chain = ps && ps->kmax > 0 && ps->chainK > 0 && (!natural || chain_lds<T>(m.tiles) <= 150 * 1024);
     T* LU = nullptr;
     if (ilu && !chain) {
         // updates beyond the diagonal, or rows too long for the stream: a factor matrix

@@ -32,7 +32,7 @@ static int replay(const Mesh& m, const StreamSet& ps, bool fp32, int q0, int q1,
         if ((int)(ps.hdr[q] & 0xffff) != nr || nr < 1 || nr > kStreamRows) return fail("rows of a record", q, nr);
         if (nr * ps.ent + ((nb * blk + 15) & ~15) > stream_record(fp32)) return fail("record too large", q);
         std::vector<double> nw(nr);
-        if (tiles && (ps.need[q] < need || ps.need[q] > 5 * (slots - own))) return fail("halo count", q, ps.need[q]);
+        if (tiles && (ps.need[q] < need || ps.need[q] > slots - own)) return fail("halo count", q, ps.need[q]);
         if (tiles) need = ps.need[q];
         for (int j = 0; j < nr; ++j) {
             const uint16_t* e = ps.entries.data() + (size_t)(ps.recRows[q] + j) * (ps.ent / 2);
@@ -50,7 +50,7 @@ static int replay(const Mesh& m, const StreamSet& ps, bool fp32, int q0, int q1,
             for (int k = 0; k < cnt; ++k, ++b) {
                 if (b >= ps.recBlk[q + 1]) return fail("block outside its record", q, j);
                 if (e[2 + k] % 5 || e[2 + k] / 5 >= slots) return fail("column out of range", q, e[2 + k]);
-                if (e[2 + k] >= 5 * own && e[2 + k] - 5 * own >= need) return fail("a halo value before it is there", q, j);
+                if (e[2 + k] >= 5 * own && e[2 + k] / 5 - own >= need) return fail("a halo value before it is there", q, j);
                 if (bwd != (ps.rowCell[b] >= 0)) return fail("sweep of a block", q, j);
                 a -= d * coef(ps.src[b]) * y[e[2 + k] / 5];
             }
@@ -77,7 +77,7 @@ static int check(const rdst_mesh_desc* desc, bool fp32, bool natural) {
     std::vector<int32_t> part(m.part);
     if (natural) {
         build_tiles(m, ts);
-        build_stream(m, {ts.nParts, ts.rowStart, ts.rows, ts.levStart, ts.levPtr, ts.localCol}, ts.nParts > 1, fp32, ps);
+        build_stream(m, {ts.nParts, ts.rowStart, ts.rows, ts.levStart, ts.levPtr, ts.localCol}, true, fp32, ps);
         std::fill(part.begin(), part.end(), 0);
     } else {
         build_stream(m, {m.nParts, m.partRowStart, m.partRows, m.partLevStart, m.partLevPtr, m.localCol}, false, fp32, ps);
@@ -131,11 +131,23 @@ static int check(const rdst_mesh_desc* desc, bool fp32, bool natural) {
             for (int s = m.rowPtr[i]; s < m.slotDiag[i]; ++s) {
                 if (part[m.cols[s]] != part[i]) continue;
                 const int32_t* q = e + 4 + 4 * cnt++;
-                if (q[0] != s || rowOf[q[1]] != m.cols[s] || m.cols[q[1]] != i || q[2] != m.cols[s] ||
-                    (uint32_t)q[3] != place[s])
+                if (q[0] != s || rowOf[q[1]] != m.cols[s] || m.cols[q[1]] != i ||
+                    q[2] != (natural ? ts.localCol[s] : m.cols[s]) || (uint32_t)q[3] != place[s])
                     return fail("chain block", i, cnt);
             }
             if (cnt != e[1] || cnt > ps.chainK) return fail("chain count", i, cnt);
+        }
+    }
+    // the halo cells that a tile's levels read are there: all of a level's below its count, in order
+    for (int t = 0; t < nP && natural; ++t) {
+        const int nr = rowStart[t + 1] - rowStart[t], nh = ts.haloFStart[t + 1] - ts.haloFStart[t];
+        int last = 0;
+        for (int L = ts.levStart[t]; L + 1 < ts.levStart[t + 1]; ++L) {
+            if (ts.needF[L] < last || ts.needF[L] > nh) return fail("halo count of a level", t, L);
+            last = ts.needF[L];
+            for (int q = ts.levPtr[L]; q < ts.levPtr[L + 1]; ++q)
+                for (int s = m.rowPtr[rows[q]]; s < m.slotDiag[rows[q]]; ++s)
+                    if (ts.localCol[s] >= nr + last) return fail("a level's halo cell is not there", t, L);
         }
     }
     // a chain must be all of the factor: no lower neighbour shares another neighbour with the row
