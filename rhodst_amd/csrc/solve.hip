@@ -157,21 +157,100 @@ __global__ void k_acc(long n, double* y, const T* a) {
 __global__ void k_add(long n, double* y, const double* a) {
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) y[i] += a[i];
 }
-// fused MGS step: h = reduce(partIn); w -= h Vj; partial dot(w, Vnext) -> partOut; block 0 stores h
+// fused MGS step: h = reduce(partIn); w -= h Vj; partial dot(w, Vnext) -> partOut;
+// block 0 stores h.  Bound by the three vectors (Infinity Cache): four places per
+// thread in flight, loaded before the reduction of the partials (1.6 M entries:
+// 10.5 us; one place at a time and after it 12.6).
 template <class T>
 __global__ __launch_bounds__(RED_BS) void k_mgs_step(long n, T* w, const T* Vj, const T* Vnext, const double* partIn,
                                                       int G, double* partOut, double* hOut) {
+    constexpr int U = 4;
     __shared__ double sh[16];
+    const long st = (long)gridDim.x * blockDim.x;
+    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    T wv[U], vj[U], vn[U];
+    const bool self = Vnext == w;
+    auto load = [&](long b) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const long e = min(b + u * st, n - 1);
+            wv[u] = w[e];
+            vj[u] = Vj[e];
+            vn[u] = self ? T(0) : Vnext[e];
+        }
+    };
+    if (i < n) load(i);
     const double h = reduce_partials(partIn, G, sh);
     if (blockIdx.x == 0 && threadIdx.x == 0) hOut[0] = h;
     double s = 0.0;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        T wi = (T)((double)w[i] - h * (double)Vj[i]);
-        w[i] = wi;
-        s += (double)wi * (double)Vnext[i];
+    while (i < n) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const long e = i + u * st;
+            if (e < n) {
+                const T wi = (T)((double)wv[u] - h * (double)vj[u]);
+                w[e] = wi;
+                s += (double)wi * (double)(self ? wi : vn[u]);
+            }
+        }
+        i += U * st;
+        if (i < n) load(i);
     }
     double t = block_sum(s, sh);
     if (threadIdx.x == 0) partOut[blockIdx.x] = t;
+}
+// All steps of a short vector's orthogonalisation in one workgroup, w in
+// registers: h_j = w . V_j, w -= h_j V_j for j = 0 .. cnt - 1, then the partial sum
+// of |w|^2 (a single one).  A launch per step costs 3.5 us of kernel and a gap for
+// work of 0.1 us; a step here is a reduction over one workgroup (1 260 entries, 20
+// vectors: 840 us by launches, 196 by this).
+constexpr int MGS_BS = 512, MGS_PER = 8;
+template <class T>
+__global__ __launch_bounds__(MGS_BS) void k_mgs_short(int n, long ld, T* w, const T* V, int cnt, double* part, double* H,
+                                                      int m, int col) {
+    __shared__ double sh[2][MGS_BS / 64];
+    const int lane = threadIdx.x & 63, wvf = threadIdx.x >> 6;
+    T wr[MGS_PER], v[MGS_PER], vn[MGS_PER];
+    auto load = [&](const T* p, T (&x)[MGS_PER]) {
+#pragma unroll
+        for (int u = 0; u < MGS_PER; ++u) {
+            const int e = threadIdx.x + u * MGS_BS;
+            x[u] = e < n ? p[e] : T(0);
+        }
+    };
+    auto total = [&](double s, int j) {
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+        if (lane == 0) sh[j & 1][wvf] = s;
+        __syncthreads();
+        double t = 0.0;
+#pragma unroll
+        for (int k = 0; k < MGS_BS / 64; ++k) t += sh[j & 1][k];
+        return t;
+    };
+    load(w, wr);
+    load(V, v);
+    for (int j = 0; j < cnt; ++j) {
+        load(V + (size_t)min(j + 1, cnt - 1) * ld, vn);
+        double s = 0.0;
+#pragma unroll
+        for (int u = 0; u < MGS_PER; ++u) s += (double)wr[u] * (double)v[u];
+        const double h = total(s, j);
+        if (threadIdx.x == 0) H[j * m + col] = h;
+#pragma unroll
+        for (int u = 0; u < MGS_PER; ++u) {
+            wr[u] = (T)((double)wr[u] - h * (double)v[u]);
+            v[u] = vn[u];
+        }
+    }
+    double s = 0.0;
+#pragma unroll
+    for (int u = 0; u < MGS_PER; ++u) {
+        const int e = threadIdx.x + u * MGS_BS;
+        if (e < n) w[e] = wr[u];
+        s += (double)wr[u] * (double)wr[u];
+    }
+    const double t = total(s, cnt);
+    if (threadIdx.x == 0) part[0] = t;
 }
 // x += sum_i yh[i] V_i (V_i at V + i ld), and for EXPAND the sum alone, rounded
 // to the basis' type, added to x (the correction of the mixed form).  The sum of
@@ -372,7 +451,7 @@ __global__ __launch_bounds__(64) void k_sell_spmv(int n, const int64_t* sellPtr,
 template <class T, int NACC>
 __global__ __launch_bounds__(RED_BS) void k_multidot_partial(long n, long ld, const T* w, const T* V, int tot,
                                                              double* part) {
-    __shared__ double sh[16];
+    __shared__ double sh[NACC * RED_BS / 64];
     const int j0 = NACC * (int)blockIdx.y, cnt = min(NACC, tot - j0);
     double acc[NACC];
     for (int q = 0; q < NACC; ++q) acc[q] = 0.0;
@@ -401,12 +480,8 @@ __global__ __launch_bounds__(RED_BS) void k_multidot_partial(long n, long ld, co
         for (int q = 0; q < NACC; ++q)
             if (q < cnt) acc[q] += wi * (double)Vb[(size_t)q * ld + i];
     }
-#pragma unroll
-    for (int q = 0; q < NACC; ++q) {
-        if (q >= cnt) break;
-        const double t = block_sum(acc[q], sh);
-        if (threadIdx.x == 0) part[(size_t)(j0 + q) * gridDim.x + blockIdx.x] = t;
-    }
+    const double t = block_sums<NACC>(acc, sh);
+    if ((int)threadIdx.x < cnt) part[(size_t)(j0 + threadIdx.x) * gridDim.x + blockIdx.x] = t;
 }
 // the same for an FP32 basis (padded with zeros to a multiple of four): each thread
 // reads four consecutive entries per 16-byte load (twice the bytes in flight
@@ -415,7 +490,7 @@ __global__ __launch_bounds__(RED_BS) void k_multidot_partial(long n, long ld, co
 template <int NACC>
 __global__ __launch_bounds__(RED_BS) void k_multidot_partial4(long ld, const float* w, const float* V, int tot,
                                                               double* part) {
-    __shared__ double sh[16];
+    __shared__ double sh[NACC * RED_BS / 64];
     const int j0 = NACC * (int)blockIdx.y, cnt = min(NACC, tot - j0);
     double acc[NACC];
     for (int q = 0; q < NACC; ++q) acc[q] = 0.0;
@@ -451,12 +526,8 @@ __global__ __launch_bounds__(RED_BS) void k_multidot_partial4(long ld, const flo
                           (double)wi.w * (double)v.w;
             }
     }
-#pragma unroll
-    for (int q = 0; q < NACC; ++q) {
-        if (q >= cnt) break;
-        const double t = block_sum(acc[q], sh);
-        if (threadIdx.x == 0) part[(size_t)(j0 + q) * gridDim.x + blockIdx.x] = t;
-    }
+    const double t = block_sums<NACC>(acc, sh);
+    if ((int)threadIdx.x < cnt) part[(size_t)(j0 + threadIdx.x) * gridDim.x + blockIdx.x] = t;
 }
 
 // H[j][col] = sum of the G partials of dot j; block j reduces dot j
@@ -1353,6 +1424,7 @@ void gmres_cycle(Ctx& k, const TM* A, const TM* LU, const TM* Dinv, double* z, c
     hipLaunchKernelGGL((k_gmres_next<TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, ld, V, wv, sc, pin, G, -1, m);
     for (int i = 0; i < m; ++i) {
         TV* Vi = V + (size_t)i * ld;
+        int nPart = G;
         if (k.right) {
             precondition(k, LU, Dinv, Vi, rv, ytmp);
             spmv(k, A, rv, wv);
@@ -1373,6 +1445,10 @@ void gmres_cycle(Ctx& k, const TM* A, const TM* LU, const TM* Dinv, double* z, c
                 hipLaunchKernelGGL(k_cgs_update4, dim3(G), dim3(RED_BS), 0, k.s, n5, ld, wv, V, H, m, i, i + 1, pin);
             else
                 hipLaunchKernelGGL((k_cgs_update<TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, wv, V, H, m, i, i + 1, pin);
+        } else if (n5 <= MGS_BS * MGS_PER) {
+            // one workgroup does a short vector (beyond it a step by the whole chip costs no more)
+            nPart = 1;
+            hipLaunchKernelGGL((k_mgs_short<TV>), dim3(1), dim3(MGS_BS), 0, k.s, (int)n5, ld, wv, V, i + 1, pin, H, m, i);
         } else {
             // partial dot(w, V0), then the fused MGS steps
             hipLaunchKernelGGL((k_dot_partial<TV, TV>), dim3(G), dim3(RED_BS), 0, k.s, n5, wv, V, pin);
@@ -1386,7 +1462,7 @@ void gmres_cycle(Ctx& k, const TM* A, const TM* LU, const TM* Dinv, double* z, c
         }
         // pin holds partials of |w|^2: the next V, the rotations
         hipLaunchKernelGGL((k_gmres_next<TV>), dim3(i + 1 < m ? G : 1), dim3(RED_BS), 0, k.s, n5, ld,
-                           i + 1 < m ? V + (size_t)(i + 1) * ld : (TV*)nullptr, (const TV*)wv, sc, pin, G, i, m);
+                           i + 1 < m ? V + (size_t)(i + 1) * ld : (TV*)nullptr, (const TV*)wv, sc, pin, nPart, i, m);
     }
     hipLaunchKernelGGL(k_gmres_backsub, dim3(1), dim3(256), m <= GMRES_TRI ? sizeof(double) * (m * m + m) : 0, k.s, sc, m);
     if (k.right) {
