@@ -325,9 +325,16 @@ static void order_partitions(const Mesh& m, const std::vector<int32_t>& part, in
         ps.maxLevels = std::max(ps.maxLevels, nl);
     }
     ps.localCol.assign(m.nnzb, -1);
-    for (int c = 0; c < n; ++c)
+    ps.maxOff = 0;
+    for (int c = 0; c < n; ++c) {
+        int off = -1;
         for (int s = m.rowPtr[c]; s < m.rowPtr[c + 1]; ++s)
-            if (part[m.cols[s]] == part[c]) ps.localCol[s] = local[m.cols[s]];
+            if (part[m.cols[s]] == part[c]) {
+                ps.localCol[s] = local[m.cols[s]];
+                ++off;
+            }
+        ps.maxOff = std::max(ps.maxOff, off);
+    }
 }
 
 // Tiles of the natural-order ILU(0).  Every lower neighbour of a row gets a

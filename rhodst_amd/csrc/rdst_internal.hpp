@@ -135,6 +135,7 @@ constexpr int kIluSegRows = 64;
 
 struct PartSet {
     int nParts = 0, maxRows = 0, maxLevels = 0;
+    int maxOff = 0;  // most off-diagonal columns of a row inside its partition
     std::vector<int32_t> rowStart, rows, levStart, levPtr, localCol;
     DBuf<int32_t> d_rowStart, d_rows, d_levStart, d_levPtr, d_localCol;
 };
