@@ -791,19 +791,22 @@ __global__ void k_av_obj_gather(MeshDev m, const int32_t* color, int pass0, cons
     g[5 * (size_t)j + comp] = s;
 }
 
-// J^T on the second-neighbour pattern: block e of J, transposed, at wideT[e]
+// J^T on the second-neighbour pattern: block e of J, transposed, at wideT[e].
+// A thread per entry, so a wavefront's stores are runs of 25 (a thread per block
+// took 370 us on the 50 k-cell airfoil, this 48; the block-CSR part 153 and 25).
 __global__ void k_wide_transpose(long nnz, const int32_t* wideT, const double* J, double* JT) {
-    for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < nnz; e += (long)gridDim.x * blockDim.x) {
-        const double* a = J + 25 * (size_t)e;
-        double* t = JT + 25 * (size_t)wideT[e];
-        for (int r = 0; r < 5; ++r)
-            for (int q = 0; q < 5; ++q) t[5 * r + q] = a[5 * q + r];
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < 25 * nnz; i += (long)gridDim.x * blockDim.x) {
+        const long e = i / 25;
+        const int q = (int)(i - 25 * e);
+        JT[25 * (size_t)wideT[e] + q] = J[25 * (size_t)e + 5 * (q % 5) + q / 5];
     }
 }
 // the block-CSR slots of a second-neighbour matrix
 __global__ void k_wide_to_slots(long nnzb, const int32_t* wideOfSlot, const double* W, double* A) {
-    for (long s = (long)blockIdx.x * blockDim.x + threadIdx.x; s < nnzb; s += (long)gridDim.x * blockDim.x)
-        for (int q = 0; q < 25; ++q) A[25 * (size_t)s + q] = W[25 * (size_t)wideOfSlot[s] + q];
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < 25 * nnzb; i += (long)gridDim.x * blockDim.x) {
+        const long s = i / 25;
+        A[i] = W[25 * (size_t)wideOfSlot[s] + (i - 25 * s)];
+    }
 }
 
 Bounds bounds_of(const Case& c) {
@@ -978,11 +981,11 @@ void viscous_linearise(Case& c) {
     AvOut out;
     out.Jw = c.adjW.p;
     av_batches(m, [&](int p0, int np) { av_pass(c, p0, np, out); });
-    const int gb = std::min(4096, blocks_for((long)nnz, 256));
+    const int gb = std::min(16384, blocks_for((long)nnz, 10));
     hipLaunchKernelGGL(k_wide_transpose, dim3(gb), dim3(256), 0, c.stream, (long)nnz, m.d_wideT.p, c.adjW.p, c.adjWT.p);
     const size_t nn = 25 * (size_t)m.nnzb;
     if (c.adjJT.n != nn) c.adjJT.alloc(nn);
-    hipLaunchKernelGGL(k_wide_to_slots, dim3(std::min(4096, blocks_for((long)m.nnzb, 256))), dim3(256), 0, c.stream,
+    hipLaunchKernelGGL(k_wide_to_slots, dim3(std::min(16384, blocks_for((long)m.nnzb, 10))), dim3(256), 0, c.stream,
                        (long)m.nnzb, m.d_wideOfSlot.p, c.adjWT.p, c.adjJT.p);
     RDST_HIP(hipGetLastError());
     RDST_HIP(hipStreamSynchronize(c.stream));
