@@ -1,0 +1,37 @@
+"""The GMRES orthogonalisations around the length up to which one workgroup
+does a vector (4096 entries), against a sparse direct solve."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+import scipy.sparse.linalg as spla
+
+from rhodst_amd import _capi, cases, meshgen
+from rhodst_amd._abi import make_bcs, make_settings, make_thermo
+
+pytestmark = pytest.mark.gpu
+
+
+# 520, 4095 and 4100 unknowns, and two blocks of a long vector's grid stride
+@pytest.mark.parametrize("nx,ny", [(13, 8), (9, 91), (10, 82), (300, 180)])
+@pytest.mark.parametrize("gs", ["modified", "classical"])
+def test_gmres_solves(nx, ny, gs):
+    mesh = meshgen.box_2d(nx, ny, jitter=0.2)
+    n, nI = mesh.n_cells, len(mesh.neighbour)
+    rng = np.random.default_rng(nx)
+    upper, lower = rng.uniform(-0.5, 0.5, (2, nI, 5, 5))
+    own, nei = np.asarray(mesh.owner[:nI]), np.asarray(mesh.neighbour)
+    diag = rng.uniform(-0.5, 0.5, (n, 5, 5)) + 8.0 * np.eye(5)
+    b = rng.standard_normal((n, 5))
+    kw = dict(n_directions=6, max_iter=8, min_iter=1, tolerance=1e-14, rel_tol=0.0, gram_schmidt=gs)
+    patches = {p[0]: {"p": "zeroGradient", "T": "zeroGradient", "U": "zeroGradient"} for p in mesh.patches if p[1] != 3}
+    spec = cases.CaseSpec("krylov", mesh, make_thermo(), make_bcs(mesh, patches), make_settings(**kw),
+                          np.ones(n), np.ones(n), np.zeros((n, 3)))
+    x, _ = _capi.DeviceCase(spec, _capi.DeviceMesh(mesh)).ldu_solve(diag, upper, lower, b, np.zeros((n, 5)))
+    i = np.concatenate([np.arange(n), own, nei])
+    j = np.concatenate([np.arange(n), nei, own])
+    order = np.lexsort((j, i))
+    A = sp.bsr_matrix((np.concatenate([diag, upper, lower])[order], j[order],
+                       np.concatenate([[0], np.cumsum(np.bincount(i, minlength=n))])), shape=(5 * n, 5 * n))
+    ref = spla.spsolve(A.tocsc(), b.ravel())
+    # residual reduced to 1e-14 of the right-hand side's, condition number below 10
+    assert np.abs(x.ravel() - ref).max() <= 1e-12 * np.abs(ref).max()
