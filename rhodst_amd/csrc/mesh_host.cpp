@@ -237,6 +237,7 @@ void StreamSet::upload() {
 }
 
 StreamSet& mesh_stream(Mesh& m, bool fp32) {
+    std::lock_guard<std::mutex> lock(m.planMutex);
     StreamSet& ps = m.ps[fp32];
     if (!ps.tried) {
         build_stream(m, {m.nParts, m.partRowStart, m.partRows, m.partLevStart, m.partLevPtr, m.localCol}, false, fp32, ps);
@@ -458,6 +459,7 @@ static void build_tiles(const Mesh& m, TileSet& ts) {
 }
 
 TileSet& mesh_tiles(Mesh& m, bool fp32) {
+    std::lock_guard<std::mutex> lock(m.planMutex);
     TileSet& ts = m.tiles;
     if (!ts.tried) {
         build_tiles(m, ts);

@@ -4,6 +4,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <mutex>
 
 #include <cstdint>
 #include <string>
@@ -198,6 +199,7 @@ struct Mesh {
     PartSet sa;
     // the record streams of the partitioned ILU(0) apply, FP64 and FP32 (made
     // by the first case that uses one)
+    std::mutex planMutex;  // of ps, tiles: built on first use
     StreamSet ps[2];
     TileSet tiles;  // of the natural-order ILU(0), made by the first case that uses it
     // sliced-ELL copy of the block-CSR pattern for the SpMV: slices of 64
@@ -248,7 +250,8 @@ constexpr int kMaxPartLevels = 32;
 void mesh_build(Mesh& m, const rdst_mesh_desc* d, const rdst_mesh_geometry* g = nullptr);
 void build_partitions(Mesh& m, int maxCells);
 void mesh_upload(Mesh& m);
-StreamSet& mesh_stream(Mesh& m, bool fp32);  // the record stream, built and uploaded on first use
+// the record stream, built and uploaded on first use (by one of the threads that share the mesh)
+StreamSet& mesh_stream(Mesh& m, bool fp32);
 TileSet& mesh_tiles(Mesh& m, bool fp32);     // the tiles and their record stream, likewise
 
 // ---------------------------------------------------------------------------
