@@ -12,7 +12,7 @@
 // level's blocks of A are loaded while this one is computed, and L and Dinv go
 // straight into the sweeps' record stream: no copy of A, no factor matrix.
 // Measured, this kernel with its pack against thread per row, copy and pack:
-// FP32 partitions 2 M cells 2.16 / 5.8 ms, 24 k cells 0.25 / 0.52 ms; FP64 natural
+// FP32 partitions 2 M cells 1.80 / 5.8 ms, 24 k cells 0.25 / 0.52 ms; FP64 natural
 // order 252 cells 0.19 / 0.52 ms, 23.5 k 2.2 / 9.5 ms, 321 k 2.1 / 9.9 ms.
 #pragma once
 #include "rdst_internal.hpp"

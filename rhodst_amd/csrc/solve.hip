@@ -5,12 +5,12 @@
 //
 // Matrix: owner/neighbour-sorted block-CSR of 5x5 row-major blocks.
 // Preconditioner: block ILU(0) in the natural cell order, computed and
-// applied level by level (rows of one level are independent), which gives
+// applied by tiles of levels (rows of one level are independent), which gives
 // the same factors as a sequential natural-order ILU(0) -- ILU(0) factors
-// are unique for a given ordering and sparsity.
+// are unique for a given ordering and sparsity (ilu_factor.hpp, ilu_stream.hpp).
 // GMRES: restarted, left-preconditioned, modified Gram-Schmidt; each MGS
 // step is one fused kernel (w -= h_j V_j and the partial dot with the next
-// vector), reductions are deterministic two-level (wavefront shuffles, then
+// vector; all of them in one for short vectors), reductions are deterministic two-level (wavefront shuffles, then
 // every block re-reduces the previous kernel's block partials in the same
 // order), and the Hessenberg/Givens/back-substitution run on the device in
 // FP64, so a restart cycle needs no host round trip.
@@ -1175,7 +1175,7 @@ size_t chain_lds(const TileSet& ts) { return 25 * sizeof(T) * (size_t)ts.maxSlot
 // neighbours (structured and box-like meshes; prisms and tetrahedra mostly):
 // the general kernels below, with a copy of A and a full pack, took 5.8 / 9.5 /
 // 0.52 ms (FP32 partitions of 2 M cells, FP64 natural order of 23.5 k and 252
-// cells), this takes 2.2 / 2.2 / 0.19 ms.  In natural order a tile's Dinv and its
+// cells), this takes 1.8 / 2.2 / 0.19 ms.  In natural order a tile's Dinv and its
 // halo's must fit in LDS; where they do not, one launch per level.
 template <class T, int K>
 void chain_launch(Ctx& k, const StreamSet& ps, const T* A, T* Dinv, bool natural, int* fail) {
