@@ -793,7 +793,7 @@ __global__ void k_av_obj_gather(MeshDev m, const int32_t* color, int pass0, cons
 
 // J^T on the second-neighbour pattern: block e of J, transposed, at wideT[e].
 // A thread per entry, so a wavefront's stores are runs of 25 (a thread per block
-// took 370 us on the 50 k-cell airfoil, this 48; the block-CSR part 153 and 25).
+// took 370 us on the 58 k-cell airfoil, this 48; the block-CSR part 153 and 25).
 __global__ void k_wide_transpose(long nnz, const int32_t* wideT, const double* J, double* JT) {
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < 25 * nnz; i += (long)gridDim.x * blockDim.x) {
         const long e = i / 25;

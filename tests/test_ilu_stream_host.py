@@ -16,7 +16,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def replay_lib(tmp_path_factory):
     so = str(tmp_path_factory.mktemp("host") / "ilu_stream_check.so")
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I", f"{rocm}/include",
@@ -67,10 +67,10 @@ MESHES = {
 
 
 @pytest.mark.parametrize("name", sorted(MESHES))
-def test_streams_and_tiles(checker, name):
+def test_streams_and_tiles(replay_lib, name):
     md = MeshDesc(MESHES[name]())
     what = C.create_string_buffer(256)
     for fp32 in (0, 1):
         for natural in (0, 1):
-            rc = checker.ilu_stream_check(C.byref(md.desc), fp32, natural, what, 256)
+            rc = replay_lib.ilu_stream_check(C.byref(md.desc), fp32, natural, what, 256)
             assert rc == 0, (name, fp32, natural, what.value.decode())
