@@ -24,10 +24,12 @@ namespace rdst {
 
 constexpr int STREAM_WAVES = 4;                          // compute wavefronts, 12 rows of 5 lanes each
 constexpr int STREAM_THREADS = 64 * (STREAM_WAVES + 1);  // + the loader
-// 16 bytes per lane straight into LDS (lane l lands at l16 past the wavefront's base)
+// 16 bytes per lane straight into LDS (lane l lands at l16 past the wavefront's base);
+// NT: non-temporal, for a stream that no cache holds until the next apply
+template <bool NT>
 __device__ __forceinline__ void lds_dma16(const uint8_t* g, uint8_t* l) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
-                                     (__attribute__((address_space(3))) void*)l, 16, 0, 0);
+                                     (__attribute__((address_space(3))) void*)l, 16, 0, NT ? 2 : 0);
 }
 template <int N>
 __device__ __forceinline__ void wait_vm() {
@@ -65,7 +67,7 @@ __device__ __forceinline__ void barrier_lds() {
 // Between the last two the compute wavefronts read the row entries of record
 // s + 2 and the values of record s + 1 from the ring, so everything before
 // record s + 1 may be overwritten.
-template <int RING>
+template <int RING, bool NT>
 __device__ __forceinline__ void stream_load(const uint8_t* stream, const uint32_t* start_, int r0, int r1, uint8_t* ring) {
     // scalar loads: the offsets must not wait behind the block loads
     const __attribute__((address_space(4))) uint32_t* start = (const __attribute__((address_space(4))) uint32_t*)start_;
@@ -76,7 +78,7 @@ __device__ __forceinline__ void stream_load(const uint8_t* stream, const uint32_
     const uint8_t* g = stream + 16 * (size_t)base + 16 * lane;
     int issued = 0;
     auto issue = [&](int limit) {
-        for (; issued < limit; ++issued) lds_dma16(g + (size_t)issued * 1024, ring + (issued & (RC - 1)) * 1024);
+        for (; issued < limit; ++issued) lds_dma16<NT>(g + (size_t)issued * 1024, ring + (issued & (RC - 1)) * 1024);
     };
     // 1 KB pieces that hold everything before the record starting at st
     auto pieces = [&](uint32_t st) { return (int)((st - base + 63) / 64); };
@@ -314,7 +316,7 @@ __device__ __forceinline__ void scatter_rows(const int32_t* rows, int nl5, const
 }
 
 // x = M^-1 r for the partitioned factor, one workgroup per partition
-template <class TM, class TV, int KDU>
+template <class TM, class TV, int KDU, bool NT>
 __global__ __launch_bounds__(STREAM_THREADS) void k_stream_apply(const int32_t* __restrict__ rowStart,
                                                                  const int32_t* __restrict__ rows,
                                                                  const int32_t* __restrict__ recBeg,
@@ -330,7 +332,7 @@ __global__ __launch_bounds__(STREAM_THREADS) void k_stream_apply(const int32_t* 
     const int pt = blockIdx.x;
     const int r0 = recBeg[pt], rm = recMid[pt], r1 = recBeg[pt + 1];
     if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == STREAM_WAVES) {
-        stream_load<RING>(stream, start, r0, r1, ring);
+        stream_load<RING, NT>(stream, start, r0, r1, ring);
         return;
     }
     const int rs = rowStart[pt], nl5 = (rowStart[pt + 1] - rs) * 5;
@@ -476,7 +478,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_sweep(int nT, int* ticket
         const int r0 = BWD ? recMid[tl] : recBeg[tl], r1 = BWD ? recBeg[tl + 1] : recMid[tl];
         const int rs = rowStart[tl], nl5 = (rowStart[tl + 1] - rs) * 5;
         if (wave == STREAM_WAVES) {
-            stream_load<RING>(stream, start, r0, r1, ring);
+            stream_load<RING, false>(stream, start, r0, r1, ring);
             if ((threadIdx.x & 63) == 0) next[(round + 1) & 1] = atomicAdd(tickets + BWD, 1);
         } else if (wave > STREAM_WAVES) {
             const int h0 = haloStart[tl];

@@ -403,6 +403,14 @@ __global__ __launch_bounds__(256) void k_bspmv(int n, const int32_t* rowPtr, con
     for (int r = 0; r < 5; ++r) y[5 * (size_t)i + r] = (TY)acc[r];
 }
 
+// Whether a matrix or stream read once per Krylov vector is loaded non-temporally:
+// when the two together pass the 256 MB of Infinity Cache, nothing keeps them until
+// the next vector, and they only push out the basis, which the Gram-Schmidt
+// kernels read again.  Steps with and without: wing 2.03 M cells 33.4 / 34.6 ms,
+// 403 k FP64 14.97 / 15.35, Newton 321 k 6.90 / 7.18; below the line it costs: airfoil
+// 205 k (100 MB each) 4.367 / 4.351, 4 032 cells 1.48 / 1.46.
+static bool past_cache(size_t bytes) { return bytes > (size_t)128 << 20; }
+
 // ---------------------------------------------------------------- sliced-ELL SpMV
 // block-CSR -> sliced ELL (64 rows per slice, entry-major inside a block column)
 template <class T>
@@ -415,7 +423,7 @@ __global__ void k_to_sell(long nnzb, const int64_t* sellOfSlot, const T* A, T* S
 }
 // one 64-lane wavefront per slice, lane = row: every value load is 64
 // consecutive entries (fully coalesced), x is gathered per block column
-template <class TA, class TX, class TY>
+template <class TA, class TX, class TY, bool NT>
 __global__ __launch_bounds__(64) void k_sell_spmv(int n, const int64_t* sellPtr, const int32_t* sellWidth,
                                                   const int32_t* sellCol, const TA* S, const TX* x, TY* y) {
     const int sl = blockIdx.x;
@@ -430,11 +438,12 @@ __global__ __launch_bounds__(64) void k_sell_spmv(int n, const int64_t* sellPtr,
         const TX* xv = x + 5 * (size_t)col;
         const double x0 = xv[0], x1 = xv[1], x2 = xv[2], x3 = xv[3], x4 = xv[4];
         const TA* v = S + 25 * blk + lane;
-        a0 += (double)v[0] * x0 + (double)v[64] * x1 + (double)v[128] * x2 + (double)v[192] * x3 + (double)v[256] * x4;
-        a1 += (double)v[320] * x0 + (double)v[384] * x1 + (double)v[448] * x2 + (double)v[512] * x3 + (double)v[576] * x4;
-        a2 += (double)v[640] * x0 + (double)v[704] * x1 + (double)v[768] * x2 + (double)v[832] * x3 + (double)v[896] * x4;
-        a3 += (double)v[960] * x0 + (double)v[1024] * x1 + (double)v[1088] * x2 + (double)v[1152] * x3 + (double)v[1216] * x4;
-        a4 += (double)v[1280] * x0 + (double)v[1344] * x1 + (double)v[1408] * x2 + (double)v[1472] * x3 + (double)v[1536] * x4;
+        auto ld = [&](int q) { return (double)(NT ? __builtin_nontemporal_load(v + q) : v[q]); };
+        a0 += ld(0) * x0 + ld(64) * x1 + ld(128) * x2 + ld(192) * x3 + ld(256) * x4;
+        a1 += ld(320) * x0 + ld(384) * x1 + ld(448) * x2 + ld(512) * x3 + ld(576) * x4;
+        a2 += ld(640) * x0 + ld(704) * x1 + ld(768) * x2 + ld(832) * x3 + ld(896) * x4;
+        a3 += ld(960) * x0 + ld(1024) * x1 + ld(1088) * x2 + ld(1152) * x3 + ld(1216) * x4;
+        a4 += ld(1280) * x0 + ld(1344) * x1 + ld(1408) * x2 + ld(1472) * x3 + ld(1536) * x4;
     }
     if (row < n) {
         TY* yr = y + 5 * (size_t)row;
@@ -1125,7 +1134,9 @@ void spmv(Ctx& k, const TA* A, const TX* x, TY* y) {
     if ((const void*)A == (const void*)k.c.A64.p) S = (const TA*)k.c.S64.p;
     if ((const void*)A == (const void*)k.c.A32.p) S = (const TA*)k.c.S32.p;
     if (S) {
-        hipLaunchKernelGGL((k_sell_spmv<TA, TX, TY>), dim3(k.m.nSlices), dim3(64), 0, k.s, k.m.nC, k.m.d_sellPtr.p,
+        auto* kernel = past_cache(25 * sizeof(TA) * (size_t)k.m.sellBlocks) ? k_sell_spmv<TA, TX, TY, true>
+                                                                         : k_sell_spmv<TA, TX, TY, false>;
+        hipLaunchKernelGGL(kernel, dim3(k.m.nSlices), dim3(64), 0, k.s, k.m.nC, k.m.d_sellPtr.p,
                            k.m.d_sellWidth.p, k.m.d_sellCol.p, S, x, y);
         return;
     }
@@ -1208,7 +1219,8 @@ void stream_launch(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV*
     // lanes read KDU + 1 blocks from wherever their row starts: room for them past a short partition's vector
     const size_t shmem = stream_ring(sizeof(TM) == 4) + std::max(sizeof(TV) * 5 * (size_t)slots, sizeof(TM) * 25 * (KDU + 1));
     if (!natural || ts.nParts == 1) {
-        hipLaunchKernelGGL((k_stream_apply<TM, TV, KDU>), dim3(natural ? 1 : m.nParts), dim3(STREAM_THREADS), shmem, k.s,
+        auto* kernel = past_cache(ps.bytes()) ? k_stream_apply<TM, TV, KDU, true> : k_stream_apply<TM, TV, KDU, false>;
+        hipLaunchKernelGGL(kernel, dim3(natural ? 1 : m.nParts), dim3(STREAM_THREADS), shmem, k.s,
                            natural ? ts.d_rowStart.p : m.d_partRowStart.p, natural ? ts.d_rows.p : m.d_partRows.p,
                            ps.d_recBeg.p, ps.d_recMid.p, ps.d_hdr.p, ps.d_start.p, stream, r, x);
         return;
