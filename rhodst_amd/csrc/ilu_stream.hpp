@@ -494,9 +494,10 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_sweep(int nT, int* ticket
 // the row entries of every record into the stream (once per buffer)
 __global__ __launch_bounds__(64) void k_stream_entries(int ent, const int32_t* recRows, const uint4* entries,
                                                        const uint32_t* start, uint8_t* stream) {
-    const int q = blockIdx.x, b = recRows[q] * ent / 16, e = recRows[q + 1] * ent / 16;
+    const int q = blockIdx.x;
+    const size_t b = entry_unit(recRows[q], ent), e = entry_unit(recRows[q + 1], ent);
     uint4* o = reinterpret_cast<uint4*>(stream + 16 * (size_t)start[q]);
-    for (int t = b + (int)threadIdx.x; t < e; t += 64) o[t - b] = entries[t];
+    for (size_t t = b + threadIdx.x; t < e; t += 64) o[t - b] = entries[t];
 }
 
 // Scatter the factor into the stream, one wavefront per record and one thread

@@ -97,6 +97,9 @@ constexpr int stream_ring(bool fp32) { return fp32 ? 32768 : 65536; }
 // most bytes of a record: the ring holds three and their padding
 constexpr int stream_record(bool fp32) { return stream_ring(fp32) / 64 * 19; }
 constexpr int stream_entry(int kmax) { return kmax <= 4 ? 16 : 32; }
+// the 16-byte unit at which row entry `row` starts; a stream has two entries per
+// cell, whose bytes pass 32 bits from 3.4e7 cells on
+constexpr size_t entry_unit(int row, int ent) { return (size_t)row * (ent / 16); }
 struct StreamSet {
     bool tried = false;               // built, or found not to fit
     int kmax = 0;                     // most off-diagonal blocks of a row (0: not built)

@@ -74,3 +74,12 @@ def test_streams_and_tiles(replay_lib, name):
         for natural in (0, 1):
             rc = replay_lib.ilu_stream_check(C.byref(md.desc), fp32, natural, what, 256)
             assert rc == 0, (name, fp32, natural, what.value.decode())
+
+
+@pytest.mark.parametrize("cells", [1, 33_554_431, 33_554_432, 67_108_864, 120_000_000])
+@pytest.mark.parametrize("ent", [16, 32])
+def test_row_entries_of_large_meshes(replay_lib, cells, ent):
+    # the last of two entries per cell, at the sizes where its byte offset passes 31 and 32 bits
+    replay_lib.ilu_entry_unit.restype = C.c_longlong
+    row = 2 * cells - 1
+    assert 16 * replay_lib.ilu_entry_unit(row, ent) == row * ent
