@@ -373,19 +373,20 @@ __device__ __forceinline__ void stream_halo(const int32_t* cells, int nh, const 
     constexpr int W = 64 * U;
     const __attribute__((address_space(4))) int32_t* need = (const __attribute__((address_space(4))) int32_t*)need_;
     const int lane = threadIdx.x & 63, nv = NV * nh;
-    int b = 0, have = 0, i[U];
+    int b = 0, have = 0;
+    uint32_t i[U];
     typename Unset<TV>::U v[U];
     auto ask = [&]() {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int t = min(b + 64 * u + lane, nv - 1);
-            i[u] = t / NV;
+            i[u] = (uint32_t)(t / NV);
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) i[u] = cells[i[u]];
+        for (int u = 0; u < U; ++u) i[u] = (uint32_t)cells[i[u]];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            i[u] = NV * i[u] + min(b + 64 * u + lane, nv - 1) % NV;
+            i[u] = cell_value((int)i[u], NV, min(b + 64 * u + lane, nv - 1) % NV);
             v[u] = load_dev(x + i[u]);
         }
     };

@@ -97,8 +97,11 @@ constexpr int stream_ring(bool fp32) { return fp32 ? 32768 : 65536; }
 // most bytes of a record: the ring holds three and their padding
 constexpr int stream_record(bool fp32) { return stream_ring(fp32) / 64 * 19; }
 constexpr int stream_entry(int kmax) { return kmax <= 4 ? 16 : 32; }
+// value q of cell's nv in a vector with nv values per cell: the 25 of an inverse
+// pass 31 bits from 8.6e7 cells on
+constexpr uint32_t cell_value(int cell, int nv, int q) { return (uint32_t)cell * (uint32_t)nv + (uint32_t)q; }
 // the 16-byte unit at which row entry `row` starts; a stream has two entries per
-// cell, whose bytes pass 32 bits from 3.4e7 cells on
+// cell, whose bytes pass 31 bits from 3.4e7 cells on
 constexpr size_t entry_unit(int row, int ent) { return (size_t)row * (ent / 16); }
 struct StreamSet {
     bool tried = false;               // built, or found not to fit

@@ -210,6 +210,8 @@ static int check(const rdst_mesh_desc* desc, bool fp32, bool natural) {
 
 extern "C" long long ilu_entry_unit(int row, int ent) { return (long long)entry_unit(row, ent); }
 
+extern "C" long long ilu_cell_value(int cell, int nv, int q) { return (long long)cell_value(cell, nv, q); }
+
 extern "C" int ilu_stream_check(const rdst_mesh_desc* desc, int fp32, int natural, char* what, int len) {
     g_what.clear();
     int rc = 2;

@@ -83,3 +83,11 @@ def test_row_entries_of_large_meshes(replay_lib, cells, ent):
     replay_lib.ilu_entry_unit.restype = C.c_longlong
     row = 2 * cells - 1
     assert 16 * replay_lib.ilu_entry_unit(row, ent) == row * ent
+
+
+@pytest.mark.parametrize("cells", [1, 85_899_345, 85_899_346, 140_000_000])
+@pytest.mark.parametrize("nv", [5, 25])
+def test_halo_values_of_large_meshes(replay_lib, cells, nv):
+    # the last value of the last cell, at the sizes where 25 per cell pass 31 bits
+    replay_lib.ilu_cell_value.restype = C.c_longlong
+    assert replay_lib.ilu_cell_value(cells - 1, nv, nv - 1) == nv * cells - 1
