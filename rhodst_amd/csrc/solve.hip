@@ -1488,8 +1488,9 @@ void gmres_cycle(Ctx& k, const TM* A, const TM* LU, const TM* Dinv, double* z, c
     }
 }
 
-// norm factor, b - A x and its normalised magnitude.  fromZero: x is zero, so
-// A x, xRef and A xRef are, and the three products are left out
+// norm factor, b - A x and its normalised magnitude.  fromZero: x is zero, so of
+// a finite matrix A x, xRef and A xRef are, and the three products are left out;
+// what that says of the matrix is checked by residual_of_zero
 template <class TA>
 void initial_residual(Ctx& k, const TA* A, const double* x, const double* b, bool fromZero, rdst_solver_perf& perf) {
     SolverWork& w = k.w;
@@ -1511,20 +1512,49 @@ void initial_residual(Ctx& k, const TA* A, const double* x, const double* b, boo
     for (int q = 0; q < 5; ++q) perf.final_residual[q] = perf.initial_residual[q];
 }
 
+// b - A x and its magnitude after a cycle
+template <class TA>
+void cycle_residual(Ctx& k, const TA* A, const double* x, const double* b, rdst_solver_perf& perf) {
+    SolverWork& w = k.w;
+    spmv(k, A, x, w.wA.p);
+    hipLaunchKernelGGL(k_sub, dim3(k.G), dim3(RED_BS), 0, k.s, (long)w.n5, w.r.p, b, w.wA.p);
+    cmptmag(k, w.r.p, w.scal.p + S_FIN, w.scal.p + S_NORM);
+    read_scalars(k, S_FIN, 5, perf.final_residual);
+}
+
+bool finite5(const double* v) {
+    for (int q = 0; q < 5; ++q)
+        if (!std::isfinite(v[q])) return false;
+    return true;
+}
+
+// A zero x times an infinity or a NaN of the matrix is no zero: the norm factor
+// and with it every residual of such a system is NaN.  A solve from zero that
+// left the products out (initial_residual) takes them here, with a zero vector,
+// when it would end at once, or when its first cycle left a residual that is not
+// finite, which a matrix that is not finite always does.
+template <class TA>
+void residual_of_zero(Ctx& k, const TA* A, const double* b, rdst_solver_perf& perf) {
+    SolverWork& w = k.w;
+    RDST_HIP(hipMemsetAsync(w.x0.p, 0, sizeof(double) * w.n5, k.s));
+    initial_residual(k, A, w.x0.p, b, false, perf);
+}
+
 rdst_solver_perf gmres_fp64(Ctx& k, const double* A, double* x, const double* b, bool fromZero) {
     SolverWork& w = k.w;
-    const long n5 = w.n5;
     rdst_solver_perf perf{};
     initial_residual(k, A, x, b, fromZero, perf);
+    if (fromZero && converged(k.c.st, perf)) residual_of_zero(k, A, b, perf);
     if (converged(k.c.st, perf)) return perf;
     const double* r = fromZero ? b : w.r.p;
     do {
         gmres_cycle<double, double>(k, A, w.LU.p, w.Dinv.p, x, r, w.wA.p, w.tmp.p, w.V.p, w.x0.p);
-        spmv(k, A, x, w.wA.p);
-        hipLaunchKernelGGL(k_sub, dim3(k.G), dim3(RED_BS), 0, k.s, n5, w.r.p, b, w.wA.p);
+        cycle_residual(k, A, x, b, perf);
+        if (fromZero && perf.n_iterations == 0 && !finite5(perf.final_residual)) {
+            residual_of_zero(k, A, b, perf);
+            cycle_residual(k, A, x, b, perf);
+        }
         r = w.r.p;
-        cmptmag(k, w.r.p, w.scal.p + S_FIN, w.scal.p + S_NORM);
-        read_scalars(k, S_FIN, 5, perf.final_residual);
         perf.n_iterations++;
     } while (!converged(k.c.st, perf));
     return perf;
@@ -1539,16 +1569,18 @@ rdst_solver_perf gmres_mixed(Ctx& k, const TO* Aout, const float* A, double* x, 
     const long n5 = w.n5;
     rdst_solver_perf perf{};
     initial_residual(k, Aout, x, b, fromZero, perf);
+    if (fromZero && converged(k.c.st, perf)) residual_of_zero(k, Aout, b, perf);
     if (converged(k.c.st, perf)) return perf;
     const double* r = fromZero ? b : w.r.p;
     do {
         hipLaunchKernelGGL((k_copy<float, double>), dim3(k.G), dim3(RED_BS), 0, k.s, n5, w.r32.p, r);
         gmres_cycle<float, float>(k, A, w.LU32.p, w.Dinv32.p, x, w.r32.p, w.w32.p, w.r32.p, w.V32.p, (float*)w.tmp.p);
-        spmv(k, Aout, x, w.wA.p);
-        hipLaunchKernelGGL(k_sub, dim3(k.G), dim3(RED_BS), 0, k.s, n5, w.r.p, b, w.wA.p);
+        cycle_residual(k, Aout, x, b, perf);
+        if (fromZero && perf.n_iterations == 0 && !finite5(perf.final_residual)) {
+            residual_of_zero(k, Aout, b, perf);
+            cycle_residual(k, Aout, x, b, perf);
+        }
         r = w.r.p;
-        cmptmag(k, w.r.p, w.scal.p + S_FIN, w.scal.p + S_NORM);
-        read_scalars(k, S_FIN, 5, perf.final_residual);
         perf.n_iterations++;
     } while (!converged(k.c.st, perf));
     return perf;

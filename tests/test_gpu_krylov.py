@@ -35,3 +35,30 @@ def test_gmres_solves(nx, ny, gs):
     ref = spla.spsolve(A.tocsc(), b.ravel())
     # residual reduced to 1e-14 of the right-hand side's, condition number below 10
     assert np.abs(x.ravel() - ref).max() <= 1e-12 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("nx,ny", [(13, 8), (40, 40)])  # one partition or tile, several
+@pytest.mark.parametrize("kw", [dict(), dict(precision="mixed"),
+                                dict(ilu_order="partitioned", precision="mixed", gram_schmidt="classical")],
+                         ids=["fp64", "mixed", "partitioned mixed"])
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+def test_a_matrix_that_is_not_finite_shows_in_the_residuals(nx, ny, kw, bad):
+    # 0 x inf and 0 x nan are nan: a solve from zero has no finite norm, whatever b is
+    mesh = meshgen.box_2d(nx, ny)
+    n, nI = mesh.n_cells, len(mesh.neighbour)
+    rng = np.random.default_rng(nx)
+    upper, lower = rng.uniform(-0.5, 0.5, (2, nI, 5, 5))
+    diag = rng.uniform(-0.5, 0.5, (n, 5, 5)) + 8.0 * np.eye(5)
+    patches = {p[0]: {"p": "zeroGradient", "T": "zeroGradient", "U": "zeroGradient"} for p in mesh.patches if p[1] != 3}
+    spec = cases.CaseSpec("krylov", mesh, make_thermo(), make_bcs(mesh, patches),
+                          make_settings(n_directions=4, min_iter=0, max_iter=2, **kw), np.ones(n), np.ones(n), np.zeros((n, 3)))
+    dc = _capi.DeviceCase(spec, _capi.DeviceMesh(mesh))
+    for b in (rng.standard_normal((n, 5)), np.zeros((n, 5))):
+        u = upper.copy()
+        u[nI // 2, 2, 3] = bad
+        _, perf = dc.ldu_solve(diag, u, lower, b, np.zeros((n, 5)), mode=2)
+        assert np.isnan(list(perf.initial_residual)).all() and np.isnan(list(perf.final_residual)).all()
+        assert perf.n_iterations == 2 and not perf.converged
+    # a finite one is converged at once for b = 0
+    x, perf = dc.ldu_solve(diag, upper, lower, np.zeros((n, 5)), np.zeros((n, 5)), mode=2)
+    assert not x.any() and perf.n_iterations == 0 and list(perf.initial_residual) == [0.0] * 5
