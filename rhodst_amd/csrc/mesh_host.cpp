@@ -72,6 +72,7 @@ struct PartView {
 // has more than kStreamKD off-diagonal blocks in one sweep or the stream passes
 // 64 GiB.
 static void build_stream(const Mesh& m, const PartView& pv, bool tiles, bool fp32, StreamSet& ps) {
+    ps.clear();
     const bool split = tiles && pv.nParts > 1;
     int kmax = 1;
     for (int i = 0; i < m.nC; ++i) {
@@ -219,6 +220,13 @@ static void build_stream(const Mesh& m, const PartView& pv, bool tiles, bool fp3
             q[3] = (int32_t)lDst[s];
         }
     }
+}
+
+void StreamSet::clear() {
+    kmax = nRec = chainK = 0;
+    for (std::vector<int32_t>* v : {&recBeg, &recMid, &recRows, &recBlk, &need, &src, &rowCell, &chain}) v->clear();
+    for (std::vector<uint32_t>* v : {&hdr, &start}) v->clear();
+    entries.clear();
 }
 
 void StreamSet::upload() {
@@ -421,6 +429,9 @@ static void build_tiles(const Mesh& m, TileSet& ts) {
     }
     order_partitions(m, tile, nT, ts);
     // columns outside the tile: halo cells, each once per tile and sweep
+    ts.haloF.clear();
+    ts.haloB.clear();
+    ts.maxSlots = 0;
     ts.haloFStart.assign(1, 0);
     ts.needF.assign(ts.levPtr.size(), 0);
     ts.haloBStart.assign(1, 0);

@@ -52,8 +52,8 @@ struct DBuf {
     }
     void alloc(size_t count) {
         release();
-        n = count;
         if (count) RDST_HIP(hipMalloc((void**)&p, count * sizeof(T)));
+        n = count;  // only now: "n is what is wanted" means that the memory is there
     }
     void upload(const T* h, size_t count) {
         alloc(count);
@@ -126,6 +126,7 @@ struct StreamSet {
     DBuf<uint16_t> d_entries;
     DBuf<uint32_t> d_hdr, d_start;
     size_t bytes() const { return 16 * (size_t)start.back(); }
+    void clear();  // the host side, before it is built (again, after an attempt that failed)
     void upload();
 };
 

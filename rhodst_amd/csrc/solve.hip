@@ -19,6 +19,7 @@
 // Givens in FP64).
 #include <algorithm>
 #include <cmath>
+#include <memory>
 #include <vector>
 
 #include "rdst_internal.hpp"
@@ -1069,9 +1070,10 @@ static void ensure_work(Case& c) {
     const bool mixed = c.st.precision == RDST_PREC_MIXED;
     SolverWork* w = c.work;
     if (w && w->n == m.nC && w->nDirs == c.st.n_directions && w->mixed == mixed) return;
-    if (w) delete w;
-    w = new SolverWork();
-    c.work = w;
+    delete w;
+    c.work = nullptr;
+    std::unique_ptr<SolverWork> made(new SolverWork());  // the case's when all of it is there
+    w = made.get();
     w->n = m.nC;
     w->n5 = 5 * m.nC;
     w->nDirs = std::max(1, c.st.n_directions);
@@ -1102,6 +1104,7 @@ static void ensure_work(Case& c) {
     w->partA.alloc(5 * RED_MAXG);
     w->partB.alloc(5 * RED_MAXG);
     w->multi.alloc((size_t)(w->nDirs + 1) * RED_MAXG);
+    c.work = made.release();
 }
 
 void solver_free(Case& c) {
@@ -1228,8 +1231,8 @@ void stream_launch(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV*
     auto& ty = tile_y(k.w, (const TV*)nullptr);
     const size_t n5 = 5 * (size_t)m.nC;
     if (ty.n != n5) {
-        ty.alloc(n5);
         k.w.tickets.alloc(2);
+        ty.alloc(n5);
         hipLaunchKernelGGL((k_fill_unset<TV>), dim3(RED_MAXG), dim3(256), 0, k.s, (long)n5, ty.p, k.w.tickets.p);
     }
     const int grid = std::min(ts.nParts, 256);
@@ -1596,7 +1599,7 @@ rdst_solver_perf bicgstab_fp64(Ctx& k, double* x, const double* b) {
     SolverWork& w = k.w;
     const long n5 = w.n5;
     const double* A = k.c.A64.p;
-    if (!w.p.p) { w.p.alloc(n5); w.ph.alloc(n5); w.v.alloc(n5); w.t.alloc(n5); w.th.alloc(n5); w.rw.alloc(n5); }
+    if (!w.rw.p) { w.p.alloc(n5); w.ph.alloc(n5); w.v.alloc(n5); w.t.alloc(n5); w.th.alloc(n5); w.rw.alloc(n5); }
     rdst_solver_perf perf{};
     norm_factor(k, A, x, b);
     spmv(k, A, x, w.p.p);

@@ -1,6 +1,29 @@
 // Host-side check of the ILU(0) record streams and of the tiles of the
 // natural-order sweeps: replays the streams on the CPU with one number per
-// block and compares with the plain sweeps over the block-CSR pattern.
+// block and compares with the plain sweeps over the block-CSR pattern.  Device
+// memory is host memory here, and an allocation can be made to fail.
+#include <hip/hip_runtime.h>
+
+#include <cstdlib>
+#include <cstring>
+
+static int g_mallocsLeft = -1;  // allocations until one fails (negative: none does)
+static hipError_t test_malloc(void** p, size_t n) {
+    if (g_mallocsLeft >= 0 && g_mallocsLeft-- == 0) return hipErrorOutOfMemory;
+    *p = std::malloc(n);
+    return *p ? hipSuccess : hipErrorOutOfMemory;
+}
+static hipError_t test_free(void* p) {
+    std::free(p);
+    return hipSuccess;
+}
+static hipError_t test_memcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
+    std::memcpy(d, s, n);
+    return hipSuccess;
+}
+#define hipMalloc test_malloc
+#define hipFree test_free
+#define hipMemcpy test_memcpy
 #include "../../rhodst_amd/csrc/mesh_host.cpp"
 
 #include <cstdio>
@@ -211,6 +234,62 @@ static int check(const rdst_mesh_desc* desc, bool fp32, bool natural) {
 extern "C" long long ilu_entry_unit(int row, int ent) { return (long long)entry_unit(row, ent); }
 
 extern "C" long long ilu_cell_value(int cell, int nv, int q) { return (long long)cell_value(cell, nv, q); }
+
+// the plan made after an attempt that ran out of device memory at every one of
+// its allocations in turn: the same as one made at once
+static int check_retry(const rdst_mesh_desc* desc, bool fp32, bool natural) {
+    DBuf<double> buf;
+    g_mallocsLeft = 0;
+    try {
+        buf.alloc(8);
+        return fail("the allocation did not fail");
+    } catch (const HipError&) {
+    }
+    g_mallocsLeft = -1;
+    if (buf.p || buf.n) return fail("a failed allocation leaves a size");
+    auto plan = [&](Mesh& m) -> StreamSet& { return natural ? mesh_tiles(m, fp32).ps[fp32] : mesh_stream(m, fp32); };
+    Mesh ref;
+    mesh_build(ref, desc);
+    const StreamSet& a = plan(ref);
+    for (int k = 0;; ++k) {
+        Mesh m;
+        mesh_build(m, desc);
+        bool threw = false;
+        g_mallocsLeft = k;
+        try {
+            plan(m);
+        } catch (const HipError&) {
+            threw = true;
+        }
+        g_mallocsLeft = -1;
+        if (!threw) return k > 3 ? 0 : fail("too few allocations", k);
+        const StreamSet& b = plan(m);
+        if (a.kmax != b.kmax || a.ent != b.ent || a.nRec != b.nRec || a.chainK != b.chainK) return fail("plan numbers", k);
+        if (a.recBeg != b.recBeg || a.recMid != b.recMid || a.recRows != b.recRows || a.recBlk != b.recBlk ||
+            a.entries != b.entries || a.hdr != b.hdr || a.start != b.start || a.need != b.need || a.src != b.src ||
+            a.rowCell != b.rowCell || a.chain != b.chain)
+            return fail("plan records", k);
+        if (b.d_hdr.n != b.hdr.size() || b.d_start.n != b.start.size() || b.d_chain.n != b.chain.size())
+            return fail("device copies", k);
+        const TileSet &s = ref.tiles, &t = m.tiles;
+        if (s.ok != t.ok || s.maxSlots != t.maxSlots || s.nParts != t.nParts || s.rows != t.rows || s.haloF != t.haloF ||
+            s.haloB != t.haloB || s.haloFStart != t.haloFStart || s.haloBStart != t.haloBStart || s.needF != t.needF ||
+            s.localCol != t.localCol || s.d_levPtr.n != t.d_levPtr.n)
+            return fail("tiles", k);
+    }
+}
+
+extern "C" int ilu_plan_retry(const rdst_mesh_desc* desc, int fp32, int natural, char* what, int len) {
+    g_what.clear();
+    int rc = 2;
+    try {
+        rc = check_retry(desc, fp32 != 0, natural != 0);
+    } catch (const std::exception& e) {
+        g_what = e.what();
+    }
+    std::snprintf(what, len, "%s", g_what.c_str());
+    return rc;
+}
 
 extern "C" int ilu_stream_check(const rdst_mesh_desc* desc, int fp32, int natural, char* what, int len) {
     g_what.clear();

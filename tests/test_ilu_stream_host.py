@@ -23,7 +23,8 @@ def replay_lib(tmp_path_factory):
                     "-I", os.path.join(HERE, "..", "include"), os.path.join(HERE, "host", "ilu_stream_check.cpp"),
                     "-L", f"{rocm}/lib", "-lamdhip64", f"-Wl,-rpath,{rocm}/lib", "-o", so], check=True)
     lib = C.CDLL(so)
-    lib.ilu_stream_check.argtypes = [C.POINTER(rdst_mesh_desc), C.c_int, C.c_int, C.c_char_p, C.c_int]
+    for f in (lib.ilu_stream_check, lib.ilu_plan_retry):
+        f.argtypes = [C.POINTER(rdst_mesh_desc), C.c_int, C.c_int, C.c_char_p, C.c_int]
     return lib
 
 
@@ -91,3 +92,13 @@ def test_halo_values_of_large_meshes(replay_lib, cells, nv):
     # the last value of the last cell, at the sizes where 25 per cell pass 31 bits
     replay_lib.ilu_cell_value.restype = C.c_longlong
     assert replay_lib.ilu_cell_value(cells - 1, nv, nv - 1) == nv * cells - 1
+
+
+@pytest.mark.parametrize("name", ["box 25x41", "tets shuffled"])
+@pytest.mark.parametrize("natural", [0, 1])
+@pytest.mark.parametrize("fp32", [0, 1])
+def test_plan_after_running_out_of_memory(replay_lib, name, natural, fp32):
+    md = MeshDesc(MESHES[name]())
+    what = C.create_string_buffer(256)
+    rc = replay_lib.ilu_plan_retry(C.byref(md.desc), fp32, natural, what, 256)
+    assert rc == 0, what.value.decode()
