@@ -283,10 +283,7 @@ int rdst_case_create(rdst_mesh* mesh, const rdst_thermo* thermo, const rdst_bc* 
         if (s.grad_u == RDST_GRAD_CELL_LIMITED && !(s.grad_u_limit >= 0.0 && s.grad_u_limit <= 1.0))
             throw ArgError("rdst_case_create: cellLimited coefficient k must be >= 0 and <= 1");
         if (!(thermo->Cp > thermo->R) || !(thermo->R > 0)) throw ArgError("rdst_case_create: need Cp > R > 0");
-        if (!m->uploaded) {
-            mesh_upload(*m);
-            m->uploaded = true;
-        }
+        mesh_upload(*m);
         if (s.precond == RDST_PRECOND_ILU0 && s.ilu_order == RDST_ILU_PARTITIONED)
             mesh_stream(*m, s.precision == RDST_PREC_MIXED);
         if (s.precond == RDST_PRECOND_ILU0 && s.ilu_order == RDST_ILU_NATURAL)

@@ -871,6 +871,8 @@ void mesh_build(Mesh& m, const rdst_mesh_desc* d, const rdst_mesh_geometry* g) {
 }
 
 void mesh_upload(Mesh& m) {
+    std::lock_guard<std::mutex> lock(m.planMutex);
+    if (m.uploaded) return;
     const int nC = m.nC, nF = m.nF, W = m.ellW;
     m.d_owner.upload(m.owner.data(), m.nI);
     m.d_neigh.upload(m.neigh);
@@ -942,6 +944,7 @@ void mesh_upload(Mesh& m) {
     m.d_sellOfSlot.upload(m.sellOfSlot);
     m.d_sellWidth.upload(m.sellWidth);
     m.d_sellCol.upload(m.sellCol);
+    m.uploaded = true;
 }
 
 }  // namespace rdst

@@ -206,7 +206,7 @@ struct Mesh {
     PartSet sa;
     // the record streams of the partitioned ILU(0) apply, FP64 and FP32 (made
     // by the first case that uses one)
-    std::mutex planMutex;  // of ps, tiles: built on first use
+    std::mutex planMutex;  // of the device copies (uploaded), ps and tiles: made on first use, by any thread
     StreamSet ps[2];
     TileSet tiles;  // of the natural-order ILU(0), made by the first case that uses it
     // sliced-ELL copy of the block-CSR pattern for the SpMV: slices of 64
@@ -256,7 +256,7 @@ constexpr int kPartCells = 1024;
 constexpr int kMaxPartLevels = 32;
 void mesh_build(Mesh& m, const rdst_mesh_desc* d, const rdst_mesh_geometry* g = nullptr);
 void build_partitions(Mesh& m, int maxCells);
-void mesh_upload(Mesh& m);
+void mesh_upload(Mesh& m);  // once; the calls of other threads wait for it
 // the record stream, built and uploaded on first use (by one of the threads that share the mesh)
 StreamSet& mesh_stream(Mesh& m, bool fp32);
 TileSet& mesh_tiles(Mesh& m, bool fp32);     // the tiles and their record stream, likewise

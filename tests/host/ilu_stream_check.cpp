@@ -4,11 +4,15 @@
 // memory is host memory here, and an allocation can be made to fail.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
+#include <thread>
 
+static std::atomic<int> g_mallocs{0};
 static int g_mallocsLeft = -1;  // allocations until one fails (negative: none does)
 static hipError_t test_malloc(void** p, size_t n) {
+    ++g_mallocs;
     if (g_mallocsLeft >= 0 && g_mallocsLeft-- == 0) return hipErrorOutOfMemory;
     *p = std::malloc(n);
     return *p ? hipSuccess : hipErrorOutOfMemory;
@@ -234,6 +238,22 @@ static int check(const rdst_mesh_desc* desc, bool fp32, bool natural) {
 extern "C" long long ilu_entry_unit(int row, int ent) { return (long long)entry_unit(row, ent); }
 
 extern "C" long long ilu_cell_value(int cell, int nv, int q) { return (long long)cell_value(cell, nv, q); }
+
+// device allocations of n threads that all ask for the mesh's device copies and plans
+extern "C" int mesh_upload_mallocs(const rdst_mesh_desc* desc, int n) {
+    Mesh m;
+    mesh_build(m, desc);
+    g_mallocs = 0;
+    std::vector<std::thread> th;
+    for (int t = 0; t < n; ++t)
+        th.emplace_back([&] {
+            mesh_upload(m);
+            mesh_stream(m, false);
+            mesh_tiles(m, false);
+        });
+    for (std::thread& t : th) t.join();
+    return g_mallocs;
+}
 
 // the plan made after an attempt that ran out of device memory at every one of
 // its allocations in turn: the same as one made at once

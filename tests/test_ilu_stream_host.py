@@ -21,7 +21,7 @@ def replay_lib(tmp_path_factory):
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I", f"{rocm}/include",
                     "-I", os.path.join(HERE, "..", "include"), os.path.join(HERE, "host", "ilu_stream_check.cpp"),
-                    "-L", f"{rocm}/lib", "-lamdhip64", f"-Wl,-rpath,{rocm}/lib", "-o", so], check=True)
+                    "-L", f"{rocm}/lib", "-lamdhip64", "-pthread", f"-Wl,-rpath,{rocm}/lib", "-o", so], check=True)
     lib = C.CDLL(so)
     for f in (lib.ilu_stream_check, lib.ilu_plan_retry):
         f.argtypes = [C.POINTER(rdst_mesh_desc), C.c_int, C.c_int, C.c_char_p, C.c_int]
@@ -102,3 +102,10 @@ def test_plan_after_running_out_of_memory(replay_lib, name, natural, fp32):
     what = C.create_string_buffer(256)
     rc = replay_lib.ilu_plan_retry(C.byref(md.desc), fp32, natural, what, 256)
     assert rc == 0, what.value.decode()
+
+
+def test_one_upload_for_all_threads(replay_lib):
+    md = MeshDesc(MESHES["box 25x41"]())
+    replay_lib.mesh_upload_mallocs.argtypes = [C.POINTER(rdst_mesh_desc), C.c_int]
+    one = replay_lib.mesh_upload_mallocs(C.byref(md.desc), 1)
+    assert one > 10 and replay_lib.mesh_upload_mallocs(C.byref(md.desc), 8) == one
