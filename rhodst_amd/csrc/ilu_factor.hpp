@@ -239,9 +239,11 @@ template <class T, int K>
 __global__ __launch_bounds__(CHAIN_THREADS) void k_ilu_chain(const int32_t* __restrict__ levStart,
                                                              const int32_t* __restrict__ levPtr,
                                                              const int32_t* __restrict__ rows, const T* __restrict__ A,
-                                                             T* Dinv, uint8_t* stream, int* fail) {
+                                                             T* Dinv, const int32_t* __restrict__ recBeg,
+                                                             const int64_t* __restrict__ start, uint8_t* stream, int* fail) {
     const int p = blockIdx.x;
-    chain_levels<T, K, CHAIN_THREADS / 64, false>(levStart[p], levStart[p + 1], levPtr, rows, A, Dinv, (T*)nullptr, stream, fail);
+    chain_levels<T, K, CHAIN_THREADS / 64, false>(levStart[p], levStart[p + 1], levPtr, rows, A, Dinv, (T*)nullptr,
+                                                  stream + 16 * start[recBeg[p]], fail);
 }
 
 // The natural-order factor by tiles, taken by ticket in an order that respects
@@ -264,6 +266,8 @@ __global__ __launch_bounds__(CHAIN_TILE_THREADS) void k_ilu_chain_tiles(int nT, 
                                                                         const int32_t* __restrict__ levPtr,
                                                                         const int32_t* __restrict__ rows,
                                                                         const T* __restrict__ A, T* Dinv,
+                                                                        const int32_t* __restrict__ recBeg,
+                                                                        const int64_t* __restrict__ start,
                                                                         uint8_t* stream, int* fail) {
     extern __shared__ __align__(16) unsigned char chain_raw[];
     T* lds = reinterpret_cast<T*>(chain_raw);
@@ -279,7 +283,7 @@ __global__ __launch_bounds__(CHAIN_TILE_THREADS) void k_ilu_chain_tiles(int nT, 
             stream_halo<T, 25, 12>(halo + h0, haloStart[t + 1] - h0, need + l0, l1 - l0 - 1, (const T*)Dinv,
                                    lds + 25 * (rowStart[t + 1] - rowStart[t]));
         } else {
-            chain_levels<T, K, CHAIN_TILE_WAVES, true>(l0, l1, levPtr, rows, A, Dinv, lds, stream, fail);
+            chain_levels<T, K, CHAIN_TILE_WAVES, true>(l0, l1, levPtr, rows, A, Dinv, lds, stream + 16 * start[recBeg[t]], fail);
         }
         __syncthreads();  // every wavefront has read cur
         if (threadIdx.x == 0) cur = atomicAdd(ticket, 1);

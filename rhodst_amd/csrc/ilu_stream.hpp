@@ -68,22 +68,23 @@ __device__ __forceinline__ void barrier_lds() {
 // s + 2 and the values of record s + 1 from the ring, so everything before
 // record s + 1 may be overwritten.
 template <int RING, bool NT>
-__device__ __forceinline__ void stream_load(const uint8_t* stream, const uint32_t* start_, int r0, int r1, uint8_t* ring) {
+__device__ __forceinline__ void stream_load(const uint8_t* stream, const int64_t* start_, int r0, int r1, uint8_t* ring) {
     // scalar loads: the offsets must not wait behind the block loads
-    const __attribute__((address_space(4))) uint32_t* start = (const __attribute__((address_space(4))) uint32_t*)start_;
+    const __attribute__((address_space(4))) int64_t* start = (const __attribute__((address_space(4))) int64_t*)start_;
     constexpr int RC = RING / 1024, MAXF = RC < 60 ? RC : 60;
     const int lane = threadIdx.x & 63;
-    const uint32_t base = start[r0];
-    const int n = r1 - r0, total = (int)((start[r1] - base + 63) / 64);
+    const int64_t base = start[r0];
+    auto from = [&](int q) { return (uint32_t)(start[r0 + q] - base); };  // of record q of the list
+    const int n = r1 - r0, total = (int)((from(n) + 63) / 64);
     const uint8_t* g = stream + 16 * (size_t)base + 16 * lane;
     int issued = 0;
     auto issue = [&](int limit) {
         for (; issued < limit; ++issued) lds_dma16<NT>(g + (size_t)issued * 1024, ring + (issued & (RC - 1)) * 1024);
     };
     // 1 KB pieces that hold everything before the record starting at st
-    auto pieces = [&](uint32_t st) { return (int)((st - base + 63) / 64); };
+    auto pieces = [&](uint32_t st) { return (int)((st + 63) / 64); };
     issue(min(total, MAXF));
-    uint32_t a1 = start[r0 + min(1, n)], a2 = start[r0 + min(2, n)], a3 = start[r0 + min(3, n)], a4 = start[r0 + min(4, n)];
+    uint32_t a1 = from(min(1, n)), a2 = from(min(2, n)), a3 = from(min(3, n)), a4 = from(min(4, n));
     wait_in_flight(issued - pieces(a2));
     barrier_raw();
     issue(min(total, RC));
@@ -91,8 +92,8 @@ __device__ __forceinline__ void stream_load(const uint8_t* stream, const uint32_
     barrier_raw();
     for (int s = 0; s < n; ++s) {
         // a1 .. a4: starts of records s + 1 .. s + 4
-        const uint32_t a5 = start[r0 + min(s + 5, n)];
-        issue(min(total, (int)((a1 - base) / 64) + RC));
+        const uint32_t a5 = from(min(s + 5, n));
+        issue(min(total, (int)(a1 / 64) + RC));
         wait_in_flight(issued - pieces(a4));
         barrier_raw();
         a1 = a2; a2 = a3; a3 = a4; a4 = a5;
@@ -322,7 +323,7 @@ __global__ __launch_bounds__(STREAM_THREADS) void k_stream_apply(const int32_t* 
                                                                  const int32_t* __restrict__ recBeg,
                                                                  const int32_t* __restrict__ recMid,
                                                                  const uint32_t* __restrict__ hdr,
-                                                                 const uint32_t* __restrict__ start,
+                                                                 const int64_t* __restrict__ start,
                                                                  const uint8_t* __restrict__ stream,
                                                                  const TV* __restrict__ r, TV* __restrict__ x) {
     constexpr int RING = stream_ring(sizeof(TM) == 4);
@@ -460,7 +461,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_sweep(int nT, int* ticket
                                                              const int32_t* __restrict__ recMid,
                                                              const int32_t* __restrict__ need,
                                                              const uint32_t* __restrict__ hdr,
-                                                             const uint32_t* __restrict__ start,
+                                                             const int64_t* __restrict__ start,
                                                              const uint8_t* __restrict__ stream, const TV* in, TV* out,
                                                              TV* reset) {
     constexpr int RING = stream_ring(sizeof(TM) == 4);
@@ -494,7 +495,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_sweep(int nT, int* ticket
 }
 // the row entries of every record into the stream (once per buffer)
 __global__ __launch_bounds__(64) void k_stream_entries(int ent, const int32_t* recRows, const uint4* entries,
-                                                       const uint32_t* start, uint8_t* stream) {
+                                                       const int64_t* start, uint8_t* stream) {
     const int q = blockIdx.x;
     const size_t b = entry_unit(recRows[q], ent), e = entry_unit(recRows[q + 1], ent);
     uint4* o = reinterpret_cast<uint4*>(stream + 16 * (size_t)start[q]);
@@ -508,7 +509,7 @@ __global__ __launch_bounds__(64) void k_stream_entries(int ent, const int32_t* r
 // in place already (k_ilu_chain), and LU is the matrix itself.
 template <class T>
 __global__ __launch_bounds__(256) void k_stream_pack(int nRec, int ent, int uOnly, const int32_t* recRows, const int32_t* recBlk,
-                                                    const int32_t* src, const int32_t* rowCell, const uint32_t* start,
+                                                    const int32_t* src, const int32_t* rowCell, const int64_t* start,
                                                     const T* LU, const T* Dinv, uint8_t* stream) {
     const int q = 4 * blockIdx.x + (threadIdx.x >> 6);
     if (q >= nRec) return;

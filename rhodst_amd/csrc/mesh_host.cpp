@@ -68,9 +68,9 @@ struct PartView {
 
 // The record stream of an ILU(0) apply, in the layout StreamSet describes.
 // tiles: the set is a TileSet; if it is more than one tile, the two sweeps are
-// read by separate launches, so the backward records start a ring of their own.  Left empty (kmax = 0) when a row
-// has more than kStreamKD off-diagonal blocks in one sweep or the stream passes
-// 64 GiB.
+// read by separate launches, so the backward records start a ring of their own.
+// Left empty (kmax = 0) when a row has more than kStreamKD off-diagonal blocks in
+// one sweep.
 static void build_stream(const Mesh& m, const PartView& pv, bool tiles, bool fp32, StreamSet& ps) {
     ps.clear();
     const bool split = tiles && pv.nParts > 1;
@@ -92,11 +92,12 @@ static void build_stream(const Mesh& m, const PartView& pv, bool tiles, bool fp3
     ps.recRows.assign(1, 0);
     ps.recBlk.assign(1, 0);
     size_t pos = 0;
-    std::vector<uint32_t> lDst(m.nnzb, 0), dDst(m.nC, 0);  // of forward blocks and Dinv, 4-byte units
+    std::vector<uint32_t> lDst(m.nnzb, 0), dDst(m.nC, 0);  // of forward blocks and Dinv, 4-byte units from the partition's start
     auto size_of = [&](int nr, int nb) { return nr * ps.ent + ((nb * blk + 15) & ~15); };
     for (int p = 0; p < pv.nParts; ++p) {
         const int rs = pv.rowStart[p], nOwn = pv.rowStart[p + 1] - rs;
         const int l0 = pv.levStart[p], nl = pv.levStart[p + 1] - l0 - 1;
+        const size_t origin = pos;
         size_t base = pos;
         for (int sweep = 0; sweep < 2; ++sweep) {
             if (sweep == 1) {
@@ -139,7 +140,7 @@ static void build_stream(const Mesh& m, const PartView& pv, bool tiles, bool fp3
                         uint16_t* e = ps.entries.data() + e0;
                         e[0] = (uint16_t)(5 * w.t);
                         e[1] = (uint16_t)(first | w.cnt << 8);
-                        const size_t at = (pos + (size_t)nr * ps.ent + (size_t)blk * first) / 4;
+                        const size_t at = (pos - origin + (size_t)nr * ps.ent + (size_t)blk * first) / 4;
                         if (sweep) {
                             dDst[w.i] = (uint32_t)at;
                             ps.src.push_back(-(w.i + 1));
@@ -158,7 +159,7 @@ static void build_stream(const Mesh& m, const PartView& pv, bool tiles, bool fp3
                             }
                         first += w.cnt + sweep;
                     }
-                    ps.start.push_back((uint32_t)(pos / 16));
+                    ps.start.push_back((int64_t)(pos / 16));
                     ps.hdr.push_back((uint32_t)nr | (uint32_t)(bytes / 16) << 16);
                     ps.recRows.push_back(ps.recRows.back() + nr);
                     ps.recBlk.push_back((int32_t)ps.src.size());
@@ -170,14 +171,13 @@ static void build_stream(const Mesh& m, const PartView& pv, bool tiles, bool fp3
         }
         ps.recBeg.push_back((int32_t)ps.hdr.size());
         pos = (pos + 1023) & ~(size_t)1023;  // the loader copies 1 KB pieces
-        if (pos / 16 > 0xffffffffull) return;
     }
-    ps.start.push_back((uint32_t)(pos / 16));
+    ps.start.push_back((int64_t)(pos / 16));
     ps.nRec = (int)ps.hdr.size();
     ps.kmax = kmax;
     // the factor as a chain: a bipartite mesh has no triangle, any other is looked through
     int K = 1;
-    bool tri = pos / 4 > 0xffffffffull;
+    bool tri = false;
     for (int i = 0; i < m.nC && !tri; ++i) {
         int lo = 0;
         for (int p = m.rowPtr[i]; p < m.slotDiag[i]; ++p) {
@@ -225,7 +225,8 @@ static void build_stream(const Mesh& m, const PartView& pv, bool tiles, bool fp3
 void StreamSet::clear() {
     kmax = nRec = chainK = 0;
     for (std::vector<int32_t>* v : {&recBeg, &recMid, &recRows, &recBlk, &need, &src, &rowCell, &chain}) v->clear();
-    for (std::vector<uint32_t>* v : {&hdr, &start}) v->clear();
+    hdr.clear();
+    start.clear();
     entries.clear();
 }
 

@@ -111,12 +111,14 @@ struct StreamSet {
     std::vector<int32_t> recBeg, recMid;    // [nParts + 1], [nParts]: forward records [recBeg, recMid), backward to the next recBeg
     std::vector<int32_t> recRows, recBlk;   // [nRec + 1] first row entry, first block
     std::vector<uint16_t> entries;          // [rows][ent / 2]
-    std::vector<uint32_t> hdr, start;       // [nRec]; [nRec + 1] first 16-byte unit
+    std::vector<uint32_t> hdr;              // [nRec]
+    std::vector<int64_t> start;             // [nRec + 1] first 16-byte unit
     std::vector<int32_t> need;              // [nRec] halo cells whose values must be there before this record (tiles only)
     std::vector<int32_t> src, rowCell;      // [blocks] block-CSR slot, or -(cell + 1) for Dinv; the row's cell in a backward record, else -1
     // The factor as a chain of diagonal blocks (no three coupled cells are
     // coupled pairwise): per row, in the partitions' row order, cell, lower
-    // blocks, diagonal slot, where Dinv goes in the stream (4-byte units); per
+    // blocks, diagonal slot, where Dinv goes in the stream (4-byte units from the
+    // partition's first record: a stream may be longer than 32 bits address); per
     // lower block its slot, the transposed coupling's slot, its cell (in a tile's
     // stream the column in the tile), where L goes.  chainK: places per row, 0 when the factor has other updates.
     int chainK = 0;
@@ -124,7 +126,8 @@ struct StreamSet {
     DBuf<int32_t> d_chain;
     DBuf<int32_t> d_recBeg, d_recMid, d_recRows, d_recBlk, d_need, d_src, d_rowCell;
     DBuf<uint16_t> d_entries;
-    DBuf<uint32_t> d_hdr, d_start;
+    DBuf<uint32_t> d_hdr;
+    DBuf<int64_t> d_start;
     size_t bytes() const { return 16 * (size_t)start.back(); }
     void clear();  // the host side, before it is built (again, after an attempt that failed)
     void upload();

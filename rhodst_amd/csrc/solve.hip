@@ -1202,10 +1202,11 @@ void chain_launch(Ctx& k, const StreamSet& ps, const T* A, T* Dinv, bool natural
                            0, k.s, nd, Dinv, fail);
         hipLaunchKernelGGL((k_ilu_chain_tiles<T, K>), dim3(std::min(ts.nParts, 512)), dim3(CHAIN_TILE_THREADS),
                            chain_lds<T>(ts), k.s, ts.nParts, fail + 1, ts.d_rowStart.p, ts.d_haloFStart.p, ts.d_haloF.p,
-                           ts.d_needF.p, ts.d_levStart.p, ts.d_levPtr.p, ps.d_chain.p, A, Dinv, st, fail);
+                           ts.d_needF.p, ts.d_levStart.p, ts.d_levPtr.p, ps.d_chain.p, A, Dinv, ps.d_recBeg.p, ps.d_start.p, st,
+                           fail);
     } else {
         hipLaunchKernelGGL((k_ilu_chain<T, K>), dim3(m.nParts), dim3(CHAIN_THREADS), 0, k.s, m.d_partLevStart.p,
-                           m.d_partLevPtr.p, ps.d_chain.p, A, Dinv, st, fail);
+                           m.d_partLevPtr.p, ps.d_chain.p, A, Dinv, ps.d_recBeg.p, ps.d_start.p, st, fail);
     }
     stream_pack<T>(k, ps, A, (const T*)Dinv, true);
 }

@@ -119,11 +119,11 @@ static int check(const rdst_mesh_desc* desc, bool fp32, bool natural) {
         for (int part2 = 0; part2 < (split ? 2 : 1); ++part2) {
             const int q0 = part2 ? ps.recMid[p] : ps.recBeg[p], q1 = split && !part2 ? ps.recMid[p] : ps.recBeg[p + 1];
             if (q0 == q1) continue;
-            const uint32_t base = ps.start[q0];
+            const int64_t base = ps.start[q0];
             if (base % 64) return fail("start of a sweep", p);
             // the last 1 KB piece ends inside the stream
             if (16 * (size_t)(base + (ps.start[q1] - base + 63) / 64 * 64) > ps.bytes()) return fail("past the stream's end", p);
-            uint32_t off = 0;
+            int64_t off = 0;
             for (int q = q0; q < q1; ++q) {
                 const int nr = ps.recRows[q + 1] - ps.recRows[q], nb = ps.recBlk[q + 1] - ps.recBlk[q];
                 const int len = (nr * ps.ent + ((nb * 25 * (fp32 ? 4 : 8) + 15) & ~15)) / 16;
@@ -131,15 +131,19 @@ static int check(const rdst_mesh_desc* desc, bool fp32, bool natural) {
                 off += ps.hdr[q] >> 16;
                 if ((int)((ps.start[q] - base) % ring) + len > ring) return fail("record crosses the ring's end", q);
                 // while record q + 1 is read, record q + 3 arrives
-                const uint32_t a = ps.start[std::min(q + 1, q1)] - base, b = ps.start[std::min(q + 4, q1)] - base;
+                const int64_t a = ps.start[std::min(q + 1, q1)] - base, b = ps.start[std::min(q + 4, q1)] - base;
                 if ((b + 63) / 64 > a / 64 + ring / 64) return fail("three records do not fit the ring", q);
             }
         }
     // the factor chain: each row's blocks, their transposed couplings and their places in the stream
     if (ps.chainK) {
+        // (from the partition's first record: nothing in the plan bounds the stream's length to 32 bits)
+        static_assert(sizeof(ps.start[0]) == 8, "the start of a record in a stream of more than 64 GiB");
         std::vector<uint32_t> place(m.nnzb, 0), placeD(n, 0);
-        for (int q = 0; q < ps.nRec; ++q) {
-            const size_t v = 16 * (size_t)ps.start[q] + (size_t)ps.ent * (ps.recRows[q + 1] - ps.recRows[q]);
+        for (int q = 0, p = 0; q < ps.nRec; ++q) {
+            while (q >= ps.recBeg[p + 1]) ++p;
+            const size_t v = 16 * (size_t)(ps.start[q] - ps.start[ps.recBeg[p]]) +
+                             (size_t)ps.ent * (ps.recRows[q + 1] - ps.recRows[q]);
             for (int b = ps.recBlk[q]; b < ps.recBlk[q + 1]; ++b) {
                 const uint32_t at = (uint32_t)((v + (size_t)(25 * (fp32 ? 4 : 8)) * (b - ps.recBlk[q])) / 4);
                 if (ps.src[b] < 0) placeD[-ps.src[b] - 1] = at;
