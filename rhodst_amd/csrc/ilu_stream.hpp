@@ -147,10 +147,21 @@ template <class TM, class TV, int KDU, int RING, bool PUB>
 __device__ __forceinline__ void stream_compute(const uint32_t* hdr, int r0, int nF, int n, const uint8_t* ring, TV* y,
                                                const int* to, TV* out) {
     constexpr int MASK = RING - 1, ENT = stream_entry(KDU), BLK = 25 * (int)sizeof(TM);
+    // Rows of more than four blocks in a sweep.  A wavefront without one skips the
+    // blocks past the fourth (K4), and FP64 with eight reads the next record's
+    // values after this one's products (LATE): a wavefront has 256 registers, and
+    // with all nine blocks of both records in them it spilled 356 of them.  Apply of
+    // 403 k hexahedra numbered at random (six blocks): all of eight 292 us, six 142,
+    // and so 125; FP32 with six gains nothing (77 / 104 us) and keeps all of them.  263 k
+    // polyhedra, seven blocks: FP64 382 us with eight blocks, 270 so; FP32 263, 229.
+    constexpr int K4 = KDU > 6 || (KDU > 4 && sizeof(TM) == 8) ? 4 : KDU;
+    constexpr bool LATE = KDU > 6 && sizeof(TM) == 8;
+    constexpr int KG = LATE ? KDU : K4;  // columns gathered before the products
     struct Ent {
         uint32_t w[ENT / 4];
         int eb, vb, nR;  // ring offset of the record's entries and values, rows (uniform)
         bool row;        // this lane has a row
+        bool wide;       // a row of this wavefront has more than K4 off-diagonal blocks (uniform)
     };
     struct Val {
         TM d[5], v[KDU][5];
@@ -201,12 +212,21 @@ __device__ __forceinline__ void stream_compute(const uint32_t* hdr, int r0, int 
 #pragma unroll
         for (int c = 0; c < 5; ++c) V.d[c] = pd[c];
 #pragma unroll
-        for (int k = 0; k < KDU; ++k)
+        for (int k = 0; k < K4; ++k)
 #pragma unroll
             for (int c = 0; c < 5; ++c) V.v[k][c] = p[25 * k + c];
+        if constexpr (KDU > K4) {
+            // rows are in descending order of their blocks: lane 0 has the wavefront's longest
+            E.wide = (int)(__builtin_amdgcn_readfirstlane(E.w[0]) >> 24) > K4;
+            if (E.wide)
+#pragma unroll
+                for (int k = K4; k < KDU; ++k)
+#pragma unroll
+                    for (int c = 0; c < 5; ++c) V.v[k][c] = p[25 * k + c];
+        }
     };
     struct Gat {
-        TV a, d[5], v[KDU][5];
+        TV a, d[5], v[KG][5];
         int to;
     };
     auto gather = [&](const Ent& E, Gat& G) {
@@ -216,22 +236,40 @@ __device__ __forceinline__ void stream_compute(const uint32_t* hdr, int r0, int 
 #pragma unroll
         for (int c = 0; c < 5; ++c) G.d[c] = yr[c];
 #pragma unroll
-        for (int k = 0; k < KDU; ++k) {
+        for (int k = 0; k < K4; ++k) {
             const uint32_t w = E.w[1 + k / 2];
             const TV* yv = y + ((k & 1) ? w >> 16 : w & 0xffff);
 #pragma unroll
             for (int c = 0; c < 5; ++c) G.v[k][c] = yv[c];
         }
+        if constexpr (KG > K4)
+            if (E.wide)
+#pragma unroll
+                for (int k = K4; k < KG; ++k) {
+                    const uint32_t w = E.w[1 + k / 2];
+                    const TV* yv = y + ((k & 1) ? w >> 16 : w & 0xffff);
+#pragma unroll
+                    for (int c = 0; c < 5; ++c) G.v[k][c] = yv[c];
+                }
     };
     auto apply = [&](int s, const Ent& E, const Val& V, const Gat& G) {
         const int cnt = (int)(E.w[0] >> 24);
         TV acc = dot5(V.d, G.d);
         acc = s < nF ? G.a : acc;
 #pragma unroll
-        for (int k = 0; k < KDU; ++k) {
+        for (int k = 0; k < K4; ++k) {
             const TV dot = dot5(V.v[k], G.v[k]);
             acc = k < cnt ? acc - dot : acc;
         }
+        if constexpr (KDU > K4)
+            if (E.wide)
+#pragma unroll
+                for (int k = K4; k < KDU; ++k) {
+                    const uint32_t w = E.w[1 + k / 2];
+                    const TV* yv = KG > K4 ? G.v[k < KG ? k : 0] : y + ((k & 1) ? w >> 16 : w & 0xffff);
+                    const TV dot = dot5(V.v[k], yv);
+                    acc = k < cnt ? acc - dot : acc;
+                }
         if (E.row) {
             y[(E.w[0] & 0xffff) + r] = acc;
             if constexpr (PUB) store_dev(out + G.to, acc);
@@ -246,9 +284,13 @@ __device__ __forceinline__ void stream_compute(const uint32_t* hdr, int r0, int 
         head(s + 2, E2);
         if (w12 < max(E0.nR, max(E1.nR, E2.nR))) {
             gather(E0, G);
+            if constexpr (LATE) {
+                apply(s, E0, V0, G);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             entry(E2);
             values(s + 1, E1, V1);
-            apply(s, E0, V0, G);
+            if constexpr (!LATE) apply(s, E0, V0, G);
         }
         barrier_lds();
     };

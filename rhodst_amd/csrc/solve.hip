@@ -1247,8 +1247,10 @@ void stream_launch(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV*
 }
 template <class TM, class TV>
 void stream_apply(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV* r, TV* x, bool natural) {
+    // tetrahedra and ordered hexahedra have up to four, hexahedra in any order six
     if (ps.kmax <= 3) stream_launch<TM, TV, 3>(k, ps, stream, r, x, natural);
     else if (ps.kmax <= 4) stream_launch<TM, TV, 4>(k, ps, stream, r, x, natural);
+    else if (ps.kmax <= 6) stream_launch<TM, TV, 6>(k, ps, stream, r, x, natural);
     else stream_launch<TM, TV, kStreamKD>(k, ps, stream, r, x, natural);
 }
 
