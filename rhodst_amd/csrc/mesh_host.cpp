@@ -470,6 +470,39 @@ static void build_tiles(const Mesh& m, TileSet& ts) {
     }
 }
 
+// Whether the sweeps go by tiles or by one launch per level, from what each is
+// expected to cost (us, both sweeps).  Tiles: the longest chain of tiles, each
+// 0.7 per level and 1.6 per 256 halo values (the halo wavefront asks for those one
+// window after the other).  Levels: 4 per launch and 0.5 per 100 rows of a level.
+// A structured numbering has many levels and thin halos; cells numbered at random
+// have a dozen levels, and tiles whose halo is several times the tile.  Step of
+// 20 vectors FP64, levels / tiles, with the two predictions per sweep: wing
+// 67.6 k 44.5 / 7.9 ms (906, 312 us), the same in the order of 4x4x4 tiles 45.2 / 32.4
+// (906, 641), hybrid airfoil 9.1 k numbered at random within 100 cells 31.8 / 16.3
+// (614, 425); 2.7 k quads at random 3.8 / 5.9 (62, 129), 10.8 k at random within 1000
+// cells 6.1 / 10.1 (122, 262), 1.5 k tetrahedra 2.8 / 3.2 (44, 49).
+bool tiles_pay(const Mesh& m, const TileSet& ts) {
+    if (ts.nParts <= 1) return true;  // no halo: one workgroup and no launches between the levels
+    std::vector<int32_t> tile(m.nC);
+    for (int t = 0; t < ts.nParts; ++t)
+        for (int q = ts.rowStart[t]; q < ts.rowStart[t + 1]; ++q) tile[ts.rows[q]] = t;
+    double tiles = 0.0;
+    for (int sweep = 0; sweep < 2; ++sweep) {
+        const std::vector<int32_t>&hs = sweep ? ts.haloBStart : ts.haloFStart, &h = sweep ? ts.haloB : ts.haloF;
+        std::vector<double> end(ts.nParts, 0.0);
+        double longest = 0.0;
+        for (int k = 0; k < ts.nParts; ++k) {
+            const int t = sweep ? ts.nParts - 1 - k : k;
+            double begin = 0.0;
+            for (int q = hs[t]; q < hs[t + 1]; ++q) begin = std::max(begin, end[tile[h[q]]]);
+            end[t] = begin + 0.7 * (ts.levStart[t + 1] - ts.levStart[t] - 1) + 1.6 * ((5 * (hs[t + 1] - hs[t]) + 255) / 256);
+            longest = std::max(longest, end[t]);
+        }
+        tiles += longest;
+    }
+    return tiles <= 4.0 * (m.nLevL + m.nLevU) + 2 * 0.005 * m.nC;
+}
+
 TileSet& mesh_tiles(Mesh& m, bool fp32) {
     std::lock_guard<std::mutex> lock(m.planMutex);
     TileSet& ts = m.tiles;
@@ -485,8 +518,8 @@ TileSet& mesh_tiles(Mesh& m, bool fp32) {
         ts.d_levStart.upload(ts.levStart);
         ts.d_levPtr.upload(ts.levPtr);
         // the tile's vector and its halo, and where the vector's entries belong, next to the
-        // ring in 160 KB of LDS; 16-bit columns
-        ts.ok = 40 * (size_t)ts.maxSlots + 20 * kTileCells + stream_ring(false) + 4096 <= 160 * 1024;
+        // ring in 160 KB of LDS (16-bit columns), and the sweeps the faster by it
+        ts.ok = 40 * (size_t)ts.maxSlots + 20 * kTileCells + stream_ring(false) + 4096 <= 160 * 1024 && tiles_pay(m, ts);
         ts.tried = true;
     }
     StreamSet& ps = ts.ps[fp32];

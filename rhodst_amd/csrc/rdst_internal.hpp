@@ -158,7 +158,7 @@ struct PartSet {
 // the tile's own: halo cell q of tile t's forward sweep is haloF[haloFStart[t]
 // + q], column nRows(t) + q, in the order in which the sweep's levels read them.
 struct TileSet : PartSet {
-    bool tried = false, ok = false;
+    bool tried = false, ok = false;  // ok: they fit and are worth it (tiles_pay), else the sweeps go level by level
     int maxSlots = 0;  // most rows + halo cells of a tile
     std::vector<int32_t> haloFStart, haloF, haloBStart, haloB;
     std::vector<int32_t> needF;  // beside levPtr: forward halo cells that a level (and those before) reads

@@ -1344,7 +1344,7 @@ void precondition(Ctx& k, const TM* LU, const TM* Dinv, const TV* r, TV* x, TV* 
         stream_apply<TM, TV>(k, ns, stream_buf(k.w, LU).p, r, x, true);
         return;
     }
-    // tiles too wide for LDS, or rows too long for the stream: level by level
+    // tiles too wide for LDS or slower than the levels, or rows too long for the stream: level by level
     for (const LevelRun& g : m.runL) {
         if (g.fused) {
             hipLaunchKernelGGL((k_ilu_fwd_seg<TM, TV>), dim3(1), dim3(ILU_SEG_THREADS), 0, k.s, g.L0, g.L1,

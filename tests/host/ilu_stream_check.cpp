@@ -303,6 +303,17 @@ static int check_retry(const rdst_mesh_desc* desc, bool fp32, bool natural) {
     }
 }
 
+// kmax, chainK, partitions or tiles, and whether the natural order goes by tiles
+extern "C" void ilu_plan_numbers(const rdst_mesh_desc* desc, int fp32, int natural, int* out) {
+    Mesh m;
+    mesh_build(m, desc);
+    const StreamSet& ps = natural ? mesh_tiles(m, fp32 != 0).ps[fp32] : mesh_stream(m, fp32 != 0);
+    out[0] = ps.kmax;
+    out[1] = ps.chainK;
+    out[2] = natural ? m.tiles.nParts : m.nParts;
+    out[3] = m.tiles.ok;
+}
+
 extern "C" int ilu_plan_retry(const rdst_mesh_desc* desc, int fp32, int natural, char* what, int len) {
     g_what.clear();
     int rc = 2;

@@ -109,3 +109,24 @@ def test_one_upload_for_all_threads(replay_lib):
     replay_lib.mesh_upload_mallocs.argtypes = [C.POINTER(rdst_mesh_desc), C.c_int]
     one = replay_lib.mesh_upload_mallocs(C.byref(md.desc), 1)
     assert one > 10 and replay_lib.mesh_upload_mallocs(C.byref(md.desc), 8) == one
+
+
+def plan_numbers(lib, mesh, natural, fp32=0):
+    out = (C.c_int * 4)()
+    lib.ilu_plan_numbers.argtypes = [C.POINTER(rdst_mesh_desc), C.c_int, C.c_int, C.POINTER(C.c_int)]
+    lib.ilu_plan_numbers.restype = None
+    md = MeshDesc(mesh)
+    lib.ilu_plan_numbers(C.byref(md.desc), fp32, natural, out)
+    return list(out)
+
+
+@pytest.mark.parametrize("name,tiles", [
+    # one tile, and numberings with many levels and thin halos
+    ("one cell", True), ("box 33x31", True), ("line", True), ("box 150x70", True), ("hybrid airfoil", True), ("wing", True),
+    ("wing tiles", True),
+    # a dozen levels
+    ("box shuffled", False), ("tets shuffled", False)])
+def test_tiles_where_they_pay(replay_lib, name, tiles):
+    kmax, _, n, ok = plan_numbers(replay_lib, MESHES[name](), natural=1)
+    assert bool(ok) == tiles and (kmax > 0) == tiles
+    assert (n == 1) == (name in ("one cell", "box 33x31"))
