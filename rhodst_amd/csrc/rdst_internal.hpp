@@ -392,8 +392,9 @@ struct Case {
     struct SolverWork* work = nullptr;
     // device copies of x and b of rdst_ldu_solve (allocated on first use)
     DBuf<double> lduX, lduB;
-    // staging of host arrays that are laid out differently on the device (at
-    // most kStageDoubles, allocated on first use)
+    // staging of host arrays that are laid out differently on the device: made
+    // with the case, so that reading a field back needs no memory and no call is
+    // slower for being the first
     DBuf<double> stage;
     // time-control scalars
     double residual = -1, residualRatio = 1, courantScalar = 1;
@@ -425,8 +426,7 @@ struct Case {
 // One copy and one pass on the device; the host side only copies.  (The
 // components copied one by one and interleaved by the host took 2.9 ms for the
 // five of R at 555 k cells, against 0.6.)
-constexpr size_t kStageDoubles = (size_t)8 << 20;  // 64 MiB
-double* stage_buf(Case& c, size_t want);            // min(want, kStageDoubles) doubles
+constexpr size_t kStageDoubles = (size_t)8 << 20;  // 64 MiB, the longest staging buffer
 void download_aos(Case& c, const double* const* comps, int k, size_t n, double* out);
 void upload_aos(Case& c, double* const* comps, int k, size_t n, const double* in);
 // face-field store modes of the face loop

@@ -1718,8 +1718,8 @@ void ldu_solve(Case& c, const double* diag, const double* upper, const double* l
             size_t n;
         } parts[3] = {{diag, m.d_slotDiag.p, (size_t)m.nC}, {upper, m.d_slotUpper.p, (size_t)m.nI},
                       {lower, m.d_slotLower.p, (size_t)m.nI}};
-        double* st = stage_buf(c, 25 * (size_t)std::max(m.nC, m.nI));
-        const size_t cap = std::min(kStageDoubles, c.stage.n) / 25;
+        double* st = c.stage.p;
+        const size_t cap = c.stage.n / 25;
         for (const Part& p : parts)
             for (size_t b0 = 0; b0 < p.n; b0 += cap) {
                 const size_t cnt = std::min(cap, p.n - b0);

@@ -505,18 +505,12 @@ __global__ void k_store_old(int n, Fields F) {
 
 }  // namespace
 
-double* stage_buf(Case& c, size_t want) {
-    want = std::min(want, kStageDoubles);
-    if (c.stage.n < want) c.stage.alloc(want);
-    return c.stage.p;
-}
-
 void download_aos(Case& c, const double* const* comps, int k, size_t n, double* out) {
     Comps cp{};
     for (int d = 0; d < k; ++d) cp.p[d] = const_cast<double*>(comps[d]);
-    double* st = stage_buf(c, k * n);
-    for (size_t e = 0; e < k * n; e += kStageDoubles) {
-        const size_t cnt = std::min(kStageDoubles, k * n - e);
+    double* st = c.stage.p;
+    for (size_t e = 0; e < k * n; e += c.stage.n) {
+        const size_t cnt = std::min(c.stage.n, k * n - e);
         hipLaunchKernelGGL(k_interleave, dim3(std::min<long>(8192, blocks_for((long)cnt, 256))), dim3(256), 0, c.stream, cp,
                            k, e, cnt, st);
         RDST_HIP(hipGetLastError());
@@ -528,9 +522,9 @@ void download_aos(Case& c, const double* const* comps, int k, size_t n, double* 
 void upload_aos(Case& c, double* const* comps, int k, size_t n, const double* in) {
     Comps cp{};
     for (int d = 0; d < k; ++d) cp.p[d] = comps[d];
-    double* st = stage_buf(c, k * n);
-    for (size_t e = 0; e < k * n; e += kStageDoubles) {
-        const size_t cnt = std::min(kStageDoubles, k * n - e);
+    double* st = c.stage.p;
+    for (size_t e = 0; e < k * n; e += c.stage.n) {
+        const size_t cnt = std::min(c.stage.n, k * n - e);
         RDST_HIP(hipMemcpyAsync(st, in + e, cnt * sizeof(double), hipMemcpyHostToDevice, c.stream));
         hipLaunchKernelGGL(k_deinterleave, dim3(std::min<long>(8192, blocks_for((long)cnt, 256))), dim3(256), 0, c.stream,
                            cp, k, e, cnt, st);

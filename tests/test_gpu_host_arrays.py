@@ -3,6 +3,7 @@
 one staging piece."""
 import numpy as np
 import pytest
+import torch
 
 from rhodst_amd import DeviceCase, cases
 
@@ -24,3 +25,15 @@ def test_momentum_round_trip(nx, ny):
     R = dc.get(8)
     assert R.shape == (nx * ny, 5) and np.isfinite(R).all()
     assert np.isclose(np.sqrt((R ** 2).sum()), dc.set_courant(), rtol=1e-12)
+
+
+def test_the_first_read_back_allocates_nothing():
+    # 480 k cells: the staging of R (19 MB) shows in the device's free memory
+    spec = cases.box_farfield_case(nx=800, ny=600, jitter=0.0)
+    dc = DeviceCase(spec)
+    dc.flux_residual()
+    free = torch.cuda.mem_get_info()[0]
+    R = dc.get(8)
+    dc.put(1, dc.get(1))
+    assert torch.cuda.mem_get_info()[0] == free
+    assert np.array_equal(R, dc.get(8))
