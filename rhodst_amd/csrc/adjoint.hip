@@ -888,8 +888,8 @@ void av_pass(Case& c, int pass0, int nPass, const AvOut& o) {
 // Passes of one launch: one pass over a mesh of a few hundred blocks leaves most
 // of the chip idle (a block per CU, one wavefront per SIMD), so several go
 // together until there are some AV_BLOCKS blocks; a mesh of that many blocks by
-// itself takes one pass at a time, with the scratch it always had.  The scratch of a
-// launch stays below 19 doubles x 256 x AV_BLOCKS (160 MB).
+// itself takes one pass at a time, with 19 doubles per cell of scratch.  A launch
+// of several stays below 19 doubles x 256 x AV_BLOCKS (160 MB).
 constexpr int AV_BLOCKS = 4096;
 int av_batch(const Mesh& m) { return std::max(1, std::min(5 * m.wideColors, AV_BLOCKS / std::max(1, blocks_for(m.nC, 256)))); }
 // passes [0, 5 x colours) in batches: f(pass0, nPass)
@@ -899,10 +899,11 @@ void av_batches(const Mesh& m, Fn f) {
     for (int p = 0; p < total; p += step) f(p, std::min(step, total - p));
 }
 
-void av_buffers(Case& c) {
-    const size_t n = (size_t)c.mesh->nC * av_batch(*c.mesh);
-    if (c.avGrad.n != 18 * n) c.avGrad.alloc(18 * n);
-    if (c.avObj.n != n) c.avObj.alloc(n);
+// the scratch of launches of up to nPass passes
+void av_buffers(Case& c, int nPass) {
+    const size_t n = (size_t)c.mesh->nC * nPass;
+    if (c.avGrad.n < 18 * n) c.avGrad.alloc(18 * n);
+    if (c.avObj.n < n) c.avObj.alloc(n);
 }
 
 }  // namespace
@@ -974,7 +975,7 @@ namespace {
 void viscous_linearise(Case& c) {
     Mesh& m = *c.mesh;
     build_wide(m);
-    av_buffers(c);
+    av_buffers(c, av_batch(m));
     const size_t nnz = m.wideCols.size();
     if (c.adjW.n != 25 * nnz) c.adjW.alloc(25 * nnz);
     if (c.adjWT.n != 25 * nnz) c.adjWT.alloc(25 * nnz);
@@ -1089,7 +1090,7 @@ void adjoint_residual(Case& c, double* R) {
     adjoint_check_scheme(c);
     if (c.st.viscous) {
         build_wide(*c.mesh);
-        av_buffers(c);
+        av_buffers(c, 1);
         AvOut out;
         out.Rv = R;
         av_pass(c, -1, 1, out);
@@ -1112,7 +1113,7 @@ void adjoint_objective_gradient(Case& c, int patch, const double* dir, double q,
         // depends on the wall cell's face neighbours: one pass per colour
         Mesh& m = *c.mesh;
         build_wide(m);
-        av_buffers(c);
+        av_buffers(c, av_batch(m));
         AvOut out;
         out.patch = patch;
         out.dir = dir;
@@ -1139,7 +1140,7 @@ void adjoint_objective_cells(Case& c, int patch, const double* dir, double q, do
     Mesh& m = *c.mesh;
     if (c.st.viscous) {
         build_wide(m);
-        av_buffers(c);
+        av_buffers(c, 1);
         AvOut out;
         out.patch = patch;
         out.dir = dir;

@@ -8,6 +8,7 @@ eddy viscosity of a Spalart-Allmaras case, and the shape gradient of a
 laminar channel bump against central differences of the re-converged Cd."""
 import numpy as np
 import pytest
+import torch
 
 from rhodst_amd import DeviceCase, cases
 
@@ -335,3 +336,19 @@ def test_objective_cells_sum_to_force(viscous):
     assert abs(o.sum() - c) <= 1e-11 * max(abs(c), 1e-30)
     # only the cells on the patch hold a share
     assert 0 < np.count_nonzero(o) <= spec.mesh.patches[patch][3]
+
+
+def test_a_residual_takes_the_scratch_of_one_pass():
+    # 10 000 cells: 1.5 MB of scratch for one pass, 1.5 MB for each of the linearisation's 60 or so together
+    spec = cases.box_viscous_case(nx=100, ny=100)
+    # the kernels' own private memory is taken at their first launch on each of the hardware queues
+    warm = [DeviceCase(spec) for _ in range(5)]
+    for w in warm:
+        w.adjoint_residual()
+    dc = DeviceCase(spec)
+    dc.iterate(1)
+    free = torch.cuda.mem_get_info()[0]
+    R = dc.adjoint_residual()
+    assert free - torch.cuda.mem_get_info()[0] < 40e6  # the coupling pattern (5 MB) and one pass
+    dc.adjoint_linearise()
+    assert np.array_equal(dc.adjoint_residual(), R)
