@@ -167,6 +167,20 @@ struct TileSet : PartSet {
 };
 constexpr int kTileCells = 512;  // most rows of a tile
 
+// Whether the Spalart-Allmaras Gauss-Seidel sweep (columns: 6 or 8 per row) reads
+// its partitions from memory level by level rather than from LDS.  Where a
+// partition's rows take more than half of a CU's LDS, one partition at a time runs
+// there, 50 us and 0.7 (six columns) or 0.85 (eight) for each of its levels; from
+// memory eight run at once, the first in 3 us per level, a further one per CU in
+// 100 us.  Measured, LDS / memory: wing 53 levels, 2.03 M cells 707 / 924 us, 3.92 M
+// 1421 / 1688; polyhedra of six columns, 89 levels, 180 k 90 / 276, 3.99 M 1738 / 1702;
+// of eight, 104 levels, 896 k 515 / 649, 1.8 M 1098 / 961.
+inline bool sgs_from_memory(int nParts, double levels, int columns, size_t lds) {
+    if (2 * lds <= 160 * 1024) return false;
+    const double perCu = (nParts + 255) / 256;
+    return 3.0 * levels + 100.0 * (perCu - 1) < perCu * (50.0 + (columns > 6 ? 0.85 : 0.7) * levels);
+}
+
 struct Mesh {
     int nC = 0, nI = 0, nB = 0, nF = 0;  // nF = nI + nB surface-field length
     int nPatches = 0;

@@ -487,7 +487,7 @@ __global__ __launch_bounds__(256) void k_sa_sgs(const int32_t* partRowStart, con
 // by the chain of levels: a level read from memory took 5 us (three dependent
 // round trips), here it is LDS accesses, a division and a barrier, with the next
 // pass's entries (256 rows of a level at most) loaded before.  Hexahedra, 400 k
-// cells 440 -> 115 us, 2 M (eight partitions per CU in turn) 924 -> 707.
+// cells 410 -> 115 us, 2 M (eight partitions per CU in turn) 924 -> 707.
 template <int W>
 __global__ __launch_bounds__(256) void k_sa_sgs_lds(int stride, const int32_t* partRowStart, const int32_t* partLevStart,
                                                     const int32_t* partLevPtr, const int32_t* partRows,
@@ -591,7 +591,9 @@ static void launch_sgs(Case& c, const double* A, const double* B, const double* 
     const PartSet& ps = m.sa;
     const int W = ps.maxOff <= 4 ? 4 : ps.maxOff <= 6 ? 6 : 8;
     const int32_t *rs = ps.d_rowStart.p, *ls = ps.d_levStart.p, *lp = ps.d_levPtr.p, *rows = ps.d_rows.p;
-    if (ps.maxOff > 8 || sgs_lds(ps, W) > 150 * 1024) {  // a polyhedral mesh whose rows do not fit
+    const double levels = (double)ps.levPtr.size() / ps.nParts - 1;
+    // polyhedra whose rows do not fit, and many deep partitions one of which fills a CU
+    if (ps.maxOff > 8 || sgs_lds(ps, W) > 150 * 1024 || sgs_from_memory(ps.nParts, levels, W, sgs_lds(ps, W))) {
         hipLaunchKernelGGL(k_sa_sgs, dim3(ps.nParts), dim3(256), 2 * sizeof(double) * (size_t)ps.maxRows, c.stream, rs, ls,
                            lp, rows, m.d_rowPtr.p, m.d_cols.p, m.d_slotDiag.p, ps.d_localCol.p, A, B, xin, xout);
         return;

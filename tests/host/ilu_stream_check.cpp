@@ -303,6 +303,10 @@ static int check_retry(const rdst_mesh_desc* desc, bool fp32, bool natural) {
     }
 }
 
+extern "C" int sa_sgs_from_memory(int nParts, double levels, int columns, int lds) {
+    return sgs_from_memory(nParts, levels, columns, (size_t)lds);
+}
+
 // kmax, chainK, partitions or tiles, and whether the natural order goes by tiles
 extern "C" void ilu_plan_numbers(const rdst_mesh_desc* desc, int fp32, int natural, int* out) {
     Mesh m;

@@ -130,3 +130,15 @@ def test_tiles_where_they_pay(replay_lib, name, tiles):
     kmax, _, n, ok = plan_numbers(replay_lib, MESHES[name](), natural=1)
     assert bool(ok) == tiles and (kmax > 0) == tiles
     assert (n == 1) == (name in ("one cell", "box 33x31"))
+
+
+@pytest.mark.parametrize("parts,levels,columns,rows,memory", [
+    # the sweeps timed both ways: partitions, mean levels, columns per row, rows of the largest
+    (2048, 53, 6, 990, False), (4096, 53, 6, 958, False), (256, 89, 6, 704, False), (4096, 89, 6, 975, True),
+    (256, 89, 8, 704, False), (1024, 100, 8, 875, False), (2048, 104, 8, 879, True),
+    # two partitions per CU
+    (16384, 40, 6, 563, False), (4096, 63, 4, 977, False)])
+def test_gauss_seidel_form(replay_lib, parts, levels, columns, rows, memory):
+    replay_lib.sa_sgs_from_memory.argtypes = [C.c_int, C.c_double, C.c_int, C.c_int]
+    lds = (8 * (columns + 3) + 2 * (columns + 1)) * rows
+    assert bool(replay_lib.sa_sgs_from_memory(parts, levels, columns, lds)) == memory
