@@ -61,30 +61,32 @@ __device__ __forceinline__ void barrier_lds() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// The loader: records [r0, r1) whose first bytes are start[r] (16-byte units).
+// The loader: records [r0, r1) whose first bytes are start[r] (16-byte units;
+// low: their low words, whose differences are all that the loop needs -- with
+// the 64-bit starts in it an airfoil's step was 0.3 % longer).
 // Barrier sequence (matched by stream_compute): one when records 0 and 1 are in
 // the ring, one when record 2 is, then one per record s when record s + 3 is.
 // Between the last two the compute wavefronts read the row entries of record
 // s + 2 and the values of record s + 1 from the ring, so everything before
 // record s + 1 may be overwritten.
 template <int RING, bool NT>
-__device__ __forceinline__ void stream_load(const uint8_t* stream, const int64_t* start_, int r0, int r1, uint8_t* ring) {
+__device__ __forceinline__ void stream_load(const uint8_t* stream, const int64_t* start, const uint32_t* low_, int r0, int r1,
+                                            uint8_t* ring) {
     // scalar loads: the offsets must not wait behind the block loads
-    const __attribute__((address_space(4))) int64_t* start = (const __attribute__((address_space(4))) int64_t*)start_;
+    const __attribute__((address_space(4))) uint32_t* low = (const __attribute__((address_space(4))) uint32_t*)low_;
     constexpr int RC = RING / 1024, MAXF = RC < 60 ? RC : 60;
     const int lane = threadIdx.x & 63;
-    const int64_t base = start[r0];
-    auto from = [&](int q) { return (uint32_t)(start[r0 + q] - base); };  // of record q of the list
-    const int n = r1 - r0, total = (int)((from(n) + 63) / 64);
-    const uint8_t* g = stream + 16 * (size_t)base + 16 * lane;
+    const uint32_t base = low[r0];
+    const int n = r1 - r0, total = (int)((low[r1] - base + 63) / 64);
+    const uint8_t* g = stream + 16 * start[r0] + 16 * lane;
     int issued = 0;
     auto issue = [&](int limit) {
         for (; issued < limit; ++issued) lds_dma16<NT>(g + (size_t)issued * 1024, ring + (issued & (RC - 1)) * 1024);
     };
     // 1 KB pieces that hold everything before the record starting at st
-    auto pieces = [&](uint32_t st) { return (int)((st + 63) / 64); };
+    auto pieces = [&](uint32_t st) { return (int)((st - base + 63) / 64); };
     issue(min(total, MAXF));
-    uint32_t a1 = from(min(1, n)), a2 = from(min(2, n)), a3 = from(min(3, n)), a4 = from(min(4, n));
+    uint32_t a1 = low[r0 + min(1, n)], a2 = low[r0 + min(2, n)], a3 = low[r0 + min(3, n)], a4 = low[r0 + min(4, n)];
     wait_in_flight(issued - pieces(a2));
     barrier_raw();
     issue(min(total, RC));
@@ -92,8 +94,8 @@ __device__ __forceinline__ void stream_load(const uint8_t* stream, const int64_t
     barrier_raw();
     for (int s = 0; s < n; ++s) {
         // a1 .. a4: starts of records s + 1 .. s + 4
-        const uint32_t a5 = from(min(s + 5, n));
-        issue(min(total, (int)(a1 / 64) + RC));
+        const uint32_t a5 = low[r0 + min(s + 5, n)];
+        issue(min(total, (int)((a1 - base) / 64) + RC));
         wait_in_flight(issued - pieces(a4));
         barrier_raw();
         a1 = a2; a2 = a3; a3 = a4; a4 = a5;
@@ -366,6 +368,7 @@ __global__ __launch_bounds__(STREAM_THREADS) void k_stream_apply(const int32_t* 
                                                                  const int32_t* __restrict__ recMid,
                                                                  const uint32_t* __restrict__ hdr,
                                                                  const int64_t* __restrict__ start,
+                                                                 const uint32_t* __restrict__ low,
                                                                  const uint8_t* __restrict__ stream,
                                                                  const TV* __restrict__ r, TV* __restrict__ x) {
     constexpr int RING = stream_ring(sizeof(TM) == 4);
@@ -375,7 +378,7 @@ __global__ __launch_bounds__(STREAM_THREADS) void k_stream_apply(const int32_t* 
     const int pt = blockIdx.x;
     const int r0 = recBeg[pt], rm = recMid[pt], r1 = recBeg[pt + 1];
     if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == STREAM_WAVES) {
-        stream_load<RING, NT>(stream, start, r0, r1, ring);
+        stream_load<RING, NT>(stream, start, low, r0, r1, ring);
         return;
     }
     const int rs = rowStart[pt], nl5 = (rowStart[pt + 1] - rs) * 5;
@@ -504,6 +507,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_sweep(int nT, int* ticket
                                                              const int32_t* __restrict__ need,
                                                              const uint32_t* __restrict__ hdr,
                                                              const int64_t* __restrict__ start,
+                                                             const uint32_t* __restrict__ low,
                                                              const uint8_t* __restrict__ stream, const TV* in, TV* out,
                                                              TV* reset) {
     constexpr int RING = stream_ring(sizeof(TM) == 4);
@@ -522,7 +526,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_sweep(int nT, int* ticket
         const int r0 = BWD ? recMid[tl] : recBeg[tl], r1 = BWD ? recBeg[tl + 1] : recMid[tl];
         const int rs = rowStart[tl], nl5 = (rowStart[tl + 1] - rs) * 5;
         if (wave == STREAM_WAVES) {
-            stream_load<RING, false>(stream, start, r0, r1, ring);
+            stream_load<RING, false>(stream, start, low, r0, r1, ring);
             if ((threadIdx.x & 63) == 0) next[(round + 1) & 1] = atomicAdd(tickets + BWD, 1);
         } else if (wave > STREAM_WAVES) {
             const int h0 = haloStart[tl];

@@ -239,6 +239,7 @@ void StreamSet::upload() {
     d_entries.upload(entries);
     d_hdr.upload(hdr);
     d_start.upload(start);
+    d_startLow.upload(std::vector<uint32_t>(start.begin(), start.end()));
     d_need.upload(need);
     d_src.upload(src);
     d_rowCell.upload(rowCell);

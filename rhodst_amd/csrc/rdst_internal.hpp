@@ -128,6 +128,7 @@ struct StreamSet {
     DBuf<uint16_t> d_entries;
     DBuf<uint32_t> d_hdr;
     DBuf<int64_t> d_start;
+    DBuf<uint32_t> d_startLow;  // their low words: a partition's records are within 32 bits of its first
     size_t bytes() const { return 16 * (size_t)start.back(); }
     void clear();  // the host side, before it is built (again, after an attempt that failed)
     void upload();

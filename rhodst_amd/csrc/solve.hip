@@ -1226,7 +1226,7 @@ void stream_launch(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV*
         auto* kernel = past_cache(ps.bytes()) ? k_stream_apply<TM, TV, KDU, true> : k_stream_apply<TM, TV, KDU, false>;
         hipLaunchKernelGGL(kernel, dim3(natural ? 1 : m.nParts), dim3(STREAM_THREADS), shmem, k.s,
                            natural ? ts.d_rowStart.p : m.d_partRowStart.p, natural ? ts.d_rows.p : m.d_partRows.p,
-                           ps.d_recBeg.p, ps.d_recMid.p, ps.d_hdr.p, ps.d_start.p, stream, r, x);
+                           ps.d_recBeg.p, ps.d_recMid.p, ps.d_hdr.p, ps.d_start.p, ps.d_startLow.p, stream, r, x);
         return;
     }
     auto& ty = tile_y(k.w, (const TV*)nullptr);
@@ -1240,10 +1240,10 @@ void stream_launch(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV*
     const size_t tshmem = shmem + 20 * kTileCells;
     hipLaunchKernelGGL((k_tile_sweep<TM, TV, KDU, false>), dim3(grid), dim3(TILE_THREADS), tshmem, k.s, ts.nParts,
                        k.w.tickets.p, ts.d_rowStart.p, ts.d_rows.p, ts.d_haloFStart.p, ts.d_haloF.p, ps.d_recBeg.p,
-                       ps.d_recMid.p, ps.d_need.p, ps.d_hdr.p, ps.d_start.p, stream, r, ty.p, x);
+                       ps.d_recMid.p, ps.d_need.p, ps.d_hdr.p, ps.d_start.p, ps.d_startLow.p, stream, r, ty.p, x);
     hipLaunchKernelGGL((k_tile_sweep<TM, TV, KDU, true>), dim3(grid), dim3(TILE_THREADS), tshmem, k.s, ts.nParts,
                        k.w.tickets.p, ts.d_rowStart.p, ts.d_rows.p, ts.d_haloBStart.p, ts.d_haloB.p, ps.d_recBeg.p,
-                       ps.d_recMid.p, ps.d_need.p, ps.d_hdr.p, ps.d_start.p, stream, (const TV*)ty.p, x, ty.p);
+                       ps.d_recMid.p, ps.d_need.p, ps.d_hdr.p, ps.d_start.p, ps.d_startLow.p, stream, (const TV*)ty.p, x, ty.p);
 }
 template <class TM, class TV>
 void stream_apply(Ctx& k, const StreamSet& ps, const uint8_t* stream, const TV* r, TV* x, bool natural) {
