@@ -54,8 +54,7 @@ static void alloc_fields(Case& c) {
     c.turbBuf.zero();
     c.cell8Buf.alloc(8 * n);
     c.cell8Buf.zero();
-    // the longest array that passes through it whole: LDU blocks, grad(U), face vectors
-    c.stage.alloc(std::min(kStageDoubles, std::max({25 * n, 25 * (size_t)m.nI, 3 * nF, 3 * nB})));
+    c.stage.alloc(std::min(kStageDoubles, std::max({9 * n, 3 * nF, 3 * nB})));  // grad(U), face vectors
     RDST_HIP(hipDeviceSynchronize());
     Fields& f = c.f;
     double* p = c.cellBuf.p;

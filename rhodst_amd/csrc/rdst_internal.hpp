@@ -408,8 +408,8 @@ struct Case {
     // device copies of x and b of rdst_ldu_solve (allocated on first use)
     DBuf<double> lduX, lduB;
     // staging of host arrays that are laid out differently on the device: made
-    // with the case, so that reading a field back needs no memory and no call is
-    // slower for being the first
+    // with the case, so that reading a field back needs no memory and is not slower
+    // for being the first (rdst_ldu_solve makes it longer for its blocks)
     DBuf<double> stage;
     // time-control scalars
     double residual = -1, residualRatio = 1, courantScalar = 1;

@@ -1718,6 +1718,8 @@ void ldu_solve(Case& c, const double* diag, const double* upper, const double* l
             size_t n;
         } parts[3] = {{diag, m.d_slotDiag.p, (size_t)m.nC}, {upper, m.d_slotUpper.p, (size_t)m.nI},
                       {lower, m.d_slotLower.p, (size_t)m.nI}};
+        const size_t want = std::min(kStageDoubles, 25 * (size_t)std::max(m.nC, m.nI));
+        if (c.stage.n < want) c.stage.alloc(want);  // with the solver's other buffers, by the first solve
         double* st = c.stage.p;
         const size_t cap = c.stage.n / 25;
         for (const Part& p : parts)
