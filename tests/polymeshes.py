@@ -44,3 +44,22 @@ def hanging_nodes(nx, ny, ratio, seed=None):
     if seed is not None:
         label = np.random.default_rng(seed).permutation(label.max() + 1)[label]
     return relabelled(mesh, label)
+
+
+def one_merged(nx, ny, i, j):
+    """A 2-D box with cells (i, j) and (i, j + 1) merged into one: its couplings
+    form two triangles (one at a side), with the two cells left and right of it."""
+    mesh = meshgen.box_2d(nx, ny)
+    label = np.arange(mesh.n_cells)
+    label[i + nx * (j + 1)] = i + nx * j
+    return relabelled(mesh, np.unique(label, return_inverse=True)[1])
+
+
+def triangles(mesh, part=None):
+    """Whether three cells (of one part) are coupled pairwise."""
+    nb = [set() for _ in range(mesh.n_cells)]
+    for a, b in zip(mesh.owner, mesh.neighbour):
+        if part is None or part[a] == part[b]:
+            nb[a].add(b)
+            nb[b].add(a)
+    return any(nb[a] & nb[b] for a in range(mesh.n_cells) for b in nb[a] if b > a)

@@ -62,3 +62,35 @@ def test_a_matrix_that_is_not_finite_shows_in_the_residuals(nx, ny, kw, bad):
     # a finite one is converged at once for b = 0
     x, perf = dc.ldu_solve(diag, upper, lower, np.zeros((n, 5)), np.zeros((n, 5)), mode=2)
     assert not x.any() and perf.n_iterations == 0 and list(perf.initial_residual) == [0.0] * 5
+
+
+# 820, 819, 182 and 169 cells: every remainder of 5 n by four, a tail of which the
+# FP32 basis is padded with; 274 400 cells: the vectors past a grid stride of the
+# four-wide loops (1.05 M entries), matrix and stream past 128 MiB in both
+# precisions (non-temporal loads).  20 directions: three groups of eight of the
+# multi-dot, five vectors at a time of the update.
+@pytest.mark.parametrize("nx,ny", [(82, 10), (9, 91), (14, 13), (13, 13), (560, 490)])
+@pytest.mark.parametrize("kw", [dict(gram_schmidt="modified"), dict(gram_schmidt="classical"),
+                                dict(gram_schmidt="modified", precision="mixed"),
+                                dict(gram_schmidt="classical", precision="mixed")],
+                         ids=lambda kw: "-".join(kw.values()))
+def test_residual_of_a_converged_solve(nx, ny, kw):
+    mesh = meshgen.box_2d(nx, ny)
+    n, nI = mesh.n_cells, len(mesh.neighbour)
+    rng = np.random.default_rng(ny)
+    upper, lower = rng.uniform(-0.5, 0.5, (2, nI, 5, 5))
+    own, nei = np.asarray(mesh.owner[:nI]), np.asarray(mesh.neighbour)
+    # coupled strongly enough that a cycle needs its 20 directions
+    diag = rng.uniform(-0.5, 0.5, (n, 5, 5)) + 4.0 * np.eye(5)
+    b = rng.standard_normal((n, 5))
+    patches = {p[0]: {"p": "zeroGradient", "T": "zeroGradient", "U": "zeroGradient"} for p in mesh.patches if p[1] != 3}
+    st = make_settings(n_directions=20, max_iter=8, min_iter=1, tolerance=1e-15, rel_tol=0.0, ilu_order="partitioned", **kw)
+    spec = cases.CaseSpec("krylov", mesh, make_thermo(), make_bcs(mesh, patches), st, np.ones(n), np.ones(n), np.zeros((n, 3)))
+    x, perf = _capi.DeviceCase(spec, _capi.DeviceMesh(mesh)).ldu_solve(diag, upper, lower, b, np.zeros((n, 5)))
+    r = b - np.einsum("nij,nj->ni", diag, x)
+    np.subtract.at(r, own, np.einsum("nij,nj->ni", upper, x[nei]))
+    np.subtract.at(r, nei, np.einsum("nij,nj->ni", lower, x[own]))
+    # rounding of the residual itself: 25 products of about |b| per entry
+    assert np.linalg.norm(r) <= 1e-13 * np.linalg.norm(b)
+    # an FP32 basis loses what FP64 has, not cycles: 1e-5 and more per cycle of 20 directions
+    assert perf.n_iterations <= 5

@@ -9,7 +9,8 @@ import subprocess
 import numpy as np
 import pytest
 
-from rhodst_amd import meshgen
+from polymeshes import hanging_nodes, one_merged, triangles
+from rhodst_amd import DeviceMesh, _capi, meshgen
 from rhodst_amd._abi import MeshDesc, rdst_mesh_desc
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -64,6 +65,10 @@ MESHES = {
     "tets": lambda: meshgen.tet_prism_box(11, 13, 12, prism_layers=3, jitter=0.1),
     "box shuffled": lambda: shuffled(meshgen.box_2d(60, 45, jitter=0.2), 1),
     "tets shuffled": lambda: shuffled(meshgen.tet_prism_box(7, 6, 8, prism_layers=3, jitter=0.1), 2),
+    # rows of up to eight blocks, couplings in triangles
+    "polyhedra": lambda: hanging_nodes(9, 40, 7),
+    "polyhedra shuffled": lambda: hanging_nodes(9, 100, 3, seed=1),
+    "one polyhedron": lambda: one_merged(40, 40, 16, 15),
 }
 
 
@@ -142,3 +147,27 @@ def test_gauss_seidel_form(replay_lib, parts, levels, columns, rows, memory):
     replay_lib.sa_sgs_from_memory.argtypes = [C.c_int, C.c_double, C.c_int, C.c_int]
     lds = (8 * (columns + 3) + 2 * (columns + 1)) * rows
     assert bool(replay_lib.sa_sgs_from_memory(parts, levels, columns, lds)) == memory
+
+
+# the polyhedron inside a tile and a partition, and at the sides of several (tiles of
+# 16 x 8 cells, the second row and column of partitions from 20 on); the last two
+# triangles are cut by a partition's side, which leaves its factor a chain
+PLACES = [(3, 3), (15, 3), (16, 3), (4, 7), (15, 7), (16, 15), (19, 19), (20, 19), (19, 20), (20, 5), (38, 37),
+          (0, 27), (39, 10)]
+
+
+@pytest.mark.parametrize("mesh", [lambda: hanging_nodes(9, 40, 7), lambda: hanging_nodes(9, 100, 3, seed=1)] +
+                         [lambda p=p: one_merged(40, 40, *p) for p in PLACES],
+                         ids=["polyhedra", "polyhedra shuffled"] + [f"{i},{j}" for i, j in PLACES])
+def test_chain_factor_only_without_triangles(replay_lib, mesh):
+    pm = mesh()
+    part = DeviceMesh(pm).get_int(_capi.M_PARTITION)
+    lower = np.zeros(pm.n_cells, dtype=int)
+    inside = part[pm.owner[:len(pm.neighbour)]] == part[pm.neighbour]
+    np.add.at(lower, pm.neighbour[inside], 1)
+    _, chain, n, _ = plan_numbers(replay_lib, pm, natural=0)
+    assert n == part.max() + 1 >= 2
+    assert (chain > 0) == (not triangles(pm, part) and lower.max() <= 4)
+    assert triangles(pm)
+    kmax, chain, n, ok = plan_numbers(replay_lib, pm, natural=1)
+    assert chain == 0 and n > 1 and bool(kmax) == bool(ok)
