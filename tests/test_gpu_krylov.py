@@ -94,3 +94,28 @@ def test_residual_of_a_converged_solve(nx, ny, kw):
     assert np.linalg.norm(r) <= 1e-13 * np.linalg.norm(b)
     # an FP32 basis loses what FP64 has, not cycles: 1e-5 and more per cycle of 20 directions
     assert perf.n_iterations <= 5
+
+
+@pytest.mark.parametrize("order,precision", [("natural", "fp64"), ("natural", "mixed"), ("partitioned", "fp64"),
+                                             ("partitioned", "mixed")])
+@pytest.mark.parametrize("nx,ny", [(13, 8), (40, 40)])  # one partition or tile, several that wait for each other
+def test_a_singular_pivot_block_is_an_error(nx, ny, order, precision):
+    mesh = meshgen.box_2d(nx, ny)
+    n, nI = mesh.n_cells, len(mesh.neighbour)
+    rng = np.random.default_rng(nx)
+    upper, lower = rng.uniform(-0.5, 0.5, (2, nI, 5, 5))
+    diag = rng.uniform(-0.5, 0.5, (n, 5, 5)) + 8.0 * np.eye(5)
+    b = rng.standard_normal((n, 5))
+    patches = {p[0]: {"p": "zeroGradient", "T": "zeroGradient", "U": "zeroGradient"} for p in mesh.patches if p[1] != 3}
+    spec = cases.CaseSpec("krylov", mesh, make_thermo(), make_bcs(mesh, patches),
+                          make_settings(n_directions=4, ilu_order=order, precision=precision),
+                          np.ones(n), np.ones(n), np.zeros((n, 3)))
+    dc = _capi.DeviceCase(spec, _capi.DeviceMesh(mesh))
+    x, _ = dc.ldu_solve(diag, upper, lower, b, np.zeros((n, 5)))
+    # cell 0 has no lower neighbour: its pivot block is the diagonal block
+    zero = diag.copy()
+    zero[0] = 0.0
+    with pytest.raises(_capi.RdstError, match="singular pivot"):
+        dc.ldu_solve(zero, upper, lower, b, np.zeros((n, 5)))
+    # and the system before it has the same solution after it
+    assert np.array_equal(dc.ldu_solve(diag, upper, lower, b, np.zeros((n, 5)))[0], x)
