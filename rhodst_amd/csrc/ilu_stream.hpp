@@ -4,10 +4,10 @@
 // wavefronts work through it record by record with the partition's vector in
 // LDS.
 //
-// What bounds it: a partition is a chain of 32 or more dependent levels per
-// sweep, each with 10-50 rows, so on small and mid-size meshes a level costs the
-// latency of whatever it waits for; from about 1e6 cells on, the stream itself
-// (HBM).  Loading a level's blocks when the level is reached cost one memory
+// What bounds it: a partition is a chain of at most 32 dependent levels per
+// sweep (a mesh that is one tile: of all its levels), each with 2-50 rows, so on
+// small and mid-size meshes a level costs the latency of whatever it waits for;
+// from about 1e6 cells on, the stream itself (HBM).  Loading a level's blocks when the level is reached cost one memory
 // round trip per level (0.75 us); here the blocks of the following records are
 // already in the ring, the next record's are in registers, and a level costs an
 // LDS gather, the products and a barrier (0.35 us).  Measured, before and after,

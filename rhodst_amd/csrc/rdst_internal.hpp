@@ -440,7 +440,7 @@ struct Case {
 // the case's staging buffer in pieces: out[k i + d] = comps[d][i], or back.
 // One copy and one pass on the device; the host side only copies.  (The
 // components copied one by one and interleaved by the host took 2.9 ms for the
-// five of R at 555 k cells, against 0.6.)
+// five of R at 599 k cells, against 0.6.)
 constexpr size_t kStageDoubles = (size_t)8 << 20;  // 64 MiB, the longest staging buffer
 void download_aos(Case& c, const double* const* comps, int k, size_t n, double* out);
 void upload_aos(Case& c, double* const* comps, int k, size_t n, const double* in);
