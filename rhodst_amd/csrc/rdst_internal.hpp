@@ -20,7 +20,8 @@ void set_error(const std::string& msg);
     do {                                                                                \
         hipError_t e_ = (call);                                                         \
         if (e_ != hipSuccess) {                                                         \
-            throw ::rdst::HipError(std::string(#call) + ": " + hipGetErrorString(e_)); \
+            (void)hipGetLastError(); /* reported here, not by the next call's check */  \
+            throw ::rdst::HipError(std::string(#call) + ": " + hipGetErrorString(e_));  \
         }                                                                               \
     } while (0)
 

@@ -11,15 +11,21 @@
 
 static std::atomic<int> g_mallocs{0};
 static int g_mallocsLeft = -1;  // allocations until one fails (negative: none does)
+static hipError_t g_last = hipSuccess;  // the runtime's last error
 static hipError_t test_malloc(void** p, size_t n) {
     ++g_mallocs;
-    if (g_mallocsLeft >= 0 && g_mallocsLeft-- == 0) return hipErrorOutOfMemory;
+    if (g_mallocsLeft >= 0 && g_mallocsLeft-- == 0) return g_last = hipErrorOutOfMemory;
     *p = std::malloc(n);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 static hipError_t test_free(void* p) {
     std::free(p);
     return hipSuccess;
+}
+static hipError_t test_last() {
+    const hipError_t e = g_last;
+    g_last = hipSuccess;
+    return e;
 }
 static hipError_t test_memcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
     std::memcpy(d, s, n);
@@ -28,6 +34,7 @@ static hipError_t test_memcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
 #define hipMalloc test_malloc
 #define hipFree test_free
 #define hipMemcpy test_memcpy
+#define hipGetLastError test_last
 #include "../../rhodst_amd/csrc/mesh_host.cpp"
 
 #include <cstdio>
@@ -271,6 +278,7 @@ static int check_retry(const rdst_mesh_desc* desc, bool fp32, bool natural) {
     }
     g_mallocsLeft = -1;
     if (buf.p || buf.n) return fail("a failed allocation leaves a size");
+    if (g_last != hipSuccess) return fail("a failed allocation leaves its error to the next check");
     auto plan = [&](Mesh& m) -> StreamSet& { return natural ? mesh_tiles(m, fp32).ps[fp32] : mesh_stream(m, fp32); };
     Mesh ref;
     mesh_build(ref, desc);
